@@ -5,6 +5,8 @@
 //  * k_recon1d / k_evolve1d / k_wall1d / k_update1d: one workgroup per cell or face, the three
 //    phases kept separate exactly as KitBase runs them, with slopes and face fluxes stored in HBM.
 //    These back the phase-level entry points and handle any velocity count (1F3V included).
+#include <algorithm>
+
 #include "kbg_device.h"
 #include "kbg_sweep.h"
 #include "kbg_types.h"
@@ -421,6 +423,155 @@ __global__ __launch_bounds__(256) void k_resid(const double* __restrict__ rows, 
     }
 }
 
+// ------------------------------------------------------------------------------------------------
+// the 1D1F3V KFVS step of kbg_step / kbg_batch_step: reconstruct! and evolve! in one launch over (face,
+// velocity chunk), the cells' FP64 chain, and the relaxation over (cell, velocity chunk).  The phase
+// kernels above take one workgroup per cell or face, 50 of them for a 50-cell shock structure on 256
+// CUs; for 24^3 velocities, FP32 / FP64, they took 44 / 51 us per step against 14 / 16 us here.  Slopes,
+// fluxes and relaxation are the phase kernels' expressions; only the moment sums' order differs.
+// ------------------------------------------------------------------------------------------------
+
+constexpr int k3vVpt = 4;                // velocities per thread of the flux kernel
+constexpr int k3vChunk = 256 * k3vVpt;   // velocities per workgroup
+
+template <class T> __global__ __launch_bounds__(256) void k_flux3v(const Solve1D* __restrict__ pS, double* __restrict__ psum) {
+    __shared__ double red_s[4 * 5];
+    const Solve1D& S = *pS;
+    const int k = S.face_lo + blockIdx.x, nfc = gridDim.x;  // physical face
+    const int ng = S.ng, nv = S.nv, N = S.nx + 2 * ng;
+    const int kL = k - 2 + ng, kR = k - 1 + ng;
+    const T dxLT = T(0.5 * S.dx[kL]), dxRT = T(0.5 * S.dx[kR]);
+    const T* __restrict__ f = (const T*)S.f[S.cur];
+    const T* __restrict__ sf = (const T*)S.sf;
+    const T* __restrict__ U = (const T*)S.u;
+    const T* __restrict__ V = (const T*)S.v;
+    const T* __restrict__ Wv = (const T*)S.wv;
+    const T* __restrict__ WT = (const T*)S.wt;
+    T* __restrict__ ff = (T*)S.ff + (size_t)(k - 1) * nv;
+    const double dt = S.dt;
+    const T dtT = T(dt), hdt2 = T(0.5 * dt * dt);
+    // slope of cell kc: reconstruct!'s where it computes one, the stored one elsewhere
+    auto inr = [&](int kc) { return kc - ng + 1 >= S.slope_lo && kc - ng + 1 <= S.slope_hi; };
+    const bool inL = inr(kL), inR = inr(kR);
+    const int kLm = kL > 0 ? kL - 1 : 0, kRp = kR < N - 1 ? kR + 1 : N - 1;
+    const T rLm = T(1.0 / (0.5 * (S.dx[kLm] + S.dx[kL]))), rM = T(1.0 / (0.5 * (S.dx[kL] + S.dx[kR]))),
+            rRp = T(1.0 / (0.5 * (S.dx[kR] + S.dx[kRp])));
+    double r[5] = {0, 0, 0, 0, 0};
+#pragma unroll
+    for (int j = 0; j < k3vVpt; j++) {
+        const int iv = blockIdx.y * k3vChunk + j * 256 + threadIdx.x;
+        if (iv < nv) {
+            const T x = U[iv], wq = WT[iv];
+            const bool d = x >= T(0);
+            const T fl = f[(size_t)kL * nv + iv], fr = f[(size_t)kR * nv + iv];
+            T su;
+            if (d ? inL : inR) {
+                const T o = f[(size_t)(d ? kLm : kRp) * nv + iv];
+                const T a = d ? o : fl, c = d ? fl : fr, e = d ? fr : o;
+                su = limf<T>(S.limiter, (c - a) * (d ? rLm : rM), (e - c) * (d ? rM : rRp));
+            } else {
+                su = sf[(size_t)(d ? kL : kR) * nv + iv];
+            }
+            const T fu = d ? fl + su * dxLT : fr - su * dxRT;
+            const T fv = dtT * x * fu - hdt2 * (x * x) * su;
+            ff[iv] = fv;
+            const T g = wq * fv, y = V[iv], z = Wv[iv];
+            r[0] += double(g);
+            r[1] += double(x * g);
+            r[2] += double(y * g);
+            r[3] += double(z * g);
+            r[4] += double((x * x + y * y + z * z) * g);
+        }
+    }
+    block_allreduce256<5>(r, red_s);
+    if (threadIdx.x == 0)
+        for (int m = 0; m < 5; m++) psum[((size_t)blockIdx.y * 5 + m) * nfc + blockIdx.x] = r[m];
+}
+
+// The faces' moments (the chunks' sums in order, stored as evolve! leaves them) and the stepped cells'
+// FP64 chain: one thread per face k and the cell to its right.  crec: 8 doubles per stepped cell.
+__global__ __launch_bounds__(64) void k_chain3v(const Solve1D* __restrict__ pS, const double* __restrict__ psum, int nchunk,
+                                                double* __restrict__ crec, double* __restrict__ rcell) {
+    const Solve1D& S = *pS;
+    const int nfc = S.face_hi - S.face_lo + 1, nx = S.nx;
+    const int k = min(S.face_lo, S.upd_lo) + blockIdx.x * 64 + threadIdx.x;
+    auto face_fw = [&](int kf, double (&fw)[5]) {
+        const int b = kf - S.face_lo;
+        if (b < 0 || b >= nfc) {  // a stored boundary face
+            for (int m = 0; m < 5; m++) fw[m] = S.fw[(size_t)(kf - 1) * 5 + m];
+            return;
+        }
+        for (int m = 0; m < 5; m++) fw[m] = 0.0;
+#pragma unroll 8
+        for (int c = 0; c < nchunk; c++)
+#pragma unroll
+            for (int m = 0; m < 5; m++) fw[m] += psum[((size_t)c * 5 + m) * nfc + b];
+        fw[4] *= 0.5;
+    };
+    double fl[5], fr[5];
+    const bool isface = k >= S.face_lo && k <= S.face_hi, cell = k >= S.upd_lo && k <= S.upd_hi;
+    if (isface || cell) face_fw(k, fl);
+    if (isface)
+        for (int m = 0; m < 5; m++) S.fw[(size_t)(k - 1) * 5 + m] = fl[m];
+    if (!cell) return;
+    face_fw(k + 1, fr);
+    const int ks = k - 1 + S.ng;
+    double* w = S.w[S.cur] + (size_t)ks * 5;
+    double wo[5], wn[5], pn[5];
+    for (int m = 0; m < 5; m++) {
+        wo[m] = w[m];
+        wn[m] = wo[m] + (fl[m] - fr[m]) / S.dx[ks];
+    }
+    conserve_prim<5>(wn, S.gam, pn);
+    flag_health(S.health, prim_health<5>(pn));
+    const double lamn = pn[4], rt = S.dt / vhs_tau(pn[0], lamn, S.mu, S.om);
+    double* o = crec + (size_t)(k - S.upd_lo) * 8;
+    o[0] = rt;
+    o[1] = 1.0 / (1.0 + rt);
+    o[2] = 1.0 / S.dx[ks];
+    o[3] = pn[0] * sqrt((lamn / kPi) * (lamn / kPi) * (lamn / kPi));
+    o[4] = lamn;
+    o[5] = pn[1];
+    o[6] = pn[2];
+    o[7] = pn[3];
+    const bool bnd = k == 1 || k == nx;
+    double* row = rcell ? rcell + (size_t)(k - S.upd_lo) * 20 : nullptr;
+    for (int m = 0; m < 5; m++) {
+        w[m] = wn[m];
+        S.prim[(size_t)ks * 5 + m] = pn[m];
+        if (row) {
+            row[(bnd ? 10 : 0) + m] = (wn[m] - wo[m]) * (wn[m] - wo[m]);
+            row[(bnd ? 15 : 5) + m] = fabs(wn[m]);
+            row[(bnd ? 0 : 10) + m] = 0.0;
+            row[(bnd ? 5 : 15) + m] = 0.0;
+        }
+    }
+}
+
+// the relaxation (or the transport update + dt Q of the fast spectral collision) of the stepped cells
+template <class T> __global__ __launch_bounds__(256) void k_relax3v(const Solve1D* __restrict__ pS, const double* __restrict__ crec) {
+    const Solve1D& S = *pS;
+    const int c = S.upd_lo + blockIdx.x, nv = S.nv, k = c - 1 + S.ng;
+    const int iv = blockIdx.y * 256 + threadIdx.x;
+    if (iv >= nv) return;
+    T* __restrict__ f = (T*)S.f[S.cur] + (size_t)k * nv;
+    const T* __restrict__ ffL = (const T*)S.ff + (size_t)(c - 1) * nv;
+    const T* __restrict__ ffR = ffL + nv;
+    const double* __restrict__ o = crec + (size_t)blockIdx.x * 8;
+    const T rdx = T(o[2]);
+    if (S.coll == FSM && c > 1 && c < S.nx) {
+        const T dtT = T(S.dt);
+        f[iv] = f[iv] + (ffL[iv] - ffR[iv]) * rdx + dtT * T(S.fsmq[(size_t)(c - S.fsm_c0) * nv + iv]);
+        return;
+    }
+    const T rT = T(o[0]), inv = T(o[1]), An = T(o[3]), ln = T(o[4]), Un = T(o[5]), Vn = T(o[6]), Wn = T(o[7]);
+    const T x = ((const T*)S.u)[iv], y = ((const T*)S.v)[iv] - Vn, z = ((const T*)S.wv)[iv] - Wn;
+    T c2 = (x - Un) * (x - Un);
+    c2 += y * y + z * z;
+    const T MH = An * texp(-ln * c2);
+    f[iv] = (f[iv] + (ffL[iv] - ffR[iv]) * rdx + rT * MH) * inv;
+}
+
 // Workgroup size of the phase kernels: 256 threads, or 1024 for large velocity grids (1D1F3V), whose
 // few cells and faces would otherwise leave each thread a long serial loop
 static int phase_threads(const Solve1D& S) { return S.nv >= 2048 ? 1024 : 256; }
@@ -484,6 +635,34 @@ hipError_t launch_update1d(bool fp64, const Solve1D& S, const Solve1D* d_S, doub
         else return hipErrorInvalidValue;
     }
 #undef KBG_U
+    return hipGetLastError();
+}
+
+size_t step3v_doubles(const Solve1D& S) {
+    const size_t nchunk = (size_t(S.nv) + k3vChunk - 1) / k3vChunk;
+    return nchunk * 5 * (size_t(S.nx) + 1) + 8 * size_t(S.nx);
+}
+
+hipError_t launch_flux3v(bool fp64, const Solve1D& S, const Solve1D* d_S, double* d_work, hipStream_t st) {
+    const int n = S.face_hi - S.face_lo + 1;
+    if (n <= 0) return hipSuccess;
+    const dim3 g(n, (S.nv + k3vChunk - 1) / k3vChunk), b(256);
+    if (fp64) hipLaunchKernelGGL(k_flux3v<double>, g, b, 0, st, d_S, d_work);
+    else hipLaunchKernelGGL(k_flux3v<float>, g, b, 0, st, d_S, d_work);
+    return hipGetLastError();
+}
+
+hipError_t launch_cell3v(bool fp64, const Solve1D& S, const Solve1D* d_S, double* d_work, double* d_rcell, hipStream_t st) {
+    const int nchunk = (S.nv + k3vChunk - 1) / k3vChunk;
+    double* crec = d_work + (size_t)nchunk * 5 * (S.nx + 1);
+    const int nt = std::max(S.face_hi, S.upd_hi) - std::min(S.face_lo, S.upd_lo) + 1, n = S.upd_hi - S.upd_lo + 1;
+    if (nt <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_chain3v, dim3((nt + 63) / 64), dim3(64), 0, st, d_S, d_work, nchunk, crec, d_rcell);
+    if (n > 0) {
+        const dim3 g(n, (S.nv + 255) / 256), b(256);
+        if (fp64) hipLaunchKernelGGL(k_relax3v<double>, g, b, 0, st, d_S, crec);
+        else hipLaunchKernelGGL(k_relax3v<float>, g, b, 0, st, d_S, crec);
+    }
     return hipGetLastError();
 }
 

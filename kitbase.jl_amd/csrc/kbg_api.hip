@@ -115,6 +115,7 @@ struct kbg_solve {
     double *dx = nullptr, *dy = nullptr;
     double* rcell = nullptr;
     double* res = nullptr;
+    double* work3v = nullptr;  // 1D1F3V KFVS, second order: sums and cell coefficients of its step kernels
     // 1D
     Solve1D h1{};
     Solve1D* d1 = nullptr;
@@ -572,6 +573,9 @@ void fill1d(kbg_solve* s) {
     }
 }
 
+// 1D1F3V solves stepped by k_flux3v / k_chain3v / k_relax3v (KCU and first order: the phase kernels)
+bool step3v(const Solve1D& S) { return S.vdim == 3 && S.flux == kbg::KFVS && S.interp2; }
+
 void fill2d(kbg_solve* s) {
     const kbg_desc& d = s->d;
     Solve2D& S = s->h2;
@@ -703,7 +707,7 @@ void build_items(kbg_solve* s, int seg, int solve_index, int nw, std::vector<Wor
     }
 }
 
-int step_phase_1d(kbg_solve* s, double dt, double* residual, hipStream_t st);
+int step_phase_1d(kbg_solve* s, double dt, double* residual, hipStream_t st, bool inline3v = false);
 int step_phase_2d(kbg_solve* s, double dt, double* residual, hipStream_t st);
 int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double* dts, int nsteps, double* residuals, bool noalloc);
 
@@ -884,8 +888,15 @@ size_t kbg_solve_bytes(const kbg_desc* d) {
             if (cn && esz == 8) fsm += ((nd + 2) * (nc + 2) * n3 + nd * (nc + 1) * 6 * cn * cn + 2 * cn) * 8;
             else fsm += (cn ? nc * (nd + 1) * n3 * 4 : nc * (2 * nd + 2) * n3 * 2 * esz) + cn * 2 * esz + (2 * nd + 1) * n3 * esz;
         }
+        size_t w3 = 0;
+        if (d->vdim == 3 && d->flux == KBG_KFVS && d->interp_order == 2) {
+            Solve1D S{};
+            S.nx = d->nx;
+            S.nv = d->nv;
+            w3 = kbg::step3v_doubles(S) * 8;
+        }
         return 2 * np * d->nf * d->nv * esz + 3 * N * nw * 8 + N * 8 + 4 * size_t(d->nv) * esz + 2 * d->nf * d->nv * esz +
-               N * 4 * nw * 8 + vt + fsm;
+               N * 4 * nw * 8 + vt + fsm + w3;
     }
     const size_t C = size_t(d->nx) * d->ny, F = size_t(d->nx + 1) * d->ny + size_t(d->nx) * (d->ny + 1);
     const size_t nv = d->nv;
@@ -1006,6 +1017,10 @@ int kbg_solve_create(kbg_ctx* ctx, const kbg_desc* desc, kbg_solve** out) {
             HIPCHK(hipMemset(s->vtab, 0, vb));
             S.vtab = s->vtab;
             if ((rc = ensure_vtab(s, 0.0))) return bail(rc);
+        }
+        if (step3v(S)) {
+            if ((rc = dev_alloc(s, &p, kbg::step3v_doubles(S) * 8))) return bail(rc);
+            s->work3v = (double*)p;
         }
         if (d.collision == KBG_FSM) {
             // Q for the interior cells 2 .. nx-1 (update! steps them with :fsm; boundary cells take BGK)
@@ -2041,6 +2056,7 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
     // residual rows are kept
     // ubase: the parity of the round's first step among the call's steps (unstructured solves flip
     // their f buffer every step)
+    bool capturing = false;
     auto enqueue_round = [&](int nst, bool last_round, int ubase) -> int {
         int e;
         for (Launch& L : launches) {
@@ -2079,6 +2095,11 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
                     HIPCHK(hipMemcpyAsync(r, s->res, 4 * 8, hipMemcpyDeviceToHost, ss));
                     HIPCHK(hipStreamSynchronize(ss));
                 }
+            } else if (s->work3v) {
+                // the last step (any captured one) also leaves its slopes where reconstruct! does
+                if (last || capturing) HIPCHK(kbg::launch_recon1d(s->fp64, s->h1, s->d1, ss));
+                HIPCHK(kbg::launch_flux3v(s->fp64, s->h1, s->d1, s->work3v, ss));
+                if ((e = step_phase_1d(s, dts[i], r, ss, true))) return e;
             } else if (s->d.dim == 1) {
                 HIPCHK(kbg::launch_recon1d(s->fp64, s->h1, s->d1, ss));
                 HIPCHK(kbg::launch_evolve1d(s->fp64, s->h1, s->d1, ss));
@@ -2154,6 +2175,7 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
         }
         if (sig != ctx->gsig || !ctx->gexec[0] || !ctx->gexec[1] || !ctx->gexec[2] || !ctx->gexec[3]) {
             ctx->drop_graphs();
+            capturing = true;
             for (int which = 0; which < 4; which++) {
                 HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeRelaxed));
                 for (Launch& L : launches) L.flips = L.two ? which >> 1 : 0;
@@ -2171,6 +2193,7 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
                 ctx->graph[which] = g;
                 HIPCHK(hipGraphInstantiate(&ctx->gexec[which], g, nullptr, nullptr, 0));
             }
+            capturing = false;
             ctx->gsig = std::move(sig);
         }
     }
@@ -2233,8 +2256,9 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
     return KBG_OK;
 }
 
-// update! on the phase-exact path (kernels k_update1d / k_resid), optional residual download
-int step_phase_1d(kbg_solve* s, double dt, double* residual, hipStream_t st) {
+// update! on the phase-exact path (kernels k_update1d / k_resid), optional residual download; inline3v:
+// after k_flux3v, whose moment sums k_chain3v adds up
+int step_phase_1d(kbg_solve* s, double dt, double* residual, hipStream_t st, bool inline3v) {
     (void)dt;
     double* rc_ = residual ? s->rcell : nullptr;
     if (s->has_fsm) {
@@ -2242,7 +2266,8 @@ int step_phase_1d(kbg_solve* s, double dt, double* residual, hipStream_t st) {
         const Solve1D& S = s->h1;
         HIPCHK(kbg::fsm_collision(s->fsm, s->fp64, S.f[S.cur], S.fcs, s->fsm.c0 - 1 + S.ng, st));
     }
-    HIPCHK(kbg::launch_update1d(s->fp64, s->h1, s->d1, rc_, st));
+    if (inline3v) HIPCHK(kbg::launch_cell3v(s->fp64, s->h1, s->d1, s->work3v, rc_, st));
+    else HIPCHK(kbg::launch_update1d(s->fp64, s->h1, s->d1, rc_, st));
     if (residual) {
         const int nrows = s->h1.upd_hi - s->h1.upd_lo + 1;
         HIPCHK(kbg::launch_resid1d(s->h1, s->rcell, nrows, 4 * s->nw, s->res, st));

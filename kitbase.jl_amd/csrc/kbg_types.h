@@ -180,6 +180,12 @@ hipError_t launch_evolve1d(bool fp64, const Solve1D& S, const Solve1D* d_S, hipS
 hipError_t launch_wall1d(bool fp64, const Solve1D& S, const Solve1D* d_S, int fused, int par, hipStream_t st);
 hipError_t launch_update1d(bool fp64, const Solve1D& S, const Solve1D* d_S, double* d_rcell, hipStream_t st);
 
+// The 1D1F3V KFVS step: face fluxes with the slopes built inline, then the cells.  d_work: step3v_doubles
+// FP64 values (the chunks' moment sums, the cells' coefficients)
+size_t step3v_doubles(const Solve1D& S);
+hipError_t launch_flux3v(bool fp64, const Solve1D& S, const Solve1D* d_S, double* d_work, hipStream_t st);
+hipError_t launch_cell3v(bool fp64, const Solve1D& S, const Solve1D* d_S, double* d_work, double* d_rcell, hipStream_t st);
+
 // The fast spectral collision of a 1D1F3V solve (kbg_fsm.hip): kernel modes and work buffers on the
 // device, hipFFT plans for the cells c0 .. c0 + ncell - 1
 struct FsmPlan {
