@@ -210,6 +210,7 @@ __global__ __launch_bounds__(256) void k_fsm_sum(const float* __restrict__ part,
     const int ci = int(i / n3), q = int(i % n3);
     const float* __restrict__ pp = part + (size_t)ci * (nd + 1) * n3 + q;
     double re = 0.0;
+#pragma unroll 10  // ten loads in flight per thread: 10.9 us for the 56 MB of 48 cells of 24^3, 15.7 without
     for (int d = 0; d < nd; d++) re += double(pp[(size_t)d * n3]);
     re -= double(pp[(size_t)nd * n3]);
     Q[i] = scale * re;
