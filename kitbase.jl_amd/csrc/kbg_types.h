@@ -118,6 +118,7 @@ struct SolveUS {
     int cur;              // buffer holding the state at the start of a call (kernels add their parity)
     double* fw;           // [nface][4] global frame
     void* ff;             // [nface][nf][nv]
+    double* fws;          // [nface][5] the fused step's face moments and wall amplitudes
     double* rcell;        // [ncell][8] residual rows (sum of squared change, sum of |w|)
     int* health;
 };
@@ -238,7 +239,7 @@ hipError_t launch_delta2d(const Solve2D& S, const Solve2D* d_S, int mode, hipStr
 int ustep_threads(int nv);
 hipError_t launch_uface(bool fp64, int threads, const SolveUS& S, const SolveUS* d_S, hipStream_t st);
 hipError_t launch_ucell(bool fp64, int threads, const SolveUS& S, const SolveUS* d_S, int rows, hipStream_t st);
-hipError_t launch_ustep(bool fp64, int threads, const SolveUS& S, const SolveUS* d_S, int par, int rows, hipStream_t st);
+hipError_t launch_ustep(bool fp64, const SolveUS& S, const SolveUS* d_S, int par, int rows, hipStream_t st);
 hipError_t launch_uavg(bool fp64, const SolveUS& S, const SolveUS* d_S, int par, hipStream_t st);
 hipError_t launch_uresid(const double* d_rows, int nrows, double* d_out, hipStream_t st);
 hipError_t launch_ucfl(const double* d_prim, const double* d_dmin, int n, double u1, double v1, double gam, double* d_out,

@@ -1,28 +1,26 @@
 // kbg_us.hip -- the unstructured-mesh DVM on triangles (2D1F2V and 2D2F2V, KFVS) for gfx950.
 //
-//   k_ustep   the fused time step: one wavefront per cell, lanes striding the velocity grid.  A
-//             stepped cell (cellType 0 or 2) evaluates the fluxes of its three faces itself --
-//             KitBase's KFVS flux between the face's two cells at interpOrder 1, where the cells'
-//             slopes are zero and the face values are the cell values (flux_kfvs.jl:615-697,
-//             with the face's normal and tangential velocities, solver_evolution.jl:872-1035) or the
-//             diffuse Maxwell wall of a boundary face (flux_boundary.jl:160-220), the face moments
-//             reduced in FP64 and turned to the global frame (geo_general.jl:6-26) -- and applies the
-//             triangle step! (step_1f.jl:228-285, step_2f.jl:256-326): the FP64 chain (w -= sum
-//             dirc fw / area, conserve_prim, tau, Shakhov heat flux), then every lane relaxes its
-//             velocities.  f is read from one buffer and written to the other, so the face fluxes
-//             never go to memory: per step f is read from HBM (own cell and the three neighbours,
-//             the neighbours and the second pass mostly from L2) and written once.  Cells that are
-//             not stepped copy f.
+//   k_usum, k_ustep   the fused time step, one wavefront per face and one per cell, lanes striding the
+//             velocity grid.  k_usum: a face's moments -- KitBase's KFVS flux between the face's two cells
+//             at interpOrder 1, where the cells' slopes are zero and the face values are the cell values
+//             (flux_kfvs.jl:615-697, with the face's normal and tangential velocities,
+//             solver_evolution.jl:872-1035) or the diffuse Maxwell wall of a boundary face
+//             (flux_boundary.jl:160-220), summed in FP64 and turned to the global frame
+//             (geo_general.jl:6-26).  k_ustep: the triangle step! (step_1f.jl:228-285, step_2f.jl:256-326)
+//             of a cell of cellType 0 or 2: the FP64 chain (w -= sum dirc fw / area, conserve_prim, tau,
+//             Shakhov heat flux), then every lane forms its velocities' three face fluxes again, from
+//             the upwind cells, and relaxes.  f is read from one buffer and written to the other, so the
+//             face fluxes never go to memory.  Cells that are not stepped copy f.
 //   k_uface   evolve! alone: the same face fluxes, stored to fw / ff (one workgroup per face).
 //   k_ucell   update! alone: the same triangle step from the stored fluxes, in place.
 //   k_uavg    one workgroup, the cellType-3 cells in index order: w and f the mean of the two
 //             neighbours (update_boundary.jl:520-590).
 //
-// k_ustep and the k_uface + k_ucell pair share the flux and cell code below; they sum the face
+// k_usum + k_ustep and the k_uface + k_ucell pair share the flux and cell code below; they sum the face
 // moments in different orders, so a fused step and an evolve! + update! pair agree to rounding.
 // k_ustep takes its cells in an XCD-aware order: the hardware deals workgroups to the 8 XCDs in
 // turn, so workgroup b steps the four cells of group (b % 8) * chunk + b / 8 and each XCD walks a
-// contiguous run of cells, whose neighbours' f it finds in its own L2.
+// contiguous run of cells, whose neighbours' f it finds in its own L2 (k_usum likewise with its faces).
 //
 // The wall is taken with rot = 1: the face normal of a boundary face points into the mesh, so the
 // velocities with vn >= 0 come from the wall (KitBase's unstructured evolve! passes no `rot`, which
@@ -394,29 +392,110 @@ template <class T, int VPT> __global__ __launch_bounds__(1024) void k_ucell(cons
     }
 }
 
-// The fused step, one wavefront per cell (W cells per workgroup, no workgroup barrier: every LDS
-// word is written and read back by the same lane).  A face's moments in the global frame are
-// moments of its flux with the face-frame velocities turned back: with |n|^2 = n1^2 + n2^2 (KitBase's
-// unit_normal leaves it slightly below 1), (un n1 - vt n2, un n2 + vt n1) = |n|^2 (u, v) and
-// un^2 + vt^2 = |n|^2 (u^2 + v^2), so
+// The fused step's faces, one wavefront per face.  A face's moments in the global frame are moments of its
+// flux with the face-frame velocities turned back: with |n|^2 = n1^2 + n2^2 (KitBase's unit_normal leaves it
+// slightly below 1), (un n1 - vt n2, un n2 + vt n1) = |n|^2 (u, v) and un^2 + vt^2 = |n|^2 (u^2 + v^2), so
 //   fw = (sum w F, |n|^2 sum w u F, |n|^2 sum w v F, (|n|^2 sum w (u^2 + v^2) F + sum w Fb) / 2).
-// Pass 1 takes one face at a time (after a first pass that fixes the wall densities when the cell
-// has a Maxwell wall): it sums these four moments in FP64 (the Fb part of the last over 2 |n|^2, so
-// that one factor |n|^2 turns the sum into fw) with a wavefront reduction per face, and adds the
-// face's dirc-weighted flux to the relaxation's flux terms sum_j dirc_j F_j, sum_j dirc_j Fb_j in
-// LDS (stored kind-2 fluxes included); the heat flux follows in a loop of its own.  The two cells of a face sum its
-// moments over the same velocities in the same order and reduce them the same way, so they see the
-// same fw and the face's mass, momentum and energy leave one cell exactly as they enter the other.
-// Every lane then runs the FP64 chain (the same values in all lanes) and pass 2 relaxes from the
-// cell's f and the LDS terms.  The moments are summed in another order than k_uface's local-frame
-// sums: a fused step and an evolve! + update! pair agree to rounding.
-template <class T> __global__ __launch_bounds__(256) void k_ustep(const SolveUS* __restrict__ pS, int par, int rows, int chunk, int W) {
-    extern __shared__ double ldsd[];
+// The four moments are FP64 sums (the Fb part of the last over 2 |n|^2, so that one factor |n|^2 turns the
+// sum into fw), stored once per face: both cells take the same fw, and a face's mass, momentum and energy
+// leave one cell exactly as they enter the other.  Stored (kind 2) faces copy their fw; walls also keep
+// their Maxwellian's amplitude.  The moments are summed in another order than k_uface's local-frame sums: a
+// fused step and an evolve! + update! pair agree to rounding.
+//
+// Bound by the latency of the loads and the FP64 sums.  One kernel with a wavefront per cell that summed its
+// three faces itself, with the flux terms kept in LDS between its passes, formed every face's FP64 sums twice
+// and held 10 kB of LDS per wavefront.  Both ways, us per step: 16^2 x 2 triangles x 16^2 velocities FP32 13.0
+// then, 12.0 now; 64^2 x 2 x 28^2 FP32 86 / 66 (k_usum 24, k_ustep 41; their reads and writes at the copy rate
+// of 4.6 TB/s 33), FP64 148 / 108; 96^2 x 2 x 40^2 FP32 541 / 290, FP64 1097 / 524.
+constexpr int kUBatch = 4;  // velocities per lane loaded together
+
+template <class T> __global__ __launch_bounds__(256) void k_usum(const SolveUS* __restrict__ pS, int par, int chunk) {
+    const SolveUS& S = *pS;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int f = __builtin_amdgcn_readfirstlane((int(blockIdx.x % kXcd) * chunk + int(blockIdx.x / kXcd)) * 4 + wave);
+    if (f >= S.nface) return;
+    const int nv = S.nv, RS = S.nf * nv;
+    const bool two = S.nf == 2;
+    const gptr<double> out = to_global(S.fws) + (size_t)f * 5;
+    const UFace F = uface_at(S, f);
+    if (F.kind == 2) {
+        if (lane < 4) out[lane] = to_global(S.fw)[(size_t)f * 4 + lane];
+        return;
+    }
+    const gptr<const T> fin = fbuf<T>(S, par);
+    const gptr<const T> U = to_global((const T*)S.u), V = to_global((const T*)S.v), WT = to_global((const T*)S.wt);
+    const double hb = 0.5 / (F.n1 * F.n1 + F.n2 * F.n2);
+    double a4[4] = {0, 0, 0, 0};
+    auto add = [&](const UVel<T>& x, T fh, T fb) {
+        const double e = double(x.wq * fh);
+        a4[0] += e;
+        a4[1] += double(x.u) * e;
+        a4[2] += double(x.v) * e;
+        a4[3] += 0.5 * double(x.u * x.u + x.v * x.v) * e;
+        if (two) a4[3] += hb * double(x.wq * fb);
+    };
+    double Aw = 0.0;
+    if (F.kind == 0) {
+        const gptr<const T> pa = fin + (size_t)F.a * RS, po = fin + (size_t)F.o * RS;
+        const T dtT = T(S.dt), lenT = T(F.len);
+        for (int v0 = lane; v0 < nv; v0 += 64 * kUBatch) {
+            UVel<T> x[kUBatch];
+            T un[kUBatch], h[kUBatch], b[kUBatch];
+#pragma unroll
+            for (int k = 0; k < kUBatch; k++) {
+                const int iv = min(v0 + 64 * k, nv - 1);
+                x[k] = UVel<T>{iv, U[iv], V[iv], v0 + 64 * k < nv ? WT[iv] : T(0)};
+                T vt;
+                rotate(F, x[k], un[k], vt);
+                const gptr<const T> p = un[k] >= T(0) ? pa : po;
+                h[k] = p[iv];
+                b[k] = two ? p[nv + iv] : T(0);
+            }
+#pragma unroll
+            for (int k = 0; k < kUBatch; k++) add(x[k], (dtT * un[k] * h[k]) * lenT, (dtT * un[k] * b[k]) * lenT);
+        }
+    } else {
+        const gptr<const T> pc = fin + (size_t)(F.a >= 0 ? F.a : F.o) * RS;
+        const T Uw = T(F.bU), Vw = T(F.bV), lw = T(F.bl), kbw = T(S.K / (2.0 * F.bl)), sc = T(F.len * S.dt);
+        double s2[2] = {0, 0};
+        for (int iv = lane; iv < nv; iv += 64) {
+            const UVel<T> x{iv, U[iv], V[iv], WT[iv]};
+            T un, vt;
+            rotate(F, x, un, vt);
+            wall_pre_vel(un, vt, x.wq, pc[iv], Uw, Vw, lw, s2[0], s2[1]);
+        }
+        wave_allreduce<2>(s2);
+        Aw = wall_amp(s2[0], s2[1], F.bl);
+        const T A = T(Aw);
+        for (int iv = lane; iv < nv; iv += 64) {
+            const UVel<T> x{iv, U[iv], V[iv], WT[iv]};
+            T un, vt, fh = T(0), fb = T(0);
+            double t[5] = {0, 0, 0, 0, 0};  // local-frame sums: unused here
+            rotate(F, x, un, vt);
+            wall_vel(un, vt, x.wq, pc[iv], two ? pc[nv + iv] : T(0), two, Uw, Vw, lw, A, kbw, sc, fh, fb, t);
+            add(x, fh, fb);
+        }
+    }
+    wave_allreduce<4>(a4);
+    const double nn = F.n1 * F.n1 + F.n2 * F.n2;
+    if (lane == 0) {
+        out[0] = a4[0];
+        out[1] = nn * a4[1];
+        out[2] = nn * a4[2];
+        out[3] = nn * a4[3];
+        out[4] = Aw;
+    }
+}
+
+// The fused step's cells, one wavefront per cell, four cells per workgroup (no workgroup barrier): every lane
+// runs the FP64 chain (the same values in all lanes), then forms its velocities' fluxes from the upwind
+// cells and relaxes from one f buffer into the other.
+template <class T> __global__ __launch_bounds__(256) void k_ustep(const SolveUS* __restrict__ pS, int par, int rows, int chunk) {
     const SolveUS& S = *pS;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     // the wavefront's cell, a wavefront-uniform value: the cell's and its faces' data go to scalar registers
-    const int c = __builtin_amdgcn_readfirstlane((int(blockIdx.x % kXcd) * chunk + int(blockIdx.x / kXcd)) * W + wave);
-    if (c >= S.ncell) return;  // per wavefront: no workgroup barrier follows
+    const int c = __builtin_amdgcn_readfirstlane((int(blockIdx.x % kXcd) * chunk + int(blockIdx.x / kXcd)) * 4 + wave);
+    if (c >= S.ncell) return;
     const int nv = S.nv, RS = S.nf * nv;
     const bool two = S.nf == 2, shak = two && S.coll == SHAKHOV;
     const gptr<const T> fin = fbuf<T>(S, par);
@@ -430,104 +509,26 @@ template <class T> __global__ __launch_bounds__(256) void k_ustep(const SolveUS*
         if (rrow && lane < 8) rrow[lane] = 0.0;
         return;
     }
-    T* g = reinterpret_cast<T*>(ldsd) + (size_t)wave * RS;  // [G0 | B0] of this wavefront's velocities
     double po[4];
 #pragma unroll
     for (int m = 0; m < 4; m++) po[m] = to_global(S.prim)[(size_t)c * 4 + m];
     const gptr<const double> dr = to_global(S.dirc) + (size_t)c * 3;
-    const gptr<const T> U = to_global((const T*)S.u);
-    const gptr<const T> V = to_global((const T*)S.v);
-    const gptr<const T> WT = to_global((const T*)S.wt);
+    const gptr<const T> U = to_global((const T*)S.u), V = to_global((const T*)S.v), WT = to_global((const T*)S.wt);
     UFace F[3];
-    gptr<const T> nb[3];  // the neighbour's f (interior face) or the stored flux (kind 2)
-    bool first[3];        // this cell is the face's first cell
-    bool wall = false;
-    T d[3];       // dirc_j
-    double hb[3];  // 1 / (2 |n_j|^2): the b part of the energy sum, taken out of |n|^2 again below
+    gptr<const T> up[3], dn[3];  // f upwind of un >= 0 and of un < 0 (interior), or the stored flux (kind 2)
+    T d[3], A[3];                // dirc_j, the wall Maxwellian's amplitude
+    double dw[4] = {0, 0, 0, 0};
 #pragma unroll
     for (int j = 0; j < 3; j++) {
         const int f = to_global(S.cf)[(size_t)c * 3 + j];
         F[j] = uface_at(S, f);
-        first[j] = F[j].a == c;
-        nb[j] = F[j].kind == 0 ? fin + (size_t)(first[j] ? F[j].o : F[j].a) * RS
-                               : (F[j].kind == 2 ? to_global((const T*)S.ff) + (size_t)f * RS : nullptr);
-        wall = wall || F[j].kind == 1;
+        up[j] = F[j].kind == 0 ? fin + (size_t)F[j].a * RS : (F[j].kind == 2 ? to_global((const T*)S.ff) + (size_t)f * RS : fc);
+        dn[j] = F[j].kind == 0 ? fin + (size_t)F[j].o * RS : up[j];
         d[j] = T(dr[j]);
-        hb[j] = 0.5 / (F[j].n1 * F[j].n1 + F[j].n2 * F[j].n2);
-    }
-    T A[3] = {T(0), T(0), T(0)};
-    if (wall) {
-        double s2[6] = {0, 0, 0, 0, 0, 0};
-        for (int iv = lane; iv < nv; iv += 64) {
-            const UVel<T> x{iv, U[iv], V[iv], WT[iv]};
-            const T h = fc[iv];
+        const gptr<const double> w = to_global(S.fws) + (size_t)f * 5;
+        A[j] = T(w[4]);
 #pragma unroll
-            for (int j = 0; j < 3; j++) {
-                if (F[j].kind != 1) continue;
-                T un, vt;
-                rotate(F[j], x, un, vt);
-                wall_pre_vel(un, vt, x.wq, h, T(F[j].bU), T(F[j].bV), T(F[j].bl), s2[2 * j], s2[2 * j + 1]);
-            }
-        }
-        wave_allreduce<6>(s2);
-#pragma unroll
-        for (int j = 0; j < 3; j++)
-            if (F[j].kind == 1) A[j] = T(wall_amp(s2[2 * j], s2[2 * j + 1], F[j].bl));
-    }
-    const T dtT = T(S.dt), KT = T(S.K);
-    // pass 1, one face at a time: its moments [sum w F, sum w u F, sum w v F, sum w (u^2 + v^2) F / 2 +
-    // sum w Fb / (2 |n|^2)] in FP64 and the flux terms sum_j dirc_j F_j, sum_j dirc_j Fb_j in LDS
-    double fw[3][4];
-#pragma unroll
-    for (int j = 0; j < 3; j++) {
-        if (F[j].kind == 2) {
-            for (int iv = lane; iv < nv; iv += 64) {
-                const T gh = nb[j][iv] * d[j];
-                g[iv] = j == 0 ? gh : g[iv] + gh;
-                if (two) {
-                    const T gb = nb[j][nv + iv] * d[j];
-                    g[nv + iv] = j == 0 ? gb : g[nv + iv] + gb;
-                }
-            }
-#pragma unroll
-            for (int m = 0; m < 4; m++) fw[j][m] = to_global(S.fw)[(size_t)to_global(S.cf)[(size_t)c * 3 + j] * 4 + m];
-            continue;
-        }
-        double a4[4] = {0, 0, 0, 0};
-        const T lenT = T(F[j].len), Uw = T(F[j].bU), Vw = T(F[j].bV), lw = T(F[j].bl), kbw = T(S.K / (2.0 * F[j].bl)),
-                sc = T(F[j].len * S.dt);
-        for (int iv = lane; iv < nv; iv += 64) {
-            const UVel<T> x{iv, U[iv], V[iv], WT[iv]};
-            const T h = fc[iv], b = two ? fc[nv + iv] : T(0);
-            double t[5] = {0, 0, 0, 0, 0};  // local-frame sums: unused here
-            T un, vt, fh = T(0), fb = T(0);
-            rotate(F[j], x, un, vt);
-            if (F[j].kind == 0) {
-                const T hn = nb[j][iv], bn = two ? nb[j][nv + iv] : T(0);
-                kfvs_vel(un, vt, x.wq, first[j] ? h : hn, first[j] ? hn : h, first[j] ? b : bn, first[j] ? bn : b, two, dtT, lenT,
-                         fh, fb, t);
-            } else {
-                wall_vel(un, vt, x.wq, h, b, two, Uw, Vw, lw, A[j], kbw, sc, fh, fb, t);
-            }
-            const double e = double(x.wq * fh);
-            a4[0] += e;
-            a4[1] += double(x.u) * e;
-            a4[2] += double(x.v) * e;
-            a4[3] += 0.5 * double(x.u * x.u + x.v * x.v) * e;
-            if (two) a4[3] += hb[j] * double(x.wq * fb);
-            const T gh = fh * d[j];
-            g[iv] = j == 0 ? gh : g[iv] + gh;
-            if (two) {
-                const T gb = fb * d[j];
-                g[nv + iv] = j == 0 ? gb : g[nv + iv] + gb;
-            }
-        }
-        wave_allreduce<4>(a4);
-        const double nn = F[j].n1 * F[j].n1 + F[j].n2 * F[j].n2;
-        fw[j][0] = a4[0];
-        fw[j][1] = nn * a4[1];
-        fw[j][2] = nn * a4[2];
-        fw[j][3] = nn * a4[3];
+        for (int m = 0; m < 4; m++) dw[m] += w[m] * dr[j];
     }
     double q[4] = {0, 0, 0, 0};
     if (shak) {
@@ -535,17 +536,54 @@ template <class T> __global__ __launch_bounds__(256) void k_ustep(const SolveUS*
         for (int iv = lane; iv < nv; iv += 64) heat_vel(U[iv], V[iv], WT[iv], fc[iv], fc[nv + iv], Uo, Vo, q);
         wave_allreduce<4>(q);
     }
-    double dw[4];
-#pragma unroll
-    for (int m = 0; m < 4; m++) dw[m] = fw[0][m] * dr[0] + fw[1][m] * dr[1] + fw[2][m] * dr[2];
+    const T dtT = T(S.dt), KT = T(S.K);
     const UCellT<T> kt = to_t<T>(cell_chain(S, c, po, q, dw, true, lane, rrow));
-    // pass 2: the relaxation
-    for (int iv = lane; iv < nv; iv += 64) {
-        const T h = fc[iv], b = two ? fc[nv + iv] : T(0);
-        T hn, bn;
-        relax_vel(kt, shak, KT, U[iv], V[iv], h, b, g[iv], two ? g[nv + iv] : T(0), hn, bn);
-        fo[iv] = hn;
-        if (two) fo[nv + iv] = bn;
+    constexpr int NB = sizeof(T) == 4 ? 2 : 1;  // velocities per lane in flight
+    for (int v0 = lane; v0 < nv; v0 += 64 * NB) {
+        UVel<T> x[NB];
+        T un[3][NB], vt[3][NB], h[NB], b[NB], hu[3][NB], bu[3][NB];
+#pragma unroll
+        for (int k = 0; k < NB; k++) {
+            const int iv = min(v0 + 64 * k, nv - 1);
+            x[k] = UVel<T>{iv, U[iv], V[iv], T(0)};
+            h[k] = fc[iv];
+            b[k] = two ? fc[nv + iv] : T(0);
+#pragma unroll
+            for (int j = 0; j < 3; j++) {
+                rotate(F[j], x[k], un[j][k], vt[j][k]);
+                const gptr<const T> p = un[j][k] >= T(0) ? up[j] : dn[j];
+                hu[j][k] = p[iv];
+                bu[j][k] = two ? p[nv + iv] : T(0);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < NB; k++) {
+            T gh = T(0), gb = T(0);
+#pragma unroll
+            for (int j = 0; j < 3; j++) {
+                T fh, fb;
+                if (F[j].kind == 0) {
+                    fh = (dtT * un[j][k] * hu[j][k]) * T(F[j].len);
+                    fb = (dtT * un[j][k] * bu[j][k]) * T(F[j].len);
+                } else if (F[j].kind == 2) {
+                    fh = hu[j][k];
+                    fb = bu[j][k];
+                } else {
+                    double t[5] = {0, 0, 0, 0, 0};
+                    fb = T(0);
+                    wall_vel(un[j][k], vt[j][k], T(0), h[k], b[k], two, T(F[j].bU), T(F[j].bV), T(F[j].bl), A[j], T(S.K / (2.0 * F[j].bl)),
+                             T(F[j].len * S.dt), fh, fb, t);
+                }
+                gh += fh * d[j];
+                gb += fb * d[j];
+            }
+            T hn, bn;
+            relax_vel(kt, shak, KT, x[k].u, x[k].v, h[k], b[k], gh, gb, hn, bn);
+            if (v0 + 64 * k < nv) {
+                fo[x[k].iv] = hn;
+                if (two) fo[nv + x[k].iv] = bn;
+            }
+        }
     }
 }
 
@@ -646,19 +684,19 @@ hipError_t launch_ucell(bool fp64, int threads, const SolveUS& S, const SolveUS*
     return hipGetLastError();
 }
 
-hipError_t launch_ustep(bool fp64, int threads, const SolveUS& S, const SolveUS* d_S, int par, int rows, hipStream_t st) {
-    (void)threads;  // one wavefront per cell
+hipError_t launch_ustep(bool fp64, const SolveUS& S, const SolveUS* d_S, int par, int rows, hipStream_t st) {
     if (S.ncell <= 0) return hipSuccess;
-    // W cells per workgroup, W the most of 4, 2, 1 whose LDS flux terms (W nf nv values) fit 64 KiB;
-    // workgroup b -> cell group (b % 8) chunk + b / 8 covers [0, 8 chunk) once (each XCD a contiguous
-    // run); cells past ncell exit
-    const size_t per = size_t(S.nf) * S.nv * (fp64 ? 8 : 4);
-    const int W = 4 * per <= 65536 ? 4 : (2 * per <= 65536 ? 2 : 1);
-    if (per > 65536) return hipErrorInvalidValue;
-    const int groups = (S.ncell + W - 1) / W, chunk = (groups + kXcd - 1) / kXcd;
-    const dim3 grid(unsigned(chunk) * kXcd), block(64 * W);
-    if (fp64) hipLaunchKernelGGL(k_ustep<double>, grid, block, W * per, st, d_S, par, rows, chunk, W);
-    else hipLaunchKernelGGL(k_ustep<float>, grid, block, W * per, st, d_S, par, rows, chunk, W);
+    // four faces or cells per workgroup; workgroup b -> group (b % 8) chunk + b / 8 covers [0, 8 chunk) once
+    // (each XCD a contiguous run); groups past the end exit
+    const int fch = ((S.nface + 3) / 4 + kXcd - 1) / kXcd, cch = ((S.ncell + 3) / 4 + kXcd - 1) / kXcd;
+    const dim3 gf(unsigned(fch) * kXcd), gc(unsigned(cch) * kXcd), b(256);
+    if (fp64) {
+        if (S.nface > 0) hipLaunchKernelGGL(k_usum<double>, gf, b, 0, st, d_S, par, fch);
+        hipLaunchKernelGGL(k_ustep<double>, gc, b, 0, st, d_S, par, rows, cch);
+    } else {
+        if (S.nface > 0) hipLaunchKernelGGL(k_usum<float>, gf, b, 0, st, d_S, par, fch);
+        hipLaunchKernelGGL(k_ustep<float>, gc, b, 0, st, d_S, par, rows, cch);
+    }
     return hipGetLastError();
 }
 

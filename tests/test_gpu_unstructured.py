@@ -301,3 +301,22 @@ def test_us_refusals():
     with pytest.raises(kb._lib.KbgError, match="slopes"):
         kb._lib.check(dev.lib.kbg_upload_slopes(dev.handle, None, None))
     dev.close()
+
+
+@pytest.mark.parametrize("space", ["2d2f2v", "2d1f2v"])
+@pytest.mark.parametrize("nu,nv", [(9, 7), (8, 8), (13, 5), (17, 15), (16, 16), (13, 20)])
+def test_us_fused_step_at_the_edges_of_its_velocity_batches(space, nu, nv):
+    """63, 64, 65, 255, 256 and 260 velocities: around one wavefront and around the four velocities per lane
+    that k_usum loads together (k_ustep: two in FP32, one in FP64), with walls, averaged cells and stored
+    faces; FP64 as above, FP32 to the same bound as test_us_fp32_matches_the_oracle."""
+    mk = kb.configs.cavity_2d2f2v if space == "2d2f2v" else kb.configs.cavity_2d1f2v
+    ks = kb.SolverSet(mk(nu=nu, nv=nv, knudsen=0.1, collision="bgk", interpOrder=1, vMeshType="rectangle"))
+    ps = kb.mesh.tri_rectangle(0.0, 1.0, 5, 0.0, 1.0, 3)
+    ps.cellType[boundary_cells(ps, 2)] = 3
+    st = kb.mesh.init_fvm_us(ks, ps)
+    dt = kb.mesh.timestep_us(ks, ps, st)
+    for precision, tol in (("fp64", 1e-10), ("fp32", 1e-4)):
+        sg, so, rg, ro = run_both(ks, ps, copy.deepcopy(st), dt, 5, precision)
+        err = rel_max if precision == "fp64" else rel_l2
+        assert err(sg.w, so.w) < tol
+        assert err(sg.f, so.f) < tol
