@@ -39,7 +39,7 @@ int fail(int code, const std::string& msg) {
         if (e_ != hipSuccess) return fail(KBG_ERR_HIP, std::string(#expr) + ": " + hipGetErrorString(e_)); \
     } while (0)
 
-constexpr int kMaxSeg = kbg::kSweepOut;  // fused 1D sweep: cells per work item
+constexpr int kMaxSeg = kbg::sweep_out(1);  // fused 1D sweep: cells per work item
 
 }  // namespace
 
@@ -52,7 +52,7 @@ struct kbg_ctx {
     static constexpr int kSide = 3;
     hipStream_t side[kSide] = {};
     hipEvent_t fork = nullptr, join[kSide] = {};
-    int seg_cells = kbg::kSweepOut;  // cells per sweep workgroup
+    int seg_cells = kbg::sweep_out(1);  // cells per sweep workgroup
     int streams = 0;                 // concurrent streams of a batch (0: all, 1 + kSide)
     // batch staging (device)
     Solve1D* d_descs = nullptr;
@@ -770,6 +770,8 @@ int kbg_ctx_create(int device, kbg_ctx** out) {
     for (auto& ev : c->join)
         if (e == hipSuccess) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
     if (e == hipSuccess) e = hipMalloc((void**)&c->d_res, 4096 * 5 * sizeof(double));
+    if (e == hipSuccess) e = kbg::sweep_narrow_attr32();
+    if (e == hipSuccess) e = kbg::sweep_narrow_attr64();
     if (e != hipSuccess) {
         kbg_ctx_destroy(c);
         return fail(KBG_ERR_HIP, std::string("kbg_ctx_create: ") + hipGetErrorString(e));
@@ -1823,20 +1825,47 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
             launches2.push_back(L);
         }
     }
-    // two time steps per sweep launch for each fused 1D solve that allows it (KFVS, no boundary-face
-    // buffers: no walls, no stepped cell next to a ghost-less boundary); not under graph replay.  The
-    // choice is the solve's own, so a solve advances in the same step pairs (counted from the first
-    // step of the call) in any batch: a two-step pass may round differently from two one-step passes.
-    const bool two_ok = ctx->sweep_steps == 2;
-    std::vector<char> two_of(n, 0);
-    bool two = false;  // some launch takes two steps per round
+    bool any_fsm = false;
+    for (int i : others) any_fsm = any_fsm || solves[i]->has_fsm;
+    // hipFFT calls stay out of stream capture: batches with :fsm solves launch eagerly
+    const bool use_graph = ctx->graphs && !residuals && nsteps >= 2 && !noalloc && !any_fsm;
+    // The sweep's width.  A launch of few wavefronts takes as long as one wavefront's serial work, and more
+    // wavefronts per item of fewer velocities shorten it; one that fills the chip loses by the extra
+    // wavefronts' set-up.  us per step, full width / narrow: Sod 100 x 64 FP64 13.4 / 6.5, FP32 14.8 / 3.5;
+    // 1000 x 256 FP32 15.6 / 7.7; 16000 x 64 FP64 13.6 / 8.9; n ragged FP32 tubes (64..2048 cells x 32..256
+    // velocities, about 55 wavefronts each at full width): n = 4 19.2 / 9.4, 24 21.2 / 13.1, 36 22.9 / 19.1,
+    // 48 26.2 / 24.9, 64 30.5 / 32.3, 96 33.1 / 47.1, 256 85.2 / 131.
+    // A solve's results do not depend on the width (kbg_sweep.h), so the rule may look at the whole batch.
+    constexpr long kNarrowWaves = 2700;
+    long waves0 = 0;
     for (int i : fused) {
         const Solve1D& S = solves[i]->h1;
-        two_of[i] = two_ok && S.flux == kbg::KFVS && !S.wallL && !S.wallR && !(S.faceL_buf && S.upd_lo == 1) &&
-                    !(S.faceR_buf && S.upd_hi == S.nx);
-        two = two || two_of[i];
+        waves0 += long(S.upd_hi - S.upd_lo + kbg::sweep_out(2)) / kbg::sweep_out(2) * solves[i]->sweep_nw;
     }
-    auto seg_of = [&](int i) { return std::min(std::max(1, ctx->seg_cells), two_of[i] ? kbg::kSweepOut2 : kbg::kSweepOut); };
+    std::vector<int> narrow_nw(n, 0);  // wavefronts per item of the narrow sweep, 0: the full-width sweep
+    for (int i : fused) {
+        const kbg_solve* s = solves[i];
+        const int nv = s->d.nv, most = kbg::sweep_vw_narrow(s->d.nf);
+        if (s->d.flux != KBG_KFVS || nv > kbg::kSweepNarrowWaves * most || waves0 > kNarrowWaves || ctx->sweep_vw > most) continue;
+        const int vw = ctx->sweep_vw > 0 ? ctx->sweep_vw : kbg::kVChunk;
+        int nw = 1;
+        while (nw < kbg::kSweepNarrowWaves && kbg::sweep_item_vw(nv, nw) > vw) nw *= 2;
+        if (nw > s->sweep_nw) narrow_nw[i] = nw;
+    }
+    // time steps per sweep launch of each fused 1D solve: two, or four in the narrow sweep, for solves
+    // that allow several (KFVS, no boundary-face buffers: no walls, no stepped cell next to a ghost-less
+    // boundary), else one; calls that return residuals take at most two, whose segments the residual sums follow
+    std::vector<int> steps_of(n, 1);
+    int round = 1;  // time steps per round of every unit
+    for (int i : fused) {
+        const Solve1D& S = solves[i]->h1;
+        if (ctx->sweep_steps == 2 && S.flux == kbg::KFVS && !S.wallL && !S.wallR && !(S.faceL_buf && S.upd_lo == 1) &&
+            !(S.faceR_buf && S.upd_hi == S.nx))
+            steps_of[i] = narrow_nw[i] && !use_graph && !residuals ? 4 : 2;
+        round = std::max(round, steps_of[i]);
+    }
+    const bool two = round >= 2;  // some launch takes two steps per round
+    auto seg_of = [&](int i) { return std::min(std::max(1, ctx->seg_cells), kbg::sweep_out(steps_of[i])); };
     // Independent units -- fused 1D solves, fused 2D groups and solves stepped by the phase kernels
     // -- are spread over the streams by work (cells x velocities x distributions), heaviest first;
     // each stream advances its own share.
@@ -1887,7 +1916,10 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
         int nf, flux, wg_waves, stream;
         size_t pack0, npacks;
         std::vector<int> members;  // solve indices (for the wall kernels)
-        bool two;                  // two time steps per launch in a round of two
+        int per;                   // most time steps per launch
+        int narrow;                // the narrow sweep: its items' most wavefronts (0: k_sweep1d)
+        int rows;                  // narrow: most velocity chunks of its solves
+        size_t item0, nitems;
         int flips;                 // sweep launches enqueued so far (the f / w buffer parity)
     };
     std::vector<Solve1D> descs;
@@ -1895,13 +1927,13 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
     std::vector<WorkItem> items;
     std::vector<kbg::Pack> packs;
     std::vector<Launch> launches;
-    std::map<std::tuple<int, int, int, int, int>, std::vector<int>> keyed;  // (stream, fp64, nf, flux, two) -> solves
+    std::map<std::tuple<int, int, int, int, int, int>, std::vector<int>> keyed;  // (stream, fp64, nf, flux, steps, narrow) -> solves
     for (int i : fused)
-        keyed[{stream_of[i], solves[i]->fp64 ? 1 : 0, solves[i]->d.nf, solves[i]->d.flux, two_of[i] ? 1 : 0}].push_back(i);
+        keyed[{stream_of[i], solves[i]->fp64 ? 1 : 0, solves[i]->d.nf, solves[i]->d.flux, steps_of[i], narrow_nw[i] ? 1 : 0}].push_back(i);
     std::vector<int> launch_of(n, -1);
     for (auto& kv : keyed) {
         Launch L{std::get<1>(kv.first) == 1, std::get<2>(kv.first), std::get<3>(kv.first), 1, std::get<0>(kv.first),
-                 packs.size(), 0, kv.second, std::get<4>(kv.first) == 1, 0};
+                 packs.size(), 0, kv.second, std::get<4>(kv.first), 0, 0, items.size(), 0, 0};
         for (int i : kv.second) launch_of[i] = (int)launches.size();
         std::map<int, std::vector<int>> by_nw;  // nw -> item indices, in solve order
         for (int i : kv.second) {
@@ -1913,12 +1945,20 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
             // wavefronts per item: the kernel's width, or more when the context caps the velocities
             // per wavefront (a function of the solve and the context only, so a solve's sums keep
             // their order in any batch)
-            int nw = s->sweep_nw;
-            if (ctx->sweep_vw > 0)
+            int nw = narrow_nw[i] ? narrow_nw[i] : s->sweep_nw;
+            if (narrow_nw[i]) {
+                L.narrow = std::max(L.narrow, nw);
+                L.rows = std::max(L.rows, (s->d.nv + kbg::kVChunk - 1) / kbg::kVChunk);
+            } else if (ctx->sweep_vw > 0)
                 while (nw < kbg::kSweepMaxWaves && (s->d.nv + nw - 1) / nw > ctx->sweep_vw) nw *= 2;
             build_items(s, seg_of(i), desc_of[i], nw, items);
             for (size_t it = i0; it < items.size(); it++) by_nw[nw].push_back((int)it);
             L.wg_waves = std::max(L.wg_waves, nw);
+        }
+        if (L.narrow) {  // one item per workgroup, no packs
+            L.nitems = items.size() - L.item0;
+            launches.push_back(std::move(L));
+            continue;
         }
         // workgroups of at least 4 wavefronts: side-by-side items of the same nw fill them
         L.wg_waves = std::max(L.wg_waves, std::min(4, kbg::kSweepMaxWaves));
@@ -2050,8 +2090,8 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
         }
         return KBG_OK;
     };
-    // one round of every unit on its stream: nst time steps (1 or 2; a fused 1D sweep launch whose
-    // solves allow it takes both in one pass, the other units are launched nst times); each sweep
+    // one round of every unit on its stream: nst time steps (a fused 1D sweep launch whose solves allow it
+    // takes several in one pass, the other units are launched nst times); each sweep
     // launch reads the f / w buffers of its own parity (launches so far), last marks the round whose
     // residual rows are kept
     // ubase: the parity of the round's first step among the call's steps (unstructured solves flip
@@ -2060,8 +2100,8 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
     auto enqueue_round = [&](int nst, bool last_round, int ubase) -> int {
         int e;
         for (Launch& L : launches) {
-            const int per = L.two ? nst : 1;  // steps per launch
-            for (int ks = 0; ks < nst; ks += per) {
+            for (int ks = 0, per; ks < nst; ks += per) {
+                for (per = L.per; per > nst - ks; per /= 2) {}
                 const int par = L.flips & 1;
                 for (int di : L.members) {
                     const Solve1D& S = descs[desc_of[di]];
@@ -2069,8 +2109,14 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
                         HIPCHK(kbg::launch_wall1d(solves[di]->fp64, S, d_descs + desc_of[di], 1, par, sst[L.stream]));
                 }
                 const bool keep = last_round && residuals && ks + per == nst;
-                HIPCHK(kbg::launch_sweep1d(L.fp64, L.nf, L.flux, L.wg_waves, d_descs, d_items, d_packs + L.pack0, (int)L.npacks,
-                                           par, keep ? d_rpart : nullptr, per, sst[L.stream]));
+                if (L.narrow) {
+                    double* rp = keep ? d_rpart + L.item0 * 12 : nullptr;
+                    HIPCHK((L.fp64 ? kbg::launch_sweep1d_narrow64 : kbg::launch_sweep1d_narrow32)(
+                        L.nf, L.narrow, L.rows, d_descs, d_items + L.item0, (int)L.nitems, par, rp, per, sst[L.stream]));
+                } else {
+                    HIPCHK(kbg::launch_sweep1d(L.fp64, L.nf, L.flux, L.wg_waves, d_descs, d_items, d_packs + L.pack0, (int)L.npacks,
+                                               par, keep ? d_rpart : nullptr, per, sst[L.stream]));
+                }
                 L.flips++;
             }
         }
@@ -2118,10 +2164,6 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
     // at both parities of the two-step launches, captured once per launch plan (the signature below: every launch's shape, stream and
     // arguments; descriptors are read from device memory, re-uploaded by every call) and reused
     // by later calls on the same batch.
-    bool any_fsm = false;
-    for (int i : others) any_fsm = any_fsm || solves[i]->has_fsm;
-    // hipFFT calls stay out of stream capture: batches with :fsm solves launch eagerly
-    const bool use_graph = ctx->graphs && !residuals && nsteps >= 2 && !noalloc && !any_fsm;
     std::string sig;
     if (use_graph) {
         auto put = [&](const void* p, size_t b) { sig.append(static_cast<const char*>(p), b); };
@@ -2137,7 +2179,8 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
         put(packs.data(), packs.size() * sizeof(kbg::Pack));
         for (const Launch& L : launches) {
             for (long long v : {(long long)L.fp64, (long long)L.nf, (long long)L.flux, (long long)L.wg_waves, (long long)L.stream,
-                                (long long)L.pack0, (long long)L.npacks, (long long)L.two})
+                                (long long)L.pack0, (long long)L.npacks, (long long)L.per, (long long)L.narrow, (long long)L.rows,
+                                (long long)L.item0, (long long)L.nitems})
                 puti(v);
             for (int di : L.members) {
                 puti(di);
@@ -2178,7 +2221,7 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
             capturing = true;
             for (int which = 0; which < 4; which++) {
                 HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeRelaxed));
-                for (Launch& L : launches) L.flips = L.two ? which >> 1 : 0;
+                for (Launch& L : launches) L.flips = L.per == 2 ? which >> 1 : 0;
                 int e = fork();
                 if (!e) e = enqueue_round((which & 1) || !two ? 1 : 2, false, 0);
                 if (!e && !(which & 1) && !two) e = enqueue_round(1, false, 1);
@@ -2203,11 +2246,11 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
         const int pairs = nsteps / 2;
         for (int t = 0; t < pairs; t++) HIPCHK(hipGraphLaunch(ctx->gexec[(t & 1) << 1], st));
         if (nsteps & 1) HIPCHK(hipGraphLaunch(ctx->gexec[(pairs & 1) << 1 | 1], st));
-        for (Launch& L : launches) L.flips = L.two ? pairs + (nsteps & 1) : nsteps;
+        for (Launch& L : launches) L.flips = L.per == 2 ? pairs + (nsteps & 1) : nsteps;
     } else {
         if ((rc = fork())) return rc;
         for (int t = 0; t < nsteps;) {
-            const int nst = two && nsteps - t >= 2 ? 2 : 1;
+            const int nst = std::min(round, nsteps - t);
             if ((rc = enqueue_round(nst, t + nst == nsteps, t & 1))) return rc;
             t += nst;
         }

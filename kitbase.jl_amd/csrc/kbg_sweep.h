@@ -32,6 +32,11 @@
 
 #include <algorithm>
 
+// Products and sums are contracted to fma within an expression, by the source, and not across expressions by
+// the optimizer, which would pick differently in each instance of the kernel: a solve's results do not depend
+// on the width and the number of time steps per launch that its batch gets.
+#pragma clang fp contract(on)
+
 #include "kbg_device.h"
 #include "kbg_types.h"
 
@@ -50,8 +55,8 @@
 namespace kbg {
 
 constexpr int kSweepLanes = 64;  // storage cells held by a wavefront
-constexpr int kSweepOut = 60;    // cells a segment updates (lanes 2 .. 61)
-constexpr int kSweepOut2 = 56;   // cells a two-step segment updates (lanes 4 .. 59)
+// cells a segment updates when a launch advances nstep time steps (lanes 2 nstep .. 63 - 2 nstep)
+constexpr int sweep_out(int nstep) { return kSweepLanes - 4 * nstep; }
 
 // DPP whole-wavefront shifts: shr1(x)[L] = x[L - 1], shl1(x)[L] = x[L + 1] (0 beyond the ends)
 KBG_D float shr1(float x) {
@@ -198,16 +203,22 @@ template <class T> struct SFace {
     T A, nl2, Ui, kb, Mxi2, M0, M1, M2, M3, M4, aL0, aL1, aL2, aR0, aR1, aR2, aT0, aT1, aT2;
 };
 
-// NSTEP = 2 advances the segment two time steps in one pass (KFVS, no boundary-face buffers): the
-// window holds 4 halo cells per side, step 1's f^{n+1} stays in the registers that carry G, and only
-// f^{n+2} is stored -- one read and one write of f per two steps.  Cells the first step does not
-// update (boundary or ghost cells) keep f^n, reloaded for the second step.
-template <class T, int NF, int FLUX, int LIMK, bool SHAK, int NSTEP>
+// NSTEP > 1 advances the segment NSTEP time steps in one pass (KFVS, no boundary-face buffers): the
+// window holds 2 NSTEP halo cells per side, a step's f^{n+1} stays in the registers that carry G, and only
+// the last step's is stored -- one read and one write of f per NSTEP steps.  Every step leaves two more
+// lanes per side without a valid neighbour; they feed no stored cell.  Cells update! does not step
+// (boundary or ghost cells) keep f^n, reloaded for every further step.
+//
+// VW: most velocities per wavefront.  NARROW (small launches, k_sweep1d_narrow): more wavefronts per item
+// than sweep_nw, and every chunk's sums get an LDS row of their own, which wavefront 0 adds in the order
+// of the sweep_nw wavefronts' chunk sums -- the same values whatever the width.
+template <class T, int NF, int FLUX, int LIMK, bool SHAK, int NSTEP, int VW, bool NARROW>
 KBG_D void sweep1d(const Solve1D& S, const WorkItem& wi, int par, int lane, int wave, int NW, double* lds,
                    double* rrow) {
-    static_assert(NSTEP == 1 || FLUX == KFVS, "two steps per pass are built for KFVS");
+    static_assert(NSTEP == 1 || FLUX == KFVS, "several steps per pass are built for KFVS");
     using C = SweepCfg<T, NF, FLUX>;
-    constexpr int VW = C::VW, CH = C::CH, NRAW = C::NRAW, NR = C::NR;
+    constexpr int CH = C::CH, NRAW = C::NRAW, NR = C::NR;
+    constexpr int OUT = sweep_out(NSTEP);
     const int nx = S.nx, ng = S.ng, nv = S.nv, N = nx + 2 * ng;
     const long np = S.np;
     const int in = (S.cur + par) & 1;
@@ -239,14 +250,12 @@ KBG_D void sweep1d(const Solve1D& S, const WorkItem& wi, int par, int lane, int 
     // KFVS carries half slopes (one multiply less in the limiter): the half cell width doubles
     constexpr bool HALF = FLUX == KFVS;
     const T dxs = HALF ? T(2.0 * dxh64) : dxh;
-    // cells stored by this item (lanes 2..61, or 4..59 for two steps), and, for two steps, the
-    // cells the first step updates (every stepped cell with two neighbours per side in the window)
-    const bool upd = NSTEP == 1 ? (lane >= 2 && lane < 2 + kSweepOut && i >= wi.c0 && i <= wi.c1)
-                                : (lane >= 4 && lane < 4 + kSweepOut2 && i >= wi.c0 && i <= wi.c1);
-    const bool upd_mid = NSTEP == 2 && lane >= 2 && lane < 62 && i >= S.upd_lo && i <= S.upd_hi;
-    // a wavefront whose lanes 2..61 (the ones the second step reads) hold cells the first step leaves
-    // alone -- boundary or ghost cells -- reloads their f^n; lanes 0, 1, 62, 63 feed no stored cell
-    const bool keep_any = NSTEP == 2 && __ballot(!upd_mid && lane >= 2 && lane < 62 && k >= 0 && k < N) != 0ull;
+    // cells stored by this item, and the cells update! steps
+    const bool upd = lane >= 2 * NSTEP && lane < 2 * NSTEP + OUT && i >= wi.c0 && i <= wi.c1;
+    const bool upd_any = i >= S.upd_lo && i <= S.upd_hi;
+    // a wavefront whose lanes 2..61 (the ones a further step reads) hold cells update! leaves alone
+    // -- boundary or ghost cells -- reloads their f^n
+    const bool keep_any = NSTEP > 1 && __ballot(!upd_any && lane >= 2 && lane < 62 && k >= 0 && k < N) != 0ull;
     // the lane's left face comes from the boundary-face buffers (only where a stepped cell uses it)
     const bool bufL = (i == 1 && S.faceL_buf && S.upd_lo == 1) || (i == nx + 1 && S.faceR_buf && S.upd_hi == nx);
     const int bside = i == 1 ? 0 : 1;
@@ -268,8 +277,8 @@ KBG_D void sweep1d(const Solve1D& S, const WorkItem& wi, int par, int lane, int 
         conserve_prim<3>(wq, S.gam, pq);
     }
     const double Uo64 = SHAK ? pq[1] : 0.0;
-    // FP32: the stored f of the lane's cell departs from M~(prim^n) (for the second step of a pass,
-    // prim^{n+1} where the first step updated the cell); lanes outside the solve read 0
+    // FP32: the stored f of the lane's cell departs from M~(prim^n) (for a further step of a pass,
+    // prim^{n+1} where the step before updated the cell); lanes outside the solve read 0
     float dA = 0.f, dnl = 0.f, dU = 0.f, dkb = 0.f;
     if constexpr (DEL) {
         const MaxwCoef mc = maxw_coef(pq, K);
@@ -338,6 +347,7 @@ KBG_D void sweep1d(const Solve1D& S, const WorkItem& wi, int par, int lane, int 
 
     // ---- pass 1: slopes, face fluxes, moment sums, transport update
     const int ivw = sweep_item_vw(nv, NW);  // this item's velocities per wavefront (<= VW)
+    const int cpw = ivw / CH;               // its chunks per wavefront
     const int vbeg = wave * ivw;
     const int vend = min(nv, vbeg + ivw);
     T G[NF][VW];
@@ -382,7 +392,7 @@ KBG_D void sweep1d(const Solve1D& S, const WorkItem& wi, int par, int lane, int 
             for (int q = 0; q < NF; q++) {
                 T f;
                 if constexpr (SS == 0) f = fr[q][j];
-                else f = G[q][c * CH + j];  // the first step's f^{n+1} (departure in FP32), still in registers
+                else f = G[q][c * CH + j];  // the last step's f^{n+1} (departure in FP32), still in registers
                 dq[q] = f;
                 if constexpr (DEL) f = (q == 0 ? T(Md[j]) : T(maxw_b(Md[j], dkb))) + f;
                 fq[q] = f;
@@ -475,15 +485,20 @@ KBG_D void sweep1d(const Solve1D& S, const WorkItem& wi, int par, int lane, int 
 #pragma unroll
             for (int q = 0; q < NF; q++) G[q][c * CH + j] = (DEL ? dq[q] : fq[q]) + (ffq[q] - shl1(ffq[q])) * rdx;
         });
+        if constexpr (NARROW) {
 #pragma unroll
-        for (int m = 0; m < NR; m++) acc[m] += double(part[m]);
+            for (int m = 0; m < NR; m++) lds[((wave * cpw + c) * NR + m) * kSweepLanes + lane] = double(part[m]);
+        } else {
+#pragma unroll
+            for (int m = 0; m < NR; m++) acc[m] += double(part[m]);
+        }
     };
     using I0 = std::integral_constant<int, 0>;
     using I1 = std::integral_constant<int, 1>;
     using I2 = std::integral_constant<int, 2>;
     using BT = std::integral_constant<bool, true>;
     using BF = std::integral_constant<bool, false>;
-    double wkeep[3] = {0.0, 0.0, 0.0}, pkeep[3] = {1.0, 0.0, 1.0};  // wavefront 0: step 1's w, prim
+    double wkeep[3] = {0.0, 0.0, 0.0}, pkeep[3] = {1.0, 0.0, 1.0};  // wavefront 0: the last step's w, prim
     static_for<NSTEP>([&](auto sc) {
         constexpr int s = sc;
         constexpr bool LAST = s == NSTEP - 1;
@@ -514,15 +529,35 @@ KBG_D void sweep1d(const Solve1D& S, const WorkItem& wi, int par, int lane, int 
         // ---- wavefront 0 adds the wavefronts' sums (fixed order) and runs the cells' step! chain;
         // the others take its coefficients from LDS
         T An, A1, nl2, Un, inv, rTi, kbn, pre = 0, Ao = 0, nlo2 = 0, Uo = 0, lo2 = 0, kbo = 0;
-        T* coef = (T*)(lds + (size_t)NW * NR * kSweepLanes);  // [13][64]
+        T* coef = (T*)(lds + (size_t)(NARROW ? (nv + CH - 1) / CH : NW) * NR * kSweepLanes);  // [13][64]
         if (NW > 1) {
+            if constexpr (!NARROW) {
 #pragma unroll
-            for (int m = 0; m < NR; m++) lds[(wave * NR + m) * kSweepLanes + lane] = acc[m];
+                for (int m = 0; m < NR; m++) lds[(wave * NR + m) * kSweepLanes + lane] = acc[m];
+            }
             __syncthreads();
         }
         if (wave == 0) {
             double tot[NR];
-            if (NW > 1) {
+            if constexpr (NARROW) {
+                // chunk by chunk within the velocities of one of the sweep_nw wavefronts, then these in order
+                const int gch = sweep_item_vw(nv, sweep_nw(sizeof(T) == 8, NF, nv)) / CH, nch = (nv + CH - 1) / CH;
+                double a[NR];
+#pragma unroll
+                for (int m = 0; m < NR; m++) tot[m] = a[m] = 0.0;
+                for (int c0 = 0; c0 < nch; c0 += gch) {
+                    const int c1 = min(nch, c0 + gch);
+#pragma unroll
+                    for (int m = 0; m < NR; m++) a[m] = 0.0;
+#pragma unroll 4
+                    for (int c = c0; c < c1; c++) {
+#pragma unroll
+                        for (int m = 0; m < NR; m++) a[m] += lds[(c * NR + m) * kSweepLanes + lane];
+                    }
+#pragma unroll
+                    for (int m = 0; m < NR; m++) tot[m] += a[m];
+                }
+            } else if (NW > 1) {
 #pragma unroll
                 for (int m = 0; m < NR; m++) {
                     double sm = 0.0;
@@ -578,7 +613,7 @@ KBG_D void sweep1d(const Solve1D& S, const WorkItem& wi, int par, int lane, int 
 
             // the cell's step! coefficients (FP64 chain, lane-parallel)
             conserve_prim<3>(wn, S.gam, pn);
-            if (LAST ? upd : upd_mid) flag_health(S.health, prim_health<3>(pn));
+            if (LAST ? upd : (upd_any && lane >= 2 * (s + 1) && lane < kSweepLanes - 2 * (s + 1))) flag_health(S.health, prim_health<3>(pn));
             const T rT = relax_ratio<T>(pn[0], pn[2], S.mu, S.om, dt);
             if constexpr (DEL) {
                 // FP32: M~^{n+1} from the same coefficients every kernel evaluates M~ with
@@ -613,11 +648,11 @@ KBG_D void sweep1d(const Solve1D& S, const WorkItem& wi, int par, int lane, int 
                 }
             }
             if constexpr (!LAST) {
-                // the first of two steps: the cells it updates carry w, prim to the second
+                // the cells this step updates carry w, prim to the next
 #pragma unroll
                 for (int m = 0; m < 3; m++) {
-                    wkeep[m] = upd_mid ? wn[m] : wo[m];
-                    pkeep[m] = upd_mid ? pn[m] : po[m];
+                    wkeep[m] = upd_any ? wn[m] : wo[m];
+                    pkeep[m] = upd_any ? pn[m] : po[m];
                 }
             }
             if (LAST && upd) {
@@ -675,7 +710,7 @@ KBG_D void sweep1d(const Solve1D& S, const WorkItem& wi, int par, int lane, int 
                 }
             }
         }
-        if constexpr (!LAST) UoT = Un;  // the second step's Shakhov heat flux is about prim^{n+1}
+        if constexpr (!LAST) UoT = Un;  // a further step's Shakhov heat flux is about prim^{n+1}
 
         // ---- pass 2: relaxation toward M (+ Shakhov) and the store of f^{n+1}
         // M at the chunk's nodes: one exp per node, or -- FP32 on equally spaced nodes -- the product
@@ -771,7 +806,7 @@ KBG_D void sweep1d(const Solve1D& S, const WorkItem& wi, int par, int lane, int 
                     }
                 }
             } else {
-                // f^{n+1} becomes the second step's input; cells the first step left alone keep f^n
+                // f^{n+1} becomes the next step's input; cells this one left alone keep f^n
                 static_for<CH>([&](auto jc) {
                     constexpr int j = jc;
 #pragma unroll
@@ -784,7 +819,7 @@ KBG_D void sweep1d(const Solve1D& S, const WorkItem& wi, int par, int lane, int 
 #pragma unroll
                             for (int q = 0; q < NF; q++) {
                                 const T f0 = bload((T*)nullptr, fin, voff, (q * nv + vb + j) * rowb);
-                                G[q][c * CH + j] = upd_mid ? G[q][c * CH + j] : f0;
+                                G[q][c * CH + j] = upd_any ? G[q][c * CH + j] : f0;
                             }
                         }
                     });
@@ -792,30 +827,30 @@ KBG_D void sweep1d(const Solve1D& S, const WorkItem& wi, int par, int lane, int 
             }
         });
         if constexpr (DEL && !LAST) {
-            // the second step's departures are from M~(prim^{n+1}) where the first step updated the cell
-            dA = upd_mid ? float(A1) : dA;
-            dnl = upd_mid ? float(nl2) : dnl;
-            dU = upd_mid ? float(Un) : dU;
-            dkb = upd_mid ? (NF == 2 ? float(kbn) : dkb) : dkb;
+            // the next step's departures are from M~(prim^{n+1}) where this one updated the cell
+            dA = upd_any ? float(A1) : dA;
+            dnl = upd_any ? float(nl2) : dnl;
+            dU = upd_any ? float(Un) : dU;
+            dkb = upd_any ? (NF == 2 ? float(kbn) : dkb) : dkb;
         }
     });
 }
 
-template <class T, int NF, int FLUX, int LIMK, int NSTEP>
+template <class T, int NF, int FLUX, int LIMK, int NSTEP, int VW, bool NARROW>
 KBG_D void sweep_coll(const Solve1D& S, const WorkItem& wi, int par, int lane, int wave, int NW, double* lds, double* rrow) {
-    if (S.coll == SHAKHOV) sweep1d<T, NF, FLUX, LIMK, true, NSTEP>(S, wi, par, lane, wave, NW, lds, rrow);
-    else sweep1d<T, NF, FLUX, LIMK, false, NSTEP>(S, wi, par, lane, wave, NW, lds, rrow);
+    if (S.coll == SHAKHOV) sweep1d<T, NF, FLUX, LIMK, true, NSTEP, VW, NARROW>(S, wi, par, lane, wave, NW, lds, rrow);
+    else sweep1d<T, NF, FLUX, LIMK, false, NSTEP, VW, NARROW>(S, wi, par, lane, wave, NW, lds, rrow);
 }
-template <class T, int NF, int FLUX, int NSTEP>
+template <class T, int NF, int FLUX, int NSTEP, int VW, bool NARROW>
 KBG_D void sweep_lim(const Solve1D& S, const WorkItem& wi, int par, int lane, int wave, int NW, double* lds, double* rrow) {
-    if (!S.interp2) sweep_coll<T, NF, FLUX, LIM_NONE, NSTEP>(S, wi, par, lane, wave, NW, lds, rrow);
-    else if (S.limiter == VANLEER) sweep_coll<T, NF, FLUX, LIM_VANLEER, NSTEP>(S, wi, par, lane, wave, NW, lds, rrow);
-    else sweep_coll<T, NF, FLUX, LIM_GENERIC, NSTEP>(S, wi, par, lane, wave, NW, lds, rrow);
+    if (!S.interp2) sweep_coll<T, NF, FLUX, LIM_NONE, NSTEP, VW, NARROW>(S, wi, par, lane, wave, NW, lds, rrow);
+    else if (S.limiter == VANLEER) sweep_coll<T, NF, FLUX, LIM_VANLEER, NSTEP, VW, NARROW>(S, wi, par, lane, wave, NW, lds, rrow);
+    else sweep_coll<T, NF, FLUX, LIM_GENERIC, NSTEP, VW, NARROW>(S, wi, par, lane, wave, NW, lds, rrow);
 }
 
-// LDS of one item (doubles): the wavefronts' moment sums and wavefront 0's cell coefficients
-template <class T, int NF, int FLUX> constexpr size_t sweep_lds_item(int nw) {
-    return nw > 1 ? (size_t)nw * SweepCfg<T, NF, FLUX>::NR * kSweepLanes + (13 * kSweepLanes * sizeof(T) + 7) / 8 : 0;
+// LDS of one item (doubles): the wavefronts' (rows: chunks') moment sums and wavefront 0's cell coefficients
+template <class T, int NF, int FLUX> constexpr size_t sweep_lds_item(int nw, int rows = 0) {
+    return nw > 1 || rows ? (size_t)(rows ? rows : nw) * SweepCfg<T, NF, FLUX>::NR * kSweepLanes + (13 * kSweepLanes * sizeof(T) + 7) / 8 : 0;
 }
 
 // occupancy target: 4 wavefronts per SIMD (<= 128 VGPRs) for the FP32 one-distribution sweeps,
@@ -855,13 +890,43 @@ __global__ __launch_bounds__(64 * kSweepMaxWaves) __attribute__((amdgpu_waves_pe
     const Solve1D& S = solves[wi.solve];
     double* lds = kbg_sweep_lds + (size_t)sub * sweep_lds_item<T, NF, FLUX>(NW);
     double* rrow = rpart ? rpart + (size_t)it * 12 : nullptr;
+    constexpr int VW = SweepCfg<T, NF, FLUX>::VW;
     if constexpr (FLUX == KFVS) {
         if (nstep == 2) {
-            sweep_lim<T, NF, FLUX, 2>(S, wi, par, lane, wave, NW, lds, rrow);
+            sweep_lim<T, NF, FLUX, 2, VW, false>(S, wi, par, lane, wave, NW, lds, rrow);
             return;
         }
     }
-    sweep_lim<T, NF, FLUX, 1>(S, wi, par, lane, wave, NW, lds, rrow);
+    sweep_lim<T, NF, FLUX, 1, VW, false>(S, wi, par, lane, wave, NW, lds, rrow);
+}
+
+// The KFVS sweep of small launches: a launch with less than a few wavefronts per SIMD takes as long as one
+// wavefront's passes over its velocities and the cells' FP64 chain, so its items get up to 16 wavefronts of
+// at most sweep_vw_narrow velocities (8 when nv allows), and up to four time steps share a launch, whose
+// start (descriptor and f loads, about 5 us) they split.  One item per workgroup of nw wavefronts.
+// Sod, 100 x 64 FP64: 13.6 us per step with k_sweep1d, 6.5 with this kernel; 24 ragged FP32 tubes 21 / 13 us
+// (more sizes at the rule that picks it, kbg_api.hip).
+template <class T, int NF>
+__global__ __launch_bounds__(64 * kSweepNarrowWaves) void k_sweep1d_narrow(const Solve1D* __restrict__ solves,
+                                                                          const WorkItem* __restrict__ items, int nitems, int par,
+                                                                          double* __restrict__ rpart, int nstep) {
+    extern __shared__ double kbg_sweep_lds[];
+    const int it = blockIdx.x;
+    if (it >= nitems) return;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const WorkItem wi = items[it];
+    if (wave >= wi.nw) {  // an unused wavefront takes part in the barriers (two per time step)
+        if (wi.nw > 1)
+            for (int b = 0; b < 2 * nstep; b++) __syncthreads();
+        return;
+    }
+    const Solve1D& S = solves[wi.solve];
+    double* rrow = rpart ? rpart + (size_t)it * 12 : nullptr;
+    constexpr int VW = sweep_vw_narrow(NF);
+    if (nstep == 4) sweep_lim<T, NF, KFVS, 4, VW, true>(S, wi, par, lane, wave, wi.nw, kbg_sweep_lds, rrow);
+    else if (nstep == 2) sweep_lim<T, NF, KFVS, 2, VW, true>(S, wi, par, lane, wave, wi.nw, kbg_sweep_lds, rrow);
+    else sweep_lim<T, NF, KFVS, 1, VW, true>(S, wi, par, lane, wave, wi.nw, kbg_sweep_lds, rrow);
 }
 
 template <class T, int NF, int FLUX>
@@ -873,6 +938,20 @@ hipError_t launch_sweep_t(int wg_waves, const Solve1D* d_solves, const WorkItem*
     hipLaunchKernelGGL((k_sweep1d<T, NF, FLUX>), dim3(npacks), dim3(64 * wg_waves), lds * sizeof(double), st, d_solves, d_items,
                        d_packs, npacks, par, d_rpart, nstep);
     return hipGetLastError();
+}
+
+// wg_waves: the largest nw of the items; rows: the most velocity chunks of their solves
+template <class T, int NF>
+hipError_t launch_sweep_narrow_t(int wg_waves, int rows, const Solve1D* d_solves, const WorkItem* d_items, int nitems, int par,
+                                 double* d_rpart, int nstep, hipStream_t st) {
+    const size_t lds = sweep_lds_item<T, NF, KFVS>(wg_waves, rows) * sizeof(double);
+    hipLaunchKernelGGL((k_sweep1d_narrow<T, NF>), dim3(nitems), dim3(64 * wg_waves), lds, st, d_solves, d_items, nitems, par, d_rpart, nstep);
+    return hipGetLastError();
+}
+template <class T, int NF> hipError_t sweep_narrow_attr_t() {
+    constexpr int rows = kSweepNarrowWaves * sweep_vw_narrow(NF) / kVChunk;
+    return hipFuncSetAttribute((const void*)k_sweep1d_narrow<T, NF>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               int(sweep_lds_item<T, NF, KFVS>(kSweepNarrowWaves, rows) * sizeof(double)));
 }
 
 }  // namespace kbg

@@ -152,7 +152,7 @@ struct Pack {
 // ---- launchers (kbg_sweep.h, kbg_1d.hip, kbg_2d.hip) --------------------------------------------------------
 // All return hipSuccess or the launch error; `fp64` selects the storage type.
 // nstep: time steps per launch, 1, or 2 for KFVS solves without boundary-face buffers (items of at most
-// kSweepOut2 = 56 cells); par counts launches, not steps
+// sweep_out(nstep) cells); par counts launches, not steps
 hipError_t launch_sweep1d(bool fp64, int nf, int flux, int wg_waves, const Solve1D* d_solves, const WorkItem* d_items,
                           const Pack* d_packs, int npacks, int par, double* d_rpart, int nstep, hipStream_t st);
 // velocities per wavefront of the sweep for a storage type / distribution count (a multiple of 8),
@@ -170,6 +170,16 @@ constexpr int sweep_nw(bool fp64, int nf, int nv) {
          : (nv + sweep_vw(fp64, nf) - 1) / sweep_vw(fp64, nf) <= 2 ? 2
          : (nv + sweep_vw(fp64, nf) - 1) / sweep_vw(fp64, nf) <= 4 ? 4 : 8;
 }
+// The narrow KFVS sweep of small launches: nstep 1, 2 or 4, items of nw <= kSweepNarrowWaves wavefronts of at
+// most sweep_vw_narrow velocities, wg_waves the largest nw, rows the most 8-velocity chunks of the solves
+constexpr int kSweepNarrowWaves = 16;
+constexpr int sweep_vw_narrow(int nf) { return 16 / nf; }
+hipError_t launch_sweep1d_narrow32(int nf, int wg_waves, int rows, const Solve1D* d_solves, const WorkItem* d_items, int nitems,
+                                   int par, double* d_rpart, int nstep, hipStream_t st);
+hipError_t launch_sweep1d_narrow64(int nf, int wg_waves, int rows, const Solve1D* d_solves, const WorkItem* d_items, int nitems,
+                                   int par, double* d_rpart, int nstep, hipStream_t st);
+hipError_t sweep_narrow_attr32();
+hipError_t sweep_narrow_attr64();
 // velocities per wavefront of an item (a multiple of 8, at most sweep_vw)
 constexpr int sweep_item_vw(int nv, int nw) { return ((nv + nw - 1) / nw + 7) / 8 * 8; }
 // Conversions of an FP32 swept solve's f buffer `buf` between its stored departure f - M~(prim) and f:

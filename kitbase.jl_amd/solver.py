@@ -460,8 +460,8 @@ class Context:
         _lib.check(self.lib.kbg_ctx_set_sweep_steps(self.handle, int(steps)))
 
     def set_sweep_vw(self, vw: int):
-        """Most velocities per fused-sweep wavefront, 0 (full width), 8, 16 or 32 (kbg_ctx_set_sweep_vw):
-        smaller values shorten the passes of small, latency-bound batches."""
+        """Most velocities per fused-sweep wavefront, 0 (by the size of the batch), 8, 16, 32 or 64
+        (kbg_ctx_set_sweep_vw): smaller values shorten the passes of small, latency-bound batches."""
         _lib.check(self.lib.kbg_ctx_set_sweep_vw(self.handle, int(vw)))
 
     def schedule(self) -> tuple[int, int]:

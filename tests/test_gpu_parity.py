@@ -641,3 +641,50 @@ def test_two_steps_per_sweep_launch_bitwise(gpu_ctx, case, nsteps):
     finally:
         gpu_ctx.set_schedule(*old)
         gpu_ctx.set_sweep_vw(0)
+
+
+# ---------------------------------------------------------------- widths of the 1D sweep
+
+@pytest.mark.parametrize("space,collision,mesh", [("1d1f1v", "bgk", "rectangle"), ("1d1f1v", "shakhov", "newton"),
+                                                  ("1d2f1v", "bgk", "newton"), ("1d2f1v", "shakhov", "rectangle")])
+@pytest.mark.parametrize("nv", [7, 8, 9, 64, 101, 128, 129, 256])
+def test_sweep_width_and_steps_per_launch_do_not_change_a_result(gpu_ctx, space, collision, mesh, nv):
+    """The narrow sweep (few velocities per wavefront, up to four steps per launch; the choice for a small
+    launch) against the full-width one (a cap of 64 velocities) and against one step per launch, bit for bit:
+    nv around 8-velocity chunks, around 16 wavefronts of 8 (128, 129) and the widest the narrow sweep takes
+    (256); 53, 57 and 64 cells around the segments of one, two and four steps; 7 = 4 + 2 + 1 steps, and a
+    call that ends after 3."""
+    rng = np.random.default_rng(nv)
+    try:
+        for precision in ("fp64", "fp32"):
+            for nx, interp in ((5, 2), (53, 2), (57, 1), (64, 2)):
+                if space == "1d1f1v":
+                    cfg = kb.configs.sod_1d1f1v(nx=nx, nu=nv, collision=collision, vMeshType=mesh, interpOrder=interp)
+                else:
+                    cfg = kb.configs.shock_1d2f1v(nx=nx, nu=nv, collision=collision, vMeshType=mesh, interpOrder=interp, flux="kfvs")
+                ks = kb.SolverSet(cfg)
+                ctr, face = kb.init_fvm(ks)
+                ctr.f *= 1.0 + 0.01 * rng.random(ctr.f.shape)
+                dt = kb.timestep(ks, ctr)
+                got = []
+                for vw, steps in ((0, 2), (64, 2), (64, 1), (8, 1)):
+                    gpu_ctx.set_sweep_vw(vw)
+                    gpu_ctx.set_sweep_steps(steps)
+                    c = copy.deepcopy(ctr)
+                    dev = kb.DeviceSolve(ks, c, face, precision, gpu_ctx)
+                    dev.step(dt, 3)
+                    dev.step(dt, 7)
+                    dev.download(c)
+                    dev.close()
+                    got.append(c)
+                for c in got[1:]:
+                    np.testing.assert_array_equal(c.f, got[0].f)
+                    np.testing.assert_array_equal(c.w, got[0].w)
+                    np.testing.assert_array_equal(c.prim, got[0].prim)
+                if precision == "fp64":
+                    co, fo = copy.deepcopy(ctr), copy.deepcopy(face)
+                    oracle.OracleSolve(ks, co, fo).run(dt, 10)
+                    assert rel_max(got[0].f, co.f) <= 1e-10 and rel_max(got[0].w, co.w) <= 1e-10
+    finally:
+        gpu_ctx.set_sweep_vw(0)
+        gpu_ctx.set_sweep_steps(2)
