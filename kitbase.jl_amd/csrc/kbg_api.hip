@@ -92,6 +92,13 @@ struct kbg_ctx {
     static constexpr size_t kPinBytes = size_t(32) << 20;
     void* pin[2] = {};
     hipEvent_t pin_ev[2] = {};
+    // download of a swept 1D solve: pinned blocks of at most kDownBytes (of 32 cells, if those are more) that
+    // the device writes in host order, grown to what the largest download so far asked for
+    static constexpr size_t kDownBytes = size_t(16) << 20;
+    void* down[2] = {};
+    size_t down_cap[2] = {};
+    hipEvent_t down_ev[2] = {};
+    std::mutex down_mx;
 };
 
 struct kbg_solve {
@@ -267,13 +274,6 @@ template <class T> void to_layout(const Solve1D& S, int N, const double* src, T*
             for (int v = 0; v < nv; v++)
                 dst[(size_t)k * S.fcs + (size_t)q * S.fqs + (size_t)v * S.fvs] = T(src[((size_t)k * nf + q) * nv + v]);
 }
-template <class T> void from_layout(const Solve1D& S, int N, const T* src, double* dst) {
-    const int nf = S.nf, nv = S.nv;
-    for (int k = 0; k < N; k++)
-        for (int q = 0; q < nf; q++)
-            for (int v = 0; v < nv; v++)
-                dst[((size_t)k * nf + q) * nv + v] = double(src[(size_t)k * S.fcs + (size_t)q * S.fqs + (size_t)v * S.fvs]);
-}
 size_t f_elems_1d(const Solve1D& S, int N) { return S.swept ? (size_t)S.nf * S.nv * S.np : (size_t)N * S.nf * S.nv; }
 
 int put_f1d(kbg_solve* s, void* dst, const double* src) {
@@ -289,23 +289,6 @@ int put_f1d(kbg_solve* s, void* dst, const double* src) {
         to_layout<float>(S, s->N, src, tmp.data());
         HIPCHK(hipMemcpyAsync(dst, tmp.data(), n * 4, hipMemcpyHostToDevice, s->ctx->stream));
         HIPCHK(hipStreamSynchronize(s->ctx->stream));
-    }
-    return KBG_OK;
-}
-
-int get_f1d(kbg_solve* s, double* dst, const void* src) {
-    const Solve1D& S = s->h1;
-    const size_t n = f_elems_1d(S, s->N);
-    if (s->fp64) {
-        std::vector<double> tmp(n);
-        HIPCHK(hipMemcpyAsync(tmp.data(), src, n * 8, hipMemcpyDeviceToHost, s->ctx->stream));
-        HIPCHK(hipStreamSynchronize(s->ctx->stream));
-        from_layout<double>(S, s->N, tmp.data(), dst);
-    } else {
-        std::vector<float> tmp(n);
-        HIPCHK(hipMemcpyAsync(tmp.data(), src, n * 4, hipMemcpyDeviceToHost, s->ctx->stream));
-        HIPCHK(hipStreamSynchronize(s->ctx->stream));
-        from_layout<float>(S, s->N, tmp.data(), dst);
     }
     return KBG_OK;
 }
@@ -329,20 +312,45 @@ int put_f1d_delta(kbg_solve* s, const double* src, std::initializer_list<int> bu
     return KBG_OK;
 }
 
-// f of buffer `buf` as FP64 on the host, exactly M~ + departure
-int get_f1d_delta(kbg_solve* s, double* dst, int buf) {
+// A swept solve's state (any of w, prim, f NULL: not wanted): blocks of cells that k_down1d writes into one
+// pinned buffer while the host copies the other one out
+int down_1d(kbg_solve* s, double* w, double* prim, double* f) {
+    kbg_ctx* c = s->ctx;
     const Solve1D& S = s->h1;
-    const size_t n = f_elems_1d(S, s->N);
-    std::vector<double> tmp(n);
-    double* stage = nullptr;
-    HIPCHK(hipMalloc((void**)&stage, n * 8));
-    hipError_t e = hipMemsetAsync(stage, 0, n * 8, s->ctx->stream);
-    if (e == hipSuccess) e = kbg::launch_delta1d(S, s->d1, stage, 1, buf, s->ctx->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(tmp.data(), stage, n * 8, hipMemcpyDeviceToHost, s->ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(s->ctx->stream);
-    (void)hipFree(stage);
-    if (e != hipSuccess) return fail(KBG_ERR_HIP, std::string("departure download: ") + hipGetErrorString(e));
-    from_layout<double>(S, s->N, tmp.data(), dst);
+    std::lock_guard<std::mutex> lock(c->down_mx);
+    const size_t N = s->N, fc = size_t(S.nf) * S.nv, cell = (fc + 6) * 8;
+    const size_t want = std::min(kbg_ctx::kDownBytes, std::max(size_t(256) << 10, N * cell / 4));
+    const size_t per = std::min(N, std::max<size_t>(1, want / cell / 32) * 32), nch = (N + per - 1) / per;
+    for (int b = 0; b < (nch > 1 ? 2 : 1); b++) {
+        if (c->down_cap[b] < per * cell) {
+            if (c->down[b]) HIPCHK(hipHostFree(c->down[b]));
+            c->down[b] = nullptr;
+            c->down_cap[b] = 0;
+            size_t cap = size_t(64) << 10;
+            while (cap < per * cell) cap *= 2;
+            HIPCHK(hipHostMalloc(&c->down[b], cap, hipHostMallocDefault));
+            c->down_cap[b] = cap;
+        }
+        if (!c->down_ev[b]) HIPCHK(hipEventCreateWithFlags(&c->down_ev[b], hipEventDisableTiming));
+    }
+    auto issue = [&](size_t k) -> int {
+        const int b = int(k & 1);
+        HIPCHK(kbg::launch_down1d(s->fp64, S.delta && !s->rep_full, S, S.cur, int(k * per), int(std::min(per, N - k * per)),
+                                  static_cast<double*>(c->down[b]), c->stream));
+        HIPCHK(hipEventRecord(c->down_ev[b], c->stream));
+        return KBG_OK;
+    };
+    int rc;
+    if ((rc = issue(0))) return rc;
+    for (size_t k = 0; k < nch; k++) {
+        if (k + 1 < nch && (rc = issue(k + 1))) return rc;  // into the buffer block k - 1 was copied from
+        HIPCHK(hipEventSynchronize(c->down_ev[k & 1]));
+        const size_t k0 = k * per, n = std::min(per, N - k0);
+        const double* src = static_cast<const double*>(c->down[k & 1]);
+        if (f) par_for(n * fc, [&](size_t a, size_t e) { std::memcpy(f + k0 * fc + a, src + a, (e - a) * 8); });
+        if (w) std::memcpy(w + k0 * 3, src + n * fc, n * 24);
+        if (prim) std::memcpy(prim + k0 * 3, src + n * (fc + 3), n * 24);
+    }
     return KBG_OK;
 }
 
@@ -350,7 +358,7 @@ int get_f1d_delta(kbg_solve* s, double* dst, int buf) {
 int to_full_rep(kbg_solve* s) {
     if (s->rep_full) return KBG_OK;
     if (s->d.dim == 1 && s->h1.delta) {
-        HIPCHK(kbg::launch_delta1d(s->h1, s->d1, nullptr, 2, s->h1.cur, s->ctx->stream));
+        HIPCHK(kbg::launch_delta1d(s->h1, s->d1, nullptr, 1, s->h1.cur, s->ctx->stream));
         s->rep_full = true;
     } else if (s->d.dim == 2 && s->h2.delta) {
         HIPCHK(kbg::launch_delta2d(s->h2, s->d2, 2, s->ctx->stream));
@@ -801,6 +809,8 @@ int kbg_ctx_destroy(kbg_ctx* c) {
     for (int b = 0; b < 2; b++) {
         if (c->pin[b]) (void)hipHostFree(c->pin[b]);
         if (c->pin_ev[b]) (void)hipEventDestroy(c->pin_ev[b]);
+        if (c->down[b]) (void)hipHostFree(c->down[b]);
+        if (c->down_ev[b]) (void)hipEventDestroy(c->down_ev[b]);
     }
     for (auto& sd : c->side)
         if (sd) (void)hipStreamDestroy(sd);
@@ -1444,14 +1454,16 @@ int kbg_download(kbg_solve* s, double* w, double* prim, double* f) {
     }
     if (s->d.dim == 1) {
         Solve1D& S = s->h1;
+        if (S.swept && f) return down_1d(s, w, prim, f);
         if (w && (rc = get_f64(s, w, S.w[S.cur], N * s->nw))) return rc;
         if (prim && (rc = get_f64(s, prim, S.prim, N * s->nw))) return rc;
-        if (f) {
-            if (S.delta && !s->rep_full) {
-                if ((rc = push1d(s)) || (rc = get_f1d_delta(s, f, S.cur))) return rc;
-            } else if ((rc = get_f1d(s, f, S.f[S.cur]))) {
-                return rc;
-            }
+        if (f) {  // [N][nf][nv] as on the host
+            const size_t n = N * s->RS;
+            if (s->fp64) return get_f64(s, f, static_cast<const double*>(S.f[S.cur]), n);
+            std::vector<float> tmp(n);
+            HIPCHK(hipMemcpyAsync(tmp.data(), S.f[S.cur], n * 4, hipMemcpyDeviceToHost, s->ctx->stream));
+            HIPCHK(hipStreamSynchronize(s->ctx->stream));
+            for (size_t i = 0; i < n; i++) f[i] = double(tmp[i]);
         }
         return KBG_OK;
     }
@@ -2060,7 +2072,7 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
     for (int i : fused) {
         kbg_solve* s = solves[i];
         if (s->h1.delta && s->rep_full) {
-            HIPCHK(kbg::launch_delta1d(s->h1, d_descs + desc_of[i], nullptr, 3, s->h1.cur, st));
+            HIPCHK(kbg::launch_delta1d(s->h1, d_descs + desc_of[i], nullptr, 2, s->h1.cur, st));
             s->rep_full = false;
         }
     }

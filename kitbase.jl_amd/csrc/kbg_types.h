@@ -183,9 +183,12 @@ hipError_t sweep_narrow_attr64();
 // velocities per wavefront of an item (a multiple of 8, at most sweep_vw)
 constexpr int sweep_item_vw(int nv, int nw) { return ((nv + nw - 1) / nw + 7) / 8 * 8; }
 // Conversions of an FP32 swept solve's f buffer `buf` between its stored departure f - M~(prim) and f:
-// mode 0: FP64 staging (the swept layout) -> departure; 1: departure -> FP64 staging (exact, f = M~ + d);
-// 2: departure -> f in place (FP32); 3: f -> departure in place
+// mode 0: FP64 staging (the swept layout) -> departure; 1: departure -> f in place (FP32); 2: f -> departure
+// in place
 hipError_t launch_delta1d(const Solve1D& S, const Solve1D* d_S, double* stage, int mode, int buf, hipStream_t st);
+// Cells k0 .. k0 + n - 1 of a swept solve in host order, into device-visible memory: f [n][nf][nv] (delta:
+// stored departures become f), w [n][3], prim [n][3], all FP64
+hipError_t launch_down1d(bool fp64, bool delta, const Solve1D& S, int buf, int k0, int n, double* out, hipStream_t st);
 hipError_t launch_recon1d(bool fp64, const Solve1D& S, const Solve1D* d_S, hipStream_t st);
 hipError_t launch_evolve1d(bool fp64, const Solve1D& S, const Solve1D* d_S, hipStream_t st);
 hipError_t launch_wall1d(bool fp64, const Solve1D& S, const Solve1D* d_S, int fused, int par, hipStream_t st);

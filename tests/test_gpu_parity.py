@@ -688,3 +688,35 @@ def test_sweep_width_and_steps_per_launch_do_not_change_a_result(gpu_ctx, space,
     finally:
         gpu_ctx.set_sweep_vw(0)
         gpu_ctx.set_sweep_steps(2)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("space,nx,nu", [("1d1f1v", 29, 7), ("1d1f1v", 30, 64), ("1d2f1v", 31, 65), ("1d1f1v", 700, 128),
+                                         ("1d2f1v", 1201, 130), ("1d1f1v", 40000, 63)])
+def test_swept_state_downloads_in_host_order(gpu_ctx, precision, space, nx, nu):
+    """k_down1d: tiles of 32 cells (31, 32 and 33 storage cells and many) x 64 velocities, one block and
+    several (the last sizes hold 3 and 20 MB), from two threads at a time.  FP64 returns what was uploaded,
+    bit for bit; FP32 stores f - M~(prim) rounded, so f comes back within 2^-24 (|f| + M~)."""
+    from concurrent.futures import ThreadPoolExecutor
+
+    mk = kb.configs.sod_1d1f1v if space == "1d1f1v" else kb.configs.shock_1d2f1v
+    ks = kb.SolverSet(mk(nx=nx, nu=nu))
+    ctr, face = kb.init_fvm(ks)
+    rng = np.random.default_rng(nx)
+    f = ctr.f * (0.5 + rng.random(ctr.f.shape))
+    eq = 2.0 * float(np.max(ctr.f))  # above every cell's Maxwellian (ctr.f holds them)
+    ctr.f[...] = f
+    devs = [kb.DeviceSolve(ks, ctr, face, precision, gpu_ctx) for _ in range(2)]
+    out = [copy.deepcopy(ctr) for _ in devs]
+    for c in out:
+        c.f[...] = c.w[...] = c.prim[...] = 0.0
+    with ThreadPoolExecutor(2) as pool:
+        list(pool.map(lambda dc: dc[0].download(dc[1]), zip(devs, out)))
+    for d, c in zip(devs, out):
+        d.close()
+        np.testing.assert_array_equal(c.w, ctr.w)
+        np.testing.assert_array_equal(c.prim, ctr.prim)
+        if precision == "fp64":
+            np.testing.assert_array_equal(c.f, f)
+        else:
+            assert float(np.max(np.abs(c.f - f) - 2.0**-24 * np.abs(f))) <= 2.0**-24 * eq
