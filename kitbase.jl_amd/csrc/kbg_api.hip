@@ -581,6 +581,67 @@ void fill1d(kbg_solve* s) {
     }
 }
 
+// 2D solves of the tiled step (kbg_tile2d.hip): van Leer slopes, BGK, Maxwell walls on all sides, an axis-aligned
+// mesh with one normal per direction (its velocity products are formed once per lane), and enough cells x
+// velocities that four short launches cost less than k_flux2d and k_cell2d, by flux (KFVS has no interface
+// chain to save) and storage.  us per step, the other kernels / tiled, square meshes, h and b: KFVS FP32 32 x
+// 24^2 velocities (590 k) 26.8 / 29.7, 45 x 28^2 (1.6 M) 42.8 / 42.7, 64 x 24^2 (2.4 M) 53.6 / 50.3; KFVS FP64 64 x 24^2
+// 70.6 / 74.5, 64 x 32^2 (4.2 M) 114 / 77; KCU / UGKS FP32 12 x 16^2 (37 k) 24.4 / 23.7 and 25.3 / 25.9, 24 x 16^2 (147 k)
+// 27.4 / 24.7 and 28.7 / 26.9; FP64 32 x 24^2 40.0 / 42.6 and 44.1 / 48.1, 45 x 28^2 66.7 / 65.0 and 74.9 / 72.8.
+// The choice is the solve's own: it sums the face moments in another order, and a solve's result must not
+// depend on its batch.
+bool tiled2d(const kbg_desc& d) {
+    const bool fp64 = d.precision == KBG_FP64;
+    const size_t FX = size_t(d.nx + 1) * d.ny, FY = size_t(d.nx) * (d.ny + 1), work = size_t(d.nx) * d.ny * d.nv;
+    if (work < (d.flux == KBG_KFVS ? (fp64 ? 3000000u : 2000000u) : (fp64 ? 1500000u : 100000u))) return false;
+    if (kbg::step2d_threads(fp64, d.nv) == 0 || std::max(FX, FY) * 2 * d.nv * (fp64 ? 8 : 4) >= (size_t(1) << 31)) return false;  // thr2 == 0
+    if (d.nx < kbg::kTile2dX || d.interp_order != 2 || d.limiter != KBG_VANLEER || d.collision != KBG_BGK) return false;
+    for (int b = 0; b < 4; b++)
+        if (d.bc[b] != KBG_BC_MAXWELL) return false;
+    if (!d.xgeo || !d.ygeo || !(d.xgeo[0] > 0.0 && d.ygeo[1] > 0.0)) return false;
+    for (size_t f = 0; f < FX; f++)
+        if (d.xgeo[f * 3] != d.xgeo[0] || d.xgeo[f * 3 + 1] != 0.0) return false;
+    for (size_t f = 0; f < FY; f++)
+        if (d.ygeo[f * 3] != 0.0 || d.ygeo[f * 3 + 1] != d.ygeo[1]) return false;
+    return true;
+}
+
+// buffers of the tiled step; a solve they do not fit beside (S.g stays NULL) is stepped by the other kernels
+int alloc_tiled2d(kbg_solve* s) {
+    const kbg_desc& d = s->d;
+    Solve2D& S = s->h2;
+    const size_t C = s->N, FX = size_t(d.nx + 1) * d.ny, FY = size_t(d.nx) * (d.ny + 1), nch = (size_t(d.nv) + 255) / 256;
+    void *rds, *perm, *g;
+    struct {
+        void** dst;
+        size_t bytes;
+    } tb[] = {{&S.xrec, FX * kbg::kFaceT * s->esz}, {&S.yrec, FY * kbg::kFaceT * s->esz}, {(void**)&S.xfrec, FX * 64},
+              {(void**)&S.yfrec, FY * 64},         {(void**)&S.psum, nch * (FX + FY) * 32}, {&S.crec, C * kbg::kCellT * s->esz},
+              {&rds, C * s->esz},                  {&perm, size_t(d.nv) * 4},              {&g, C * 2 * d.nv * s->esz}};
+    const size_t kept = s->allocs.size();
+    for (auto& b : tb) {
+        if (dev_alloc(s, b.dst, b.bytes) == KBG_OK) continue;
+        (void)hipGetLastError();
+        for (size_t k = kept; k < s->allocs.size(); k++) (void)hipFree(s->allocs[k]);
+        s->allocs.resize(kept);
+        return KBG_OK;
+    }
+    for (auto& b : tb) HIPCHK(hipMemset(*b.dst, 0, b.bytes));
+    int rc;
+    std::vector<double> r(C);
+    for (size_t c = 0; c < C; c++) r[c] = 1.0 / (d.dx[c] * d.dy[c]);
+    if ((rc = put_real(s, rds, r.data(), C, !s->fp64))) return rc;
+    std::vector<int> order(d.nv);
+    for (int k = 0; k < d.nv; k++) order[k] = k;
+    auto quadrant = [&](int k) { return (d.v[k] >= 0.0 ? 2 : 0) + (d.u[k] >= 0.0 ? 1 : 0); };
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return quadrant(a) < quadrant(b); });
+    HIPCHK(hipMemcpy(perm, order.data(), size_t(d.nv) * 4, hipMemcpyHostToDevice));
+    S.rds = rds;
+    S.vperm = static_cast<const int*>(perm);
+    S.g = g;
+    return KBG_OK;
+}
+
 // 1D1F3V solves stepped by k_flux3v / k_chain3v / k_relax3v (KCU and first order: the phase kernels)
 bool step3v(const Solve1D& S) { return S.vdim == 3 && S.flux == kbg::KFVS && S.interp2; }
 
@@ -780,6 +841,7 @@ int kbg_ctx_create(int device, kbg_ctx** out) {
     if (e == hipSuccess) e = hipMalloc((void**)&c->d_res, 4096 * 5 * sizeof(double));
     if (e == hipSuccess) e = kbg::sweep_narrow_attr32();
     if (e == hipSuccess) e = kbg::sweep_narrow_attr64();
+    if (e == hipSuccess) e = kbg::tile2d_attr();
     if (e != hipSuccess) {
         kbg_ctx_destroy(c);
         return fail(KBG_ERR_HIP, std::string("kbg_ctx_create: ") + hipGetErrorString(e));
@@ -917,6 +979,8 @@ size_t kbg_solve_bytes(const kbg_desc* d) {
     if (d->flux != KBG_KFVS) b += F * kbg::kFaceCoef * 8 + (esz == 4 ? F * kbg::kFaceC32 * 4 : 0);
     if (kbg::step2d_threads(d->precision == KBG_FP64, d->nv) == 0) b += C * 8 * 8 + C * 4 * nv * esz;  // slopes
     else if (esz == 4) b += 2 * nv * 4 + F * 8;  // departure form: reference Maxwellian, per-face coefficients
+    if (tiled2d(*d))  // G, face records, moment sums
+        b += C * (2 * nv + 1 + kbg::kCellT) * esz + F * (kbg::kFaceT * esz + 64 + (nv + 255) / 256 * 32) + nv * 4;
     return b;
 }
 
@@ -1173,6 +1237,7 @@ int kbg_solve_create(kbg_ctx* ctx, const kbg_desc* desc, kbg_solve** out) {
             HIPCHK(hipMemset(p, 0, FY * 8));
             S.ycref = (double*)p;
         }
+        if (tiled2d(d) && (rc = alloc_tiled2d(s))) return bail(rc);
         if ((rc = dev_alloc(s, &p, 8 * 8))) return bail(rc);
         s->res = (double*)p;
         if ((rc = dev_alloc(s, &p, 8))) return bail(rc);
@@ -1795,23 +1860,54 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
             others.push_back(i);
         }
     }
-    // fused 2D solves: face-chain, face-flux and cell launches per (precision, flux, workgroup size)
-    // group and step, all on the context stream
+    // fused 2D solves: three launches per (precision, flux, workgroup size, tiled or not) group and step
     struct Launch2 {
         bool fp64;
         int flux, threads, n, ncells, nfaces, ninterior;
         size_t desc0, cpref0, fpref0, ipref0;
         double work;
+        int ty;  // rows per tile of the tiled step (kbg_tile2d.hip; 0: the other kernels); its four prefix arrays start at fpref0
+        int totals[4];
     };
     std::vector<Launch2> launches2;
     std::vector<Solve2D> descs2;
     std::vector<int> pref2;
     {
-        std::map<std::tuple<int, int, int>, std::vector<int>> groups;
-        for (int i : fused2) groups[{solves[i]->fp64 ? 1 : 0, solves[i]->d.flux, solves[i]->thr2}].push_back(i);
+        std::map<std::tuple<int, int, int, int>, std::vector<int>> groups;
+        for (int i : fused2)
+            groups[{solves[i]->fp64 ? 1 : 0, solves[i]->d.flux, solves[i]->h2.g ? 0 : solves[i]->thr2, solves[i]->h2.g ? 1 : 0}].push_back(i);
         for (auto& kv : groups) {
             Launch2 L{std::get<0>(kv.first) == 1, std::get<1>(kv.first), std::get<2>(kv.first), (int)kv.second.size(), 0, 0, 0,
-                      descs2.size(), 0, 0, 0, 0.0};
+                      descs2.size(), 0, 0, 0, 0.0, 0, {0, 0, 0, 0}};
+            if (std::get<3>(kv.first)) {
+                long one_row = 0;
+                for (int i : kv.second)
+                    one_row += long((solves[i]->d.nx + kbg::kTile2dX - 1) / kbg::kTile2dX) * solves[i]->d.ny * ((solves[i]->d.nv + 255) / 256);
+                L.ty = kbg::tile2d_rows(L.fp64, one_row);
+                std::vector<int> p[4] = {{0}, {0}, {0}, {0}};
+                for (int i : kv.second) {
+                    kbg_solve* s = solves[i];
+                    s->h2.dt = dts[i];
+                    s->h2.ty = L.ty;
+                    descs2.push_back(s->h2);
+                    const long nx = s->d.nx, ny = s->d.ny;
+                    const long k[4] = {kbg::pre2d_wgs(s->d.nx, s->d.ny),
+                                       (nx + kbg::kTile2dX - 1) / kbg::kTile2dX * ((ny + L.ty - 1) / L.ty) * ((s->d.nv + 255) / 256), nx * ny,
+                                       kbg::relax2d_wgs(s->d.nx, s->d.ny, s->d.nv)};
+                    for (int m = 0; m < 4; m++) {
+                        if (p[m].back() + k[m] > INT_MAX / 2) return fail(KBG_ERR_ARG, "2D batch too large for one launch");
+                        p[m].push_back(int(p[m].back() + k[m]));
+                    }
+                    L.work += double(nx) * ny * s->d.nv * 2;
+                }
+                L.fpref0 = pref2.size();
+                for (int m = 0; m < 4; m++) {
+                    L.totals[m] = p[m].back();
+                    pref2.insert(pref2.end(), p[m].begin(), p[m].end());
+                }
+                launches2.push_back(L);
+                continue;
+            }
             std::vector<int> cp{0}, fp{0}, ip{0};
             for (int i : kv.second) {
                 kbg_solve* s = solves[i];
@@ -2109,7 +2205,7 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
     // ubase: the parity of the round's first step among the call's steps (unstructured solves flip
     // their f buffer every step)
     bool capturing = false;
-    auto enqueue_round = [&](int nst, bool last_round, int ubase) -> int {
+    auto enqueue_round = [&](int nst, bool last_round, int ubase, bool first_round) -> int {
         int e;
         for (Launch& L : launches) {
             for (int ks = 0, per; ks < nst; ks += per) {
@@ -2133,11 +2229,17 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
             }
         }
         for (int ks = 0; ks < nst; ks++) {
-        const bool last = last_round && ks == nst - 1;
+        const bool last = last_round && ks == nst - 1, first = first_round && ks == 0;
         for (size_t g = 0; g < launches2.size(); g++) {
             const Launch2& L = launches2[g];
             const Solve2D* dd = d_descs2 + L.desc0;
             hipStream_t ss = sst[stream2[g]];
+            if (L.ty) {
+                const int w = last || capturing ? 1 : 0;
+                HIPCHK(kbg::launch_tile2d(L.fp64, L.flux, L.ty, dd, d_pref2 + L.fpref0, L.n, L.totals, (last && residuals) ? 1 : 0,
+                                          first || capturing ? 1 : 0, w, w, ss));
+                continue;
+            }
             HIPCHK(kbg::launch_face2d(true, L.flux, dd, d_pref2 + L.ipref0, L.n, L.ninterior, ss));
             HIPCHK(kbg::launch_flux2d(L.fp64, L.flux, L.threads, dd, d_pref2 + L.fpref0, L.n, L.nfaces, ss));
             HIPCHK(kbg::launch_cell2d(L.fp64, L.threads, dd, d_pref2 + L.cpref0, L.n, L.ncells, (last && residuals) ? 1 : 0, ss));
@@ -2207,7 +2309,8 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
             const Launch2& L = launches2[g];
             for (long long v : {(long long)L.fp64, (long long)L.flux, (long long)L.threads, (long long)L.n, (long long)L.ncells,
                                 (long long)L.nfaces, (long long)L.ninterior, (long long)L.desc0, (long long)L.cpref0,
-                                (long long)L.fpref0, (long long)L.ipref0, (long long)stream2[g]})
+                                (long long)L.fpref0, (long long)L.ipref0, (long long)stream2[g], (long long)L.ty,
+                                (long long)L.totals[0], (long long)L.totals[1], (long long)L.totals[2], (long long)L.totals[3]})
                 puti(v);
         }
         for (int i : others) {
@@ -2235,8 +2338,8 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
                 HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeRelaxed));
                 for (Launch& L : launches) L.flips = L.per == 2 ? which >> 1 : 0;
                 int e = fork();
-                if (!e) e = enqueue_round((which & 1) || !two ? 1 : 2, false, 0);
-                if (!e && !(which & 1) && !two) e = enqueue_round(1, false, 1);
+                if (!e) e = enqueue_round((which & 1) || !two ? 1 : 2, false, 0, true);
+                if (!e && !(which & 1) && !two) e = enqueue_round(1, false, 1, false);
                 if (!e) e = join();
                 hipGraph_t g = nullptr;
                 const hipError_t ce = hipStreamEndCapture(st, &g);
@@ -2263,7 +2366,7 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
         if ((rc = fork())) return rc;
         for (int t = 0; t < nsteps;) {
             const int nst = std::min(round, nsteps - t);
-            if ((rc = enqueue_round(nst, t + nst == nsteps, t & 1))) return rc;
+            if ((rc = enqueue_round(nst, t + nst == nsteps, t & 1, t == 0))) return rc;
             t += nst;
         }
         if ((rc = join())) return rc;

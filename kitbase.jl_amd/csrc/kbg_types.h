@@ -89,6 +89,17 @@ struct Solve2D {
     double mmom[11];                               // sum w u^a v^b Mr_h: (a,b) = 10 01 20 11 02 30 21 12 03; Mr_b: 10 01
     double* xcref;                                 // [(nx+1)*ny] c of each x-face
     double* ycref;                                 // [nx*(ny+1)]
+    // the tiled step (kbg_tile2d.hip; NULL where the solve does not take it)
+    int ty;                                        // rows per tile
+    const void* rds;                               // [nx*ny] 1 / (dx dy), storage type
+    void* g;                                       // [nx*ny][2][nv] f + sum of face fluxes / ds
+    void* xrec;                                    // [(nx+1)*ny][kFaceT] interior faces' flux coefficients
+    void* yrec;                                    // [nx*(ny+1)][kFaceT]
+    double* xfrec;                                 // [(nx+1)*ny][8] fw0 len, Mr's coefficient, n1, n2
+    double* yfrec;                                 // [nx*(ny+1)][8]
+    double* psum;                                  // [chunks of 256 velocities][faces][4] moment sums
+    void* crec;                                    // [nx*ny][kCellT] relaxation coefficients, storage type
+    const int* vperm;                              // [nv] velocities sorted by the signs of v and u
 };
 
 // An unstructured triangle solve (2D1F2V / 2D2F2V, KFVS): faces with their two cells, normal (from
@@ -129,6 +140,10 @@ constexpr int kFaceCoef = 32;
 // aL[4], aR[4], aT[4], the six aX[3] products of the UGKS flux, the reciprocal centre spacings of
 // the two cells (rL, rR each) and their half widths
 constexpr int kFaceC32 = 40;
+// values per face record of the tiled step, and its tiles' columns
+constexpr int kFaceT = 24;
+constexpr int kCellT = 16;
+constexpr int kTile2dX = 4, kTile2dRows = 6;
 // Threads per workgroup of the fused 2D step (one face or cell per workgroup): 64 ceil(nv / 256), 4
 // velocities per thread, at most 1024 in FP32 and 512 in FP64 (the register budget of an FP64
 // thread); 0 when the velocity grid is larger (the phase kernels then step the solve)
@@ -276,5 +291,16 @@ hipError_t launch_flux2d(bool fp64, int flux, int threads, const Solve2D* d_solv
                          hipStream_t st);
 hipError_t launch_cell2d(bool fp64, int threads, const Solve2D* d_solves, const int* d_wg0, int nsolves, int ncells, int rows,
                          hipStream_t st);
+// The tiled 2D step of n solves of one precision and flux, ty rows per tile (at most kTile2dRows).  d_pref:
+// four prefix arrays of n + 1 (workgroups of k_pre2d, pre2d_wgs; of k_tile2d, ceil(nx / kTile2dX) ceil(ny / ty)
+// ceil(nv / 256); cells; workgroups of k_relax2d, relax2d_wgs), totals their last entries.  first: the walls'
+// fluxes and the interface records of this step are not there yet; last: leave the next step's out; keep:
+// also leave the face fluxes, moments and coefficients of Mr where the other kernels do
+hipError_t launch_tile2d(bool fp64, int flux, int ty, const Solve2D* d_solves, const int* d_pref, int n, const int* totals, int rows, int first,
+                         int last, int keep, hipStream_t st);
+int tile2d_rows(bool fp64, long one_row);  // rows per tile for a group of `one_row` workgroups of one row
+int pre2d_wgs(int nx, int ny);
+int relax2d_wgs(int nx, int ny, int nv);
+hipError_t tile2d_attr();
 
 }  // namespace kbg
