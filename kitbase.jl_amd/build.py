@@ -35,7 +35,7 @@ HIP_FLAGS = [
 # hipFFT for the fast spectral collision's batched 3D transforms (ROCm's own library, found through
 # the image's /opt/rocm)
 LINK = ["-L/opt/rocm/lib", "-lhipfft", "-Wl,-rpath,/opt/rocm/lib"]
-SOURCES = ["kbg_sweep_f32.hip", "kbg_sweep_f32b.hip", "kbg_sweep_f32c.hip", "kbg_sweep_f64.hip", "kbg_sweep_f64c.hip", "kbg_sweep_n32.hip", "kbg_sweep_n64.hip", "kbg_1d.hip", "kbg_2d.hip", "kbg_step2d.hip", "kbg_tile2d.hip", "kbg_us.hip", "kbg_fsm.hip", "kbg_api.hip"]
+SOURCES = ["kbg_sweep_f32.hip", "kbg_sweep_f32b.hip", "kbg_sweep_f32c.hip", "kbg_sweep_f64.hip", "kbg_sweep_f64c.hip", "kbg_sweep_n32.hip", "kbg_sweep_n64.hip", "kbg_split1d.hip", "kbg_1d.hip", "kbg_2d.hip", "kbg_step2d.hip", "kbg_tile2d.hip", "kbg_us.hip", "kbg_fsm.hip", "kbg_api.hip"]
 
 
 def _run(cmds: list[list[str]]) -> None:

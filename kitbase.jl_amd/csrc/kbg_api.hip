@@ -581,6 +581,23 @@ void fill1d(kbg_solve* s) {
     }
 }
 
+// wavefronts of a k_split1d launch over a solve's cells and 8-velocity chunks
+long split1d_waves(const Solve1D& S) {
+    return long(S.upd_hi - S.upd_lo + kbg::kSplitOut) / kbg::kSplitOut * ((S.nv + kbg::kVChunk - 1) / kbg::kVChunk);
+}
+// most wavefronts of a k_split1d launch: one per SIMD.  Every wavefront of a segment runs its cells' and faces'
+// chains, so the split pays only where the CUs are idle otherwise.  us per step, k_sweep1d / split, 2 distributions:
+// UGKS 30 cells x 16 velocities (2 wavefronts) 22.5 / 14.2, 400 x 101 (91) 35.7 / 19.0, 4000 x 64 (544) 29.5 / 19.0,
+// 4000 x 101 (884) 38.1 / 22.2; KCU 400 x 101 23.3 / 16.5, 4000 x 64 18.3 / 16.7, 4000 x 101 24.1 / 19.3.
+constexpr long kSplitWaves = 1024;
+
+// solves that may take k_split1d: FP64 KCU / UGKS with no face from the boundary-face buffers
+bool split_1d(const kbg_solve* s) {
+    const Solve1D& S = s->h1;
+    return s->fp64 && S.swept && S.flux != kbg::KFVS && !S.wallL && !S.wallR && !(S.faceL_buf && S.upd_lo == 1) &&
+           !(S.faceR_buf && S.upd_hi == S.nx) && S.upd_lo <= S.upd_hi && split1d_waves(S) <= kSplitWaves;
+}
+
 // 2D solves of the tiled step (kbg_tile2d.hip): van Leer slopes, BGK, Maxwell walls on all sides, an axis-aligned
 // mesh with one normal per direction (its velocity products are formed once per lane), and enough cells x
 // velocities that four short launches cost less than k_flux2d and k_cell2d, by flux (KFVS has no interface
@@ -969,8 +986,17 @@ size_t kbg_solve_bytes(const kbg_desc* d) {
             S.nv = d->nv;
             w3 = kbg::step3v_doubles(S) * 8;
         }
+        size_t psum = 0;  // k_split1d's moment sums
+        if (swept && esz == 8) {
+            kbg_solve t;
+            t.d = *d;
+            t.fp64 = true;
+            t.nw = nw;
+            fill1d(&t);
+            if (split_1d(&t)) psum = kbg::split1d_psum(d->nf, d->flux, d->nv, t.h1.np) * 8;
+        }
         return 2 * np * d->nf * d->nv * esz + 3 * N * nw * 8 + N * 8 + 4 * size_t(d->nv) * esz + 2 * d->nf * d->nv * esz +
-               N * 4 * nw * 8 + vt + fsm + w3;
+               N * 4 * nw * 8 + vt + fsm + w3 + psum;
     }
     const size_t C = size_t(d->nx) * d->ny, F = size_t(d->nx + 1) * d->ny + size_t(d->nx) * (d->ny + 1);
     const size_t nv = d->nv;
@@ -1058,6 +1084,10 @@ int kbg_solve_create(kbg_ctx* ctx, const kbg_desc* desc, kbg_solve** out) {
         if ((rc = dev_alloc(s, &p, N * s->nw * 8))) return bail(rc);
         S.prim = (double*)p;
         HIPCHK(hipMemset(S.prim, 0, N * s->nw * 8));
+        if (split_1d(s)) {
+            if ((rc = dev_alloc(s, &p, kbg::split1d_psum(d.nf, d.flux, d.nv, S.np) * 8))) return bail(rc);
+            S.psum = (double*)p;
+        }
         if ((rc = dev_alloc(s, &p, 2 * s->nw * 8))) return bail(rc);
         S.bfw = (double*)p;
         HIPCHK(hipMemset(S.bfw, 0, 2 * s->nw * 8));
@@ -1973,7 +2003,16 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
         round = std::max(round, steps_of[i]);
     }
     const bool two = round >= 2;  // some launch takes two steps per round
-    auto seg_of = [&](int i) { return std::min(std::max(1, ctx->seg_cells), kbg::sweep_out(steps_of[i])); };
+    // small FP64 KCU / UGKS solves split over workgroups.  Bit-identical to the sweep (kbg_split1d.hip), so the
+    // rule may look at the whole batch; not under graph replay, whose rounds end with f in memory, nor for
+    // residuals, whose sums follow the sweep's segments.
+    std::vector<char> split(n, 0);
+    {
+        long waves = 0;
+        for (int i : fused) waves += solves[i]->h1.psum ? split1d_waves(solves[i]->h1) : kSplitWaves + 1;
+        for (int i : fused) split[i] = waves <= kSplitWaves && !use_graph && !residuals && ctx->sweep_vw == 0;
+    }
+    auto seg_of = [&](int i) { return std::min(std::max(1, ctx->seg_cells), split[i] ? kbg::kSplitOut : kbg::sweep_out(steps_of[i])); };
     // Independent units -- fused 1D solves, fused 2D groups and solves stepped by the phase kernels
     // -- are spread over the streams by work (cells x velocities x distributions), heaviest first;
     // each stream advances its own share.
@@ -2026,7 +2065,8 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
         std::vector<int> members;  // solve indices (for the wall kernels)
         int per;                   // most time steps per launch
         int narrow;                // the narrow sweep: its items' most wavefronts (0: k_sweep1d)
-        int rows;                  // narrow: most velocity chunks of its solves
+        int rows;                  // narrow, split: most velocity chunks of its solves
+        bool split;                // k_split1d
         size_t item0, nitems;
         int flips;                 // sweep launches enqueued so far (the f / w buffer parity)
     };
@@ -2041,7 +2081,7 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
     std::vector<int> launch_of(n, -1);
     for (auto& kv : keyed) {
         Launch L{std::get<1>(kv.first) == 1, std::get<2>(kv.first), std::get<3>(kv.first), 1, std::get<0>(kv.first),
-                 packs.size(), 0, kv.second, std::get<4>(kv.first), 0, 0, items.size(), 0, 0};
+                 packs.size(), 0, kv.second, std::get<4>(kv.first), 0, 0, split[kv.second[0]] != 0, items.size(), 0, 0};
         for (int i : kv.second) launch_of[i] = (int)launches.size();
         std::map<int, std::vector<int>> by_nw;  // nw -> item indices, in solve order
         for (int i : kv.second) {
@@ -2054,8 +2094,8 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
             // per wavefront (a function of the solve and the context only, so a solve's sums keep
             // their order in any batch)
             int nw = narrow_nw[i] ? narrow_nw[i] : s->sweep_nw;
-            if (narrow_nw[i]) {
-                L.narrow = std::max(L.narrow, nw);
+            if (narrow_nw[i] || split[i]) {
+                if (!split[i]) L.narrow = std::max(L.narrow, nw);
                 L.rows = std::max(L.rows, (s->d.nv + kbg::kVChunk - 1) / kbg::kVChunk);
             } else if (ctx->sweep_vw > 0)
                 while (nw < kbg::kSweepMaxWaves && (s->d.nv + nw - 1) / nw > ctx->sweep_vw) nw *= 2;
@@ -2063,7 +2103,7 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
             for (size_t it = i0; it < items.size(); it++) by_nw[nw].push_back((int)it);
             L.wg_waves = std::max(L.wg_waves, nw);
         }
-        if (L.narrow) {  // one item per workgroup, no packs
+        if (L.narrow || L.split) {  // no packs
             L.nitems = items.size() - L.item0;
             launches.push_back(std::move(L));
             continue;
@@ -2217,7 +2257,9 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
                         HIPCHK(kbg::launch_wall1d(solves[di]->fp64, S, d_descs + desc_of[di], 1, par, sst[L.stream]));
                 }
                 const bool keep = last_round && residuals && ks + per == nst;
-                if (L.narrow) {
+                if (L.split) {
+                    HIPCHK(kbg::launch_split1d(L.nf, L.flux, d_descs, d_items + L.item0, (int)L.nitems, L.rows, L.flips, 0, sst[L.stream]));
+                } else if (L.narrow) {
                     double* rp = keep ? d_rpart + L.item0 * 12 : nullptr;
                     HIPCHK((L.fp64 ? kbg::launch_sweep1d_narrow64 : kbg::launch_sweep1d_narrow32)(
                         L.nf, L.narrow, L.rows, d_descs, d_items + L.item0, (int)L.nitems, par, rp, per, sst[L.stream]));
@@ -2369,6 +2411,9 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
             if ((rc = enqueue_round(nst, t + nst == nsteps, t & 1, t == 0))) return rc;
             t += nst;
         }
+        for (const Launch& L : launches)
+            if (L.split)
+                HIPCHK(kbg::launch_split1d(L.nf, L.flux, d_descs, d_items + L.item0, (int)L.nitems, L.rows, L.flips, 1, sst[L.stream]));
         if ((rc = join())) return rc;
     }
     HIPCHK(hipEventRecord(ctx->ev[KBG_EV_STEPS_END], st));

@@ -50,6 +50,7 @@ struct Solve1D {
     int* health;                                   // failure flags (kbg_device.h prim_health)
     const double* fsmq;                            // collision :fsm: Q of the cells fsm_c0 .. [ncell][nv]
     int fsm_c0;                                    // first physical cell of fsmq
+    double* psum;                                  // k_split1d: moment sums of two steps (kbg_split1d.hip; or NULL)
 };
 
 struct Solve2D {
@@ -195,6 +196,12 @@ hipError_t launch_sweep1d_narrow64(int nf, int wg_waves, int rows, const Solve1D
                                    int par, double* d_rpart, int nstep, hipStream_t st);
 hipError_t sweep_narrow_attr32();
 hipError_t sweep_narrow_attr64();
+// The FP64 KCU / UGKS step of small launches (kbg_split1d.hip), one step per launch; items of at most kSplitOut
+// cells, chunks: the most 8-velocity chunks of their solves; par counts the call's launches; end: after the
+// last step, par = its number of launches
+constexpr int kSplitOut = 59;
+hipError_t launch_split1d(int nf, int flux, const Solve1D* d_solves, const WorkItem* d_items, int nitems, int chunks, int par, int end, hipStream_t st);
+size_t split1d_psum(int nf, int flux, int nv, long np);  // doubles of Solve1D::psum
 // velocities per wavefront of an item (a multiple of 8, at most sweep_vw)
 constexpr int sweep_item_vw(int nv, int nw) { return ((nv + nw - 1) / nw + 7) / 8 * 8; }
 // Conversions of an FP32 swept solve's f buffer `buf` between its stored departure f - M~(prim) and f:

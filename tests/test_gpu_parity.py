@@ -720,3 +720,39 @@ def test_swept_state_downloads_in_host_order(gpu_ctx, precision, space, nx, nu):
             np.testing.assert_array_equal(c.f, f)
         else:
             assert float(np.max(np.abs(c.f - f) - 2.0**-24 * np.abs(f))) <= 2.0**-24 * eq
+
+
+@pytest.mark.parametrize("space,flux,collision", [("1d2f1v", "ugks", "bgk"), ("1d2f1v", "ugks", "shakhov"), ("1d2f1v", "kcu", "shakhov"),
+                                                  ("1d1f1v", "kcu", "bgk")])
+@pytest.mark.parametrize("nv", [7, 8, 9, 64, 101, 128])
+def test_split_sweep_equals_the_sweep(gpu_ctx, space, flux, collision, nv):
+    """k_split1d (small FP64 KCU / UGKS launches) against the full-width sweep (a cap of 64 velocities), bit for
+    bit, and against the oracle: velocities around its 8-velocity chunks and the sweep's wavefronts, meshes
+    around its 59-cell segments, first order and the generic limiters, ghost cells, one step and several."""
+    mk = kb.configs.shock_1d2f1v if space == "1d2f1v" else kb.configs.sod_1d1f1v
+    rng = np.random.default_rng(nv)
+    try:
+        for nx, over in ((6, {}), (60, dict(interpOrder=1)), (61, {}), (62, dict(limiter="minmod")), (120, dict(nxg=1)), (121, {})):
+            ks = kb.SolverSet(mk(nx=nx, nu=nv, flux=flux, collision=collision, vMeshType="rectangle", **over))
+            ctr, face = kb.init_fvm(ks)
+            ctr.f *= 1.0 + 0.01 * rng.random(ctr.f.shape)
+            dt = kb.timestep(ks, ctr)
+            got = []
+            for vw in (0, 64):
+                gpu_ctx.set_sweep_vw(vw)
+                c = copy.deepcopy(ctr)
+                dev = kb.DeviceSolve(ks, c, face, "fp64", gpu_ctx)
+                dev.step(dt, 1)
+                dev.step(dt, 6)
+                dev.download(c)
+                assert dev.health() == 0
+                dev.close()
+                got.append(c)
+            np.testing.assert_array_equal(got[0].f, got[1].f)
+            np.testing.assert_array_equal(got[0].w, got[1].w)
+            np.testing.assert_array_equal(got[0].prim, got[1].prim)
+            co, fo = copy.deepcopy(ctr), copy.deepcopy(face)
+            oracle.OracleSolve(ks, co, fo).run(dt, 7)
+            assert rel_max(got[0].f, co.f) <= 1e-10 and rel_max(got[0].w, co.w) <= 1e-10
+    finally:
+        gpu_ctx.set_sweep_vw(0)
