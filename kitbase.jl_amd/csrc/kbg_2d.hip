@@ -47,171 +47,29 @@ template <class T> __global__ __launch_bounds__(256) void k_recon2d(const Solve2
     }
 }
 
-// evolve!  solver_evolution.jl:608-679: interior x-faces (i = 2..nx) then y-faces (j = 2..ny).
-// Wrappers flux_kfvs.jl:98-135 and flux_kcu.jl:149-191; UGKS uses the KCU wrapper's framing with
-// flux_ugks.jl:121-253.  The KCU / UGKS face chain (FP64) comes from the records of k_face2d.
-template <class T, int FLUX> __global__ __launch_bounds__(256) void k_evolve2d(const Solve2D* __restrict__ pS) {
-    __shared__ double red_s[4 * 10];
-    const Solve2D& S = *pS;
-    const int nx = S.nx, ny = S.ny, nv = S.nv, RS = 2 * nv;
-    const int nxf = (nx - 1) * ny;
-    int b = blockIdx.x, dir, fi, cL, cR;
-    if (b < nxf) {
-        dir = 0;
-        const int i = b % (nx - 1) + 2, j = b / (nx - 1) + 1;
-        fi = (i - 1) + (nx + 1) * (j - 1);
-        cL = (i - 2) + nx * (j - 1);
-        cR = cL + 1;
-    } else {
-        b -= nxf;
-        dir = 1;
-        const int i = b % nx + 1, j = b / nx + 2;
-        fi = (i - 1) + nx * (j - 1);
-        cL = (i - 1) + nx * (j - 2);
-        cR = cL + nx;
+// workgroup totals of N <= 8 values, in all threads: a reduce-scatter per wavefront, then the wavefronts in order
+template <int N> KBG_D void block_sum(double* v, double* scratch) {
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    double r8[8];
+#pragma unroll
+    for (int m = 0; m < 8; m++) r8[m] = m < N ? v[m] : 0.0;
+    const double t = wave_reduce_scatter<8>(r8);
+    if ((lane & 7) == 0) scratch[wv * 8 + (lane >> 3)] = t;
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < N; m++) {
+        double q = scratch[m];
+        for (int w = 1; w < nw; w++) q += scratch[w * 8 + m];
+        v[m] = q;
     }
-    const double* geo = (dir == 0 ? S.xgeo : S.ygeo) + (size_t)fi * 3;
-    const double n1 = geo[0], n2 = geo[1], len = geo[2];
-    const double* d = dir == 0 ? S.dx : S.dy;
-    const double dxL = 0.5 * d[cL], dxR = 0.5 * d[cR];
-    const T dxLT = T(dxL), dxRT = T(dxR);
-    double* fwout = (dir == 0 ? S.xfw : S.yfw) + (size_t)fi * 4;
-    T* ffh = (T*)(dir == 0 ? S.xff : S.yff) + (size_t)fi * RS;
-    T* ffb = ffh + nv;
-    const T* f = (const T*)S.f;
-    const T* sf = (const T*)S.sf;
-    const T* hL = f + (size_t)cL * RS;
-    const T* bL = hL + nv;
-    const T* hR = f + (size_t)cR * RS;
-    const T* bR = hR + nv;
-    const T* shL = sf + (size_t)cL * 2 * RS + (size_t)dir * RS;
-    const T* sbL = shL + nv;
-    const T* shR = sf + (size_t)cR * 2 * RS + (size_t)dir * RS;
-    const T* sbR = shR + nv;
-    const T* U = (const T*)S.u;
-    const T* V = (const T*)S.v;
-    const T* WT = (const T*)S.wt;
-    const T n1T = T(n1), n2T = T(n2), lenT = T(len);
-    const double dt = S.dt, K = S.K;
-    const T dtT = T(dt), hdt2 = T(0.5 * dt * dt);
-    double fw[4];
-    if (FLUX == KFVS) {
-        KSum<T> a[5];
-        for (int iv = threadIdx.x; iv < nv; iv += blockDim.x) {
-            const T x = U[iv] * n1T + V[iv] * n2T, y = V[iv] * n1T - U[iv] * n2T, wq = WT[iv];
-            const bool dd = x >= T(0);
-            const T h = dd ? hL[iv] + shL[iv] * dxLT : hR[iv] - shR[iv] * dxRT;
-            const T bb = dd ? bL[iv] + sbL[iv] * dxLT : bR[iv] - sbR[iv] * dxRT;
-            const T sh = dd ? shL[iv] : shR[iv];
-            const T sb = dd ? sbL[iv] : sbR[iv];
-            const T fh = (dtT * x * h - hdt2 * (x * x) * sh) * lenT;
-            const T fb = (dtT * x * bb - hdt2 * (x * x) * sb) * lenT;
-            ffh[iv] = fh;
-            ffb[iv] = fb;
-            a[0].add(wq * fh);
-            a[1].add(x * wq * fh);
-            a[2].add(y * wq * fh);
-            a[3].add((x * x + y * y) * wq * fh);
-            a[4].add(wq * fb);
-        }
-        double r[5] = {a[0].val(), a[1].val(), a[2].val(), a[3].val(), a[4].val()};
-        block_allreduce256<5>(r, red_s);
-        fw[0] = r[0];
-        fw[1] = r[1];
-        fw[2] = r[2];
-        fw[3] = 0.5 * (r[3] + r[4]);
-    } else {
-        // the face chain was evaluated once per face by k_face2d
-        const double* rec = (dir == 0 ? S.xcoef : S.ycoef) + (size_t)fi * kFaceCoef;
-        if (FLUX == KCU) {
-            const KcuFace<4>& F = *(const KcuFace<4>*)rec;
-            const T A = T(F.prim[0] * (F.prim[3] / kPi)), lam = T(F.prim[3]), Ui = T(F.prim[1]), Vi = T(F.prim[2]);
-            const T Mt1 = T(F.Mt1), Mt2 = T(F.Mt2), kb = T(K / (2.0 * F.prim[3]));
-            KSum<T> a[5];
-            for (int iv = threadIdx.x; iv < nv; iv += blockDim.x) {
-                const T x = U[iv] * n1T + V[iv] * n2T, y = V[iv] * n1T - U[iv] * n2T, wq = WT[iv];
-                const bool dd = x >= T(0);
-                const T h = dd ? hL[iv] + shL[iv] * dxLT : hR[iv] - shR[iv] * dxRT;
-                const T bb = dd ? bL[iv] + sbL[iv] * dxLT : bR[iv] - sbR[iv] * dxRT;
-                const T cu = x - Ui, cv = y - Vi;
-                const T H = A * texp(-lam * (cu * cu + cv * cv));
-                const T B = H * kb;
-                a[0].add(wq * x * h);
-                a[1].add(wq * (x * x) * h);
-                a[2].add(wq * y * x * h);
-                a[3].add(wq * x * (x * x + y * y) * h);
-                a[4].add(wq * x * bb);
-                ffh[iv] = (Mt1 * x * H + Mt2 * x * h) * lenT;
-                ffb[iv] = (Mt1 * x * B + Mt2 * x * bb) * lenT;
-            }
-            double r[5] = {a[0].val(), a[1].val(), a[2].val(), a[3].val(), a[4].val()};
-            block_allreduce256<5>(r, red_s);
-            fw[0] = F.fw0[0] * len + F.Mt2 * r[0] * len;
-            fw[1] = F.fw0[1] * len + F.Mt2 * r[1] * len;
-            fw[2] = F.fw0[2] * len + F.Mt2 * r[2] * len;
-            fw[3] = F.fw0[3] * len + F.Mt2 * 0.5 * (r[3] + r[4]) * len;
-        } else {
-            const UgksFace2& F = *(const UgksFace2*)rec;
-            const T A = T(F.prim[0] * (F.prim[3] / kPi)), lam = T(F.prim[3]), Ui = T(F.prim[1]), Vi = T(F.prim[2]);
-            const T kb = T(K / (2.0 * F.prim[3])), Mxi2 = T(F.Mxi2);
-            const T Mt0 = T(F.Mt[0]), Mt1 = T(F.Mt[1]), Mt2 = T(F.Mt[2]), Mt3 = T(F.Mt[3]), Mt4 = T(F.Mt[4]);
-            T aL[4], aR[4], aT[4];
-            for (int m = 0; m < 4; m++) {
-                aL[m] = T(F.aL[m]);
-                aR[m] = T(F.aR[m]);
-                aT[m] = T(F.aT[m]);
-            }
-            KSum<T> a[8];
-            for (int iv = threadIdx.x; iv < nv; iv += blockDim.x) {
-                const T x = U[iv] * n1T + V[iv] * n2T, y = V[iv] * n1T - U[iv] * n2T, wq = WT[iv];
-                const bool dd = x >= T(0);
-                const T uu = x * x, q2 = uu + y * y;
-                const T h = dd ? hL[iv] + shL[iv] * dxLT : hR[iv] - shR[iv] * dxRT;
-                const T bb = dd ? bL[iv] + sbL[iv] * dxLT : bR[iv] - sbR[iv] * dxRT;
-                const T sh = dd ? shL[iv] : shR[iv];
-                const T sb = dd ? sbL[iv] : sbR[iv];
-                const T cu = x - Ui, cv = y - Vi;
-                const T H = A * texp(-lam * (cu * cu + cv * cv));
-                const T B = H * kb;
-                a[0].add(wq * x * h);
-                a[1].add(wq * uu * sh);
-                a[2].add(wq * uu * h);
-                a[3].add(wq * (uu * x) * sh);
-                a[4].add(wq * y * x * h);
-                a[5].add(wq * y * uu * sh);
-                a[6].add(wq * x * q2 * h + wq * x * bb);
-                a[7].add(wq * uu * q2 * sh + wq * uu * sb);
-                const T* s = dd ? aL : aR;
-                const T pH = s[0] * H + s[1] * x * H + s[2] * y * H + T(0.5) * s[3] * (q2 * H + B);
-                const T pTH = aT[0] * H + aT[1] * x * H + aT[2] * y * H + T(0.5) * aT[3] * (q2 * H + B);
-                const T pB = s[0] * B + s[1] * x * B + s[2] * y * B + T(0.5) * s[3] * (q2 * B + Mxi2 * H);
-                const T pTB = aT[0] * B + aT[1] * x * B + aT[2] * y * B + T(0.5) * aT[3] * (q2 * B + Mxi2 * H);
-                ffh[iv] = (Mt0 * x * H + Mt1 * uu * pH + Mt2 * x * pTH + Mt3 * x * h - Mt4 * uu * sh) * lenT;
-                ffb[iv] = (Mt0 * x * B + Mt1 * uu * pB + Mt2 * x * pTB + Mt3 * x * bb - Mt4 * uu * sb) * lenT;
-            }
-            double r[8];
-            for (int m = 0; m < 8; m++) r[m] = a[m].val();
-            block_allreduce256<8>(r, red_s);
-            fw[0] = (F.fw0[0] + (F.Mt[3] * r[0] - F.Mt[4] * r[1])) * len;
-            fw[1] = (F.fw0[1] + (F.Mt[3] * r[2] - F.Mt[4] * r[3])) * len;
-            fw[2] = (F.fw0[2] + (F.Mt[3] * r[4] - F.Mt[4] * r[5])) * len;
-            fw[3] = (F.fw0[3] + (F.Mt[3] * 0.5 * r[6] - F.Mt[4] * 0.5 * r[7])) * len;
-        }
-    }
-    if (threadIdx.x == 0) {
-        double g[4];
-        global_frame4(fw, n1, n2, g);
-        for (int m = 0; m < 4; m++) fwout[m] = g[m];
-    }
+    __syncthreads();
 }
 
 // Maxwell diffuse walls: evolve_boundary.jl:52-178 -> flux_boundary.jl:190-220.
-// Blocks: [0, ny) left, [ny, 2ny) right, [2ny, 2ny+nx) bottom, [2ny+nx, 2ny+2nx) top.
-template <class T> __global__ __launch_bounds__(256) void k_wall2d(const Solve2D* __restrict__ pS) {
-    __shared__ double red_s[4 * 8];
-    const Solve2D& S = *pS;
+// Walls: [0, ny) left, [ny, 2ny) right, [2ny, 2ny+nx) bottom, [2ny+nx, 2ny+2nx) top.
+template <class T> KBG_D void wall2d(const Solve2D& S, int b, double* red_s) {
     const int nx = S.nx, ny = S.ny, nv = S.nv, RS = 2 * nv;
-    int b = blockIdx.x, side, fi, c, rot;
+    int side, fi, c, rot;
     if (b < ny) {
         side = 0; const int j = b + 1;
         fi = (nx + 1) * (j - 1); c = nx * (j - 1); rot = 1;
@@ -254,7 +112,7 @@ template <class T> __global__ __launch_bounds__(256) void k_wall2d(const Solve2D
         }
     }
     double r[2] = {a0.val(), a1.val()};
-    block_allreduce256<2>(r, red_s);
+    block_sum<2>(r, red_s);
     const double rho = -r[0] / ((bcl[3] / kPi) * r[1]);
     const T A = T(rho * (bcl[3] / kPi)), kb = T(K / (2.0 * bcl[3])), sc = T(len * dt);
     KSum<T> m[5];
@@ -274,11 +132,173 @@ template <class T> __global__ __launch_bounds__(256) void k_wall2d(const Solve2D
         ffb[iv] = x * bW * sc;
     }
     double s[5] = {m[0].val(), m[1].val(), m[2].val(), m[3].val(), m[4].val()};
-    block_allreduce256<5>(s, red_s);
+    block_sum<5>(s, red_s);
     if (threadIdx.x == 0) {
         double fw[4] = {s[0] * len * dt, s[1] * len * dt, s[2] * len * dt, (0.5 * s[3] + 0.5 * s[4]) * len * dt}, g[4];
         global_frame4(fw, n1, n2, g);
         for (int k = 0; k < 4; k++) fwout[k] = g[k];
+    }
+}
+
+// evolve!  solver_evolution.jl:608-679: the walls (their two passes are the longest of the launch), interior
+// x-faces (i = 2..nx), then y-faces (j = 2..ny).
+// Wrappers flux_kfvs.jl:98-135 and flux_kcu.jl:149-191; UGKS uses the KCU wrapper's framing with
+// flux_ugks.jl:121-253.  The KCU / UGKS face chain (FP64) comes from the records of k_face2d.  Bound by the
+// latency of its few passes per thread: UGKS FP64, 32 x 32 cells x 24^2 velocities 21.9 us with the walls; 28.8 + 7.3
+// with the walls in a launch of their own, both cells' loads per lane and every sum reduced by itself.
+template <class T, int FLUX> __global__ __launch_bounds__(256) void k_evolve2d(const Solve2D* __restrict__ pS) {
+    __shared__ double red_s[4 * 8];
+    const Solve2D& S = *pS;
+    const int nx = S.nx, ny = S.ny, nv = S.nv, RS = 2 * nv;
+    const int nxf = (nx - 1) * ny;
+    int b = int(blockIdx.x) - 2 * (nx + ny), dir, fi, cL, cR;
+    if (b < 0) {
+        wall2d<T>(S, blockIdx.x, red_s);
+        return;
+    }
+    if (b < nxf) {
+        dir = 0;
+        const int i = b % (nx - 1) + 2, j = b / (nx - 1) + 1;
+        fi = (i - 1) + (nx + 1) * (j - 1);
+        cL = (i - 2) + nx * (j - 1);
+        cR = cL + 1;
+    } else {
+        b -= nxf;
+        dir = 1;
+        const int i = b % nx + 1, j = b / nx + 2;
+        fi = (i - 1) + nx * (j - 1);
+        cL = (i - 1) + nx * (j - 2);
+        cR = cL + nx;
+    }
+    const double* geo = (dir == 0 ? S.xgeo : S.ygeo) + (size_t)fi * 3;
+    const double n1 = geo[0], n2 = geo[1], len = geo[2];
+    const double* d = dir == 0 ? S.dx : S.dy;
+    const double dxL = 0.5 * d[cL], dxR = 0.5 * d[cR];
+    const T dxLT = T(dxL), dxRT = T(dxR);
+    double* fwout = (dir == 0 ? S.xfw : S.yfw) + (size_t)fi * 4;
+    T* __restrict__ ffh = (T*)(dir == 0 ? S.xff : S.yff) + (size_t)fi * RS;
+    T* __restrict__ ffb = ffh + nv;
+    // f and slope along dir of the left cell, the right one at oR (2 oR): a lane loads its upwind cell's only.  No
+    // alias with the fluxes, so that a pass's loads need not wait for the last one's stores
+    const T* __restrict__ f = (const T*)S.f + (size_t)cL * RS;
+    const T* __restrict__ sf = (const T*)S.sf + (size_t)cL * 2 * RS + (size_t)dir * RS;
+    const long oR = (long)(cR - cL) * RS;
+    const T* __restrict__ U = (const T*)S.u;
+    const T* __restrict__ V = (const T*)S.v;
+    const T* __restrict__ WT = (const T*)S.wt;
+    const T n1T = T(n1), n2T = T(n2), lenT = T(len);
+    const double dt = S.dt, K = S.K;
+    const T dtT = T(dt), hdt2 = T(0.5 * dt * dt);
+    double fw[4];
+    if (FLUX == KFVS) {
+        KSum<T> a[5];
+        for (int iv = threadIdx.x; iv < nv; iv += blockDim.x) {
+            const T x = U[iv] * n1T + V[iv] * n2T, y = V[iv] * n1T - U[iv] * n2T, wq = WT[iv];
+            const bool dd = x >= T(0);
+            const T *fp = f + (dd ? 0 : oR) + iv, *sp = sf + (dd ? 0 : 2 * oR) + iv;
+            const T dx = dd ? dxLT : -dxRT, sh = sp[0], sb = sp[nv];
+            const T h = fp[0] + sh * dx;
+            const T bb = fp[nv] + sb * dx;
+            const T fh = (dtT * x * h - hdt2 * (x * x) * sh) * lenT;
+            const T fb = (dtT * x * bb - hdt2 * (x * x) * sb) * lenT;
+            ffh[iv] = fh;
+            ffb[iv] = fb;
+            a[0].add(wq * fh);
+            a[1].add(x * wq * fh);
+            a[2].add(y * wq * fh);
+            a[3].add((x * x + y * y) * wq * fh);
+            a[4].add(wq * fb);
+        }
+        double r[5] = {a[0].val(), a[1].val(), a[2].val(), a[3].val(), a[4].val()};
+        block_sum<5>(r, red_s);
+        fw[0] = r[0];
+        fw[1] = r[1];
+        fw[2] = r[2];
+        fw[3] = 0.5 * (r[3] + r[4]);
+    } else {
+        // the face chain was evaluated once per face by k_face2d
+        const double* rec = (dir == 0 ? S.xcoef : S.ycoef) + (size_t)fi * kFaceCoef;
+        if (FLUX == KCU) {
+            const KcuFace<4>& F = *(const KcuFace<4>*)rec;
+            const T A = T(F.prim[0] * (F.prim[3] / kPi)), lam = T(F.prim[3]), Ui = T(F.prim[1]), Vi = T(F.prim[2]);
+            const T Mt1 = T(F.Mt1), Mt2 = T(F.Mt2), kb = T(K / (2.0 * F.prim[3]));
+            KSum<T> a[5];
+            for (int iv = threadIdx.x; iv < nv; iv += blockDim.x) {
+                const T x = U[iv] * n1T + V[iv] * n2T, y = V[iv] * n1T - U[iv] * n2T, wq = WT[iv];
+                const bool dd = x >= T(0);
+                const T *fp = f + (dd ? 0 : oR) + iv, *sp = sf + (dd ? 0 : 2 * oR) + iv;
+                const T dx = dd ? dxLT : -dxRT, sh = sp[0], sb = sp[nv];
+                const T h = fp[0] + sh * dx;
+                const T bb = fp[nv] + sb * dx;
+                const T cu = x - Ui, cv = y - Vi;
+                const T H = A * texp(-lam * (cu * cu + cv * cv));
+                const T B = H * kb;
+                a[0].add(wq * x * h);
+                a[1].add(wq * (x * x) * h);
+                a[2].add(wq * y * x * h);
+                a[3].add(wq * x * (x * x + y * y) * h);
+                a[4].add(wq * x * bb);
+                ffh[iv] = (Mt1 * x * H + Mt2 * x * h) * lenT;
+                ffb[iv] = (Mt1 * x * B + Mt2 * x * bb) * lenT;
+            }
+            double r[5] = {a[0].val(), a[1].val(), a[2].val(), a[3].val(), a[4].val()};
+            block_sum<5>(r, red_s);
+            fw[0] = F.fw0[0] * len + F.Mt2 * r[0] * len;
+            fw[1] = F.fw0[1] * len + F.Mt2 * r[1] * len;
+            fw[2] = F.fw0[2] * len + F.Mt2 * r[2] * len;
+            fw[3] = F.fw0[3] * len + F.Mt2 * 0.5 * (r[3] + r[4]) * len;
+        } else {
+            const UgksFace2& F = *(const UgksFace2*)rec;
+            const T A = T(F.prim[0] * (F.prim[3] / kPi)), lam = T(F.prim[3]), Ui = T(F.prim[1]), Vi = T(F.prim[2]);
+            const T kb = T(K / (2.0 * F.prim[3])), Mxi2 = T(F.Mxi2);
+            const T Mt0 = T(F.Mt[0]), Mt1 = T(F.Mt[1]), Mt2 = T(F.Mt[2]), Mt3 = T(F.Mt[3]), Mt4 = T(F.Mt[4]);
+            T aL[4], aR[4], aT[4];
+            for (int m = 0; m < 4; m++) {
+                aL[m] = T(F.aL[m]);
+                aR[m] = T(F.aR[m]);
+                aT[m] = T(F.aT[m]);
+            }
+            KSum<T> a[8];
+            for (int iv = threadIdx.x; iv < nv; iv += blockDim.x) {
+                const T x = U[iv] * n1T + V[iv] * n2T, y = V[iv] * n1T - U[iv] * n2T, wq = WT[iv];
+                const bool dd = x >= T(0);
+                const T uu = x * x, q2 = uu + y * y;
+                const T *fp = f + (dd ? 0 : oR) + iv, *sp = sf + (dd ? 0 : 2 * oR) + iv;
+                const T dx = dd ? dxLT : -dxRT, sh = sp[0], sb = sp[nv];
+                const T h = fp[0] + sh * dx;
+                const T bb = fp[nv] + sb * dx;
+                const T cu = x - Ui, cv = y - Vi;
+                const T H = A * texp(-lam * (cu * cu + cv * cv));
+                const T B = H * kb;
+                a[0].add(wq * x * h);
+                a[1].add(wq * uu * sh);
+                a[2].add(wq * uu * h);
+                a[3].add(wq * (uu * x) * sh);
+                a[4].add(wq * y * x * h);
+                a[5].add(wq * y * uu * sh);
+                a[6].add(wq * x * q2 * h + wq * x * bb);
+                a[7].add(wq * uu * q2 * sh + wq * uu * sb);
+                const T* s = dd ? aL : aR;
+                const T pH = s[0] * H + s[1] * x * H + s[2] * y * H + T(0.5) * s[3] * (q2 * H + B);
+                const T pTH = aT[0] * H + aT[1] * x * H + aT[2] * y * H + T(0.5) * aT[3] * (q2 * H + B);
+                const T pB = s[0] * B + s[1] * x * B + s[2] * y * B + T(0.5) * s[3] * (q2 * B + Mxi2 * H);
+                const T pTB = aT[0] * B + aT[1] * x * B + aT[2] * y * B + T(0.5) * aT[3] * (q2 * B + Mxi2 * H);
+                ffh[iv] = (Mt0 * x * H + Mt1 * uu * pH + Mt2 * x * pTH + Mt3 * x * h - Mt4 * uu * sh) * lenT;
+                ffb[iv] = (Mt0 * x * B + Mt1 * uu * pB + Mt2 * x * pTB + Mt3 * x * bb - Mt4 * uu * sb) * lenT;
+            }
+            double r[8];
+            for (int m = 0; m < 8; m++) r[m] = a[m].val();
+            block_sum<8>(r, red_s);
+            fw[0] = (F.fw0[0] + (F.Mt[3] * r[0] - F.Mt[4] * r[1])) * len;
+            fw[1] = (F.fw0[1] + (F.Mt[3] * r[2] - F.Mt[4] * r[3])) * len;
+            fw[2] = (F.fw0[2] + (F.Mt[3] * r[4] - F.Mt[4] * r[5])) * len;
+            fw[3] = (F.fw0[3] + (F.Mt[3] * 0.5 * r[6] - F.Mt[4] * 0.5 * r[7])) * len;
+        }
+    }
+    if (threadIdx.x == 0) {
+        double g[4];
+        global_frame4(fw, n1, n2, g);
+        for (int m = 0; m < 4; m++) fwout[m] = g[m];
     }
 }
 
@@ -386,24 +406,29 @@ template <class T> __global__ __launch_bounds__(256) void k_update2d(const Solve
     }
 }
 
-__global__ void k_resid2(const double* __restrict__ rows, int nrows, double ncell, double* __restrict__ out) {
-    __shared__ double part[256 * 16];
-    for (int col = 0; col < 16; col++) {
-        double s = 0.0;
-        for (int r = threadIdx.x; r < nrows; r += 256) s += rows[(size_t)r * 16 + col];
-        part[threadIdx.x * 16 + col] = s;
-    }
-    __syncthreads();
-    __shared__ double tot[16];
-    if (threadIdx.x < 16) {
-        double s = 0.0;
-        for (int t = 0; t < 256; t++) s += part[t * 16 + threadIdx.x];
-        tot[threadIdx.x] = s;
-    }
+// One workgroup: thread = (row of 64) 16 + column, coalesced; the rows' sums within a wavefront, then the
+// wavefronts in order.  (Each of 256 threads over all 16 columns and 16 threads over 256 partial sums in a row
+// took 13.7 us for 1024 cells, 4.1 here.)
+__global__ __launch_bounds__(1024) void k_resid2(const double* __restrict__ rows, int nrows, double ncell, double* __restrict__ out) {
+    __shared__ double part[16 * 16];
+    const int col = threadIdx.x & 15, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    double s = 0.0;
+#pragma unroll 8
+    for (int r = threadIdx.x >> 4; r < nrows; r += 64) s += rows[(size_t)r * 16 + col];
+    s += __shfl_xor(s, 16, 64);
+    s += __shfl_xor(s, 32, 64);
+    if (lane < 16) part[wv * 16 + col] = s;
     __syncthreads();
     if (threadIdx.x < 4) {
         const int m = threadIdx.x;
-        out[m] = sqrt(tot[m] * ncell) / (tot[4 + m] + 1.e-7) + sqrt(tot[8 + m] * 2.0) / (tot[12 + m] + 1.e-7);
+        double tot[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            tot[k] = 0.0;
+#pragma unroll
+            for (int w = 0; w < 16; w++) tot[k] += part[w * 16 + 4 * k + m];
+        }
+        out[m] = sqrt(tot[0] * ncell) / (tot[1] + 1.e-7) + sqrt(tot[2] * 2.0) / (tot[3] + 1.e-7);
     }
 }
 
@@ -446,27 +471,27 @@ hipError_t launch_recon2d(bool fp64, const Solve2D& S, const Solve2D* d_S, hipSt
     return hipGetLastError();
 }
 
+// wavefronts of a face's workgroup: the fewest that take as few passes over the velocities as four do
+// (576 velocities: three wavefronts, three passes)
+static int phase_threads(int nv) {
+    const int w = (nv + 63) / 64, passes = (w + 3) / 4;
+    return 64 * ((w + passes - 1) / passes);
+}
+
 hipError_t launch_evolve2d(bool fp64, const Solve2D& S, const Solve2D* d_S, hipStream_t st) {
     const int nfaces = (S.nx - 1) * S.ny + S.nx * (S.ny - 1);
-    if (nfaces > 0) {
-        hipError_t e0 = launch_face2d(false, S.flux, d_S, nullptr, 1, nfaces, st);
-        if (e0 != hipSuccess) return e0;
-        dim3 g(nfaces), b(256);
-        if (fp64) {
-            if (S.flux == KFVS) hipLaunchKernelGGL((k_evolve2d<double, KFVS>), g, b, 0, st, d_S);
-            else if (S.flux == KCU) hipLaunchKernelGGL((k_evolve2d<double, KCU>), g, b, 0, st, d_S);
-            else hipLaunchKernelGGL((k_evolve2d<double, UGKS>), g, b, 0, st, d_S);
-        } else {
-            if (S.flux == KFVS) hipLaunchKernelGGL((k_evolve2d<float, KFVS>), g, b, 0, st, d_S);
-            else if (S.flux == KCU) hipLaunchKernelGGL((k_evolve2d<float, KCU>), g, b, 0, st, d_S);
-            else hipLaunchKernelGGL((k_evolve2d<float, UGKS>), g, b, 0, st, d_S);
-        }
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
+    const hipError_t e0 = launch_face2d(false, S.flux, d_S, nullptr, 1, nfaces, st);
+    if (e0 != hipSuccess) return e0;
+    const dim3 g(nfaces + 2 * (S.nx + S.ny)), b(phase_threads(S.nv));
+    if (fp64) {
+        if (S.flux == KFVS) hipLaunchKernelGGL((k_evolve2d<double, KFVS>), g, b, 0, st, d_S);
+        else if (S.flux == KCU) hipLaunchKernelGGL((k_evolve2d<double, KCU>), g, b, 0, st, d_S);
+        else hipLaunchKernelGGL((k_evolve2d<double, UGKS>), g, b, 0, st, d_S);
+    } else {
+        if (S.flux == KFVS) hipLaunchKernelGGL((k_evolve2d<float, KFVS>), g, b, 0, st, d_S);
+        else if (S.flux == KCU) hipLaunchKernelGGL((k_evolve2d<float, KCU>), g, b, 0, st, d_S);
+        else hipLaunchKernelGGL((k_evolve2d<float, UGKS>), g, b, 0, st, d_S);
     }
-    const int nw = 2 * (S.nx + S.ny);
-    if (fp64) hipLaunchKernelGGL(k_wall2d<double>, dim3(nw), dim3(256), 0, st, d_S);
-    else hipLaunchKernelGGL(k_wall2d<float>, dim3(nw), dim3(256), 0, st, d_S);
     return hipGetLastError();
 }
 
@@ -478,7 +503,7 @@ hipError_t launch_update2d(bool fp64, const Solve2D& S, const Solve2D* d_S, doub
 }
 
 hipError_t launch_resid2d(const Solve2D& S, const double* d_rcell, double* d_res, hipStream_t st) {
-    hipLaunchKernelGGL(k_resid2, dim3(1), dim3(256), 0, st, d_rcell, S.nx * S.ny, double(S.nx) * double(S.ny), d_res);
+    hipLaunchKernelGGL(k_resid2, dim3(1), dim3(1024), 0, st, d_rcell, S.nx * S.ny, double(S.nx) * double(S.ny), d_res);
     return hipGetLastError();
 }
 

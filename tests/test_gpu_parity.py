@@ -756,3 +756,31 @@ def test_split_sweep_equals_the_sweep(gpu_ctx, space, flux, collision, nv):
             assert rel_max(got[0].f, co.f) <= 1e-10 and rel_max(got[0].w, co.w) <= 1e-10
     finally:
         gpu_ctx.set_sweep_vw(0)
+
+
+@pytest.mark.parametrize("space,flux", [("2d2f2v", "ugks"), ("2d2f2v", "kcu"), ("2d2f2v", "kfvs"), ("2d1f2v", "kfvs")])
+@pytest.mark.parametrize("nu,nv", [(9, 7), (8, 8), (13, 5), (16, 16), (13, 20), (24, 24), (17, 33)])
+def test_phase_calls_at_the_edges_of_their_workgroups(gpu_ctx, space, flux, nu, nv):
+    """reconstruct!, evolve! (walls in the same launch) and update! with the residual at 63 to 576 velocities,
+    which take one to four wavefronts per face; bounds as in test_cavity_phase_exact."""
+    mk = kb.configs.cavity_2d2f2v if space == "2d2f2v" else kb.configs.cavity_2d1f2v
+    ks = kb.SolverSet(mk(nx=7, ny=9, nu=nu, nv=nv, flux=flux, vMeshType="rectangle"))
+    ctr, face = kb.init_fvm(ks)
+    ctr.f *= 1.0 + 0.02 * np.random.default_rng(nu).random(ctr.f.shape)
+    dt = kb.timestep(ks, ctr)
+    co, fo = copy.deepcopy(ctr), copy.deepcopy(face)
+    o = oracle.OracleSolve(ks, co, fo)
+    dev = kb.DeviceSolve(ks, ctr, face, precision="fp64", ctx=gpu_ctx)
+    cg, fg, rg = copy.deepcopy(ctr), copy.deepcopy(face), np.zeros(4)
+    for _ in range(2):
+        for s in (o, dev):
+            s.reconstruct()
+            s.evolve(dt)
+        ro = o.update(dt)
+        dev.update(dt, rg)
+        dev.download(cg, fg)
+        assert rel_max(fg.ff, fo.ff) <= 1e-11 and rel_max(fg.yff, fo.yff) <= 1e-11
+        assert rel_max(fg.fw, fo.fw) <= 1e-10 and rel_max(fg.yfw, fo.yfw) <= 1e-10
+        assert rel_max(cg.f, co.f) <= 1e-11
+        assert np.allclose(rg, ro[:4], rtol=1e-8)
+    dev.close()
