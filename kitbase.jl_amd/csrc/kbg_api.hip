@@ -1293,7 +1293,7 @@ size_t kbg_usolve_bytes(const kbg_udesc* d) {
     const size_t nv = d->nv > 0 ? d->nv : 0, nf = d->nf > 0 ? d->nf : 0;
     // f and face fluxes; w, prim, dmin, area, dirc, residual rows; fw, geometry, walls; index arrays;
     // velocity grid
-    return (2 * C + F) * nf * nv * esz + C * (4 + 4 + 1 + 1 + 3 + 8) * 8 + F * (4 + 3 + 4 + 5) * 8 + (C * 8 + F * 3) * 4 + 3 * nv * esz +
+    return (2 * C + F) * nf * nv * esz + C * kbg::kUCellT * esz + C * (4 + 4 + 1 + 1 + 3 + 8) * 8 + F * (4 + 3 + 4 + 5) * 8 + (C * 8 + F * 3) * 4 + 3 * nv * esz +
            sizeof(kbg::SolveUS) + 16 * 8;
 }
 
@@ -1437,6 +1437,7 @@ int kbg_usolve_create(kbg_ctx* ctx, const kbg_udesc* ud, kbg_solve** out) {
         {(void**)&S.w, C * 4 * 8},          {(void**)&S.prim, C * 4 * 8}, {&S.f, C * s->RS * s->esz}, {&S.f1, C * s->RS * s->esz},
         {(void**)&S.fw, F * 4 * 8},         {&S.ff, F * s->RS * s->esz},  {(void**)&s->rcell, C * 8 * 8},
         {(void**)&s->res, 8 * 8},           {(void**)&S.health, 8},       {(void**)&S.fws, F * 5 * 8},
+        {&S.ucell, C * kbg::kUCellT * s->esz},
     };
     for (auto& b : bufs) {
         if ((rc = dev_alloc(s, &p, b.bytes))) return bail(rc);

@@ -131,6 +131,7 @@ struct SolveUS {
     double* fw;           // [nface][4] global frame
     void* ff;             // [nface][nf][nv]
     double* fws;          // [nface][5] the fused step's face moments and wall amplitudes
+    void* ucell;          // [ncell][kUCellT] its cells' relaxation (BGK), storage type
     double* rcell;        // [ncell][8] residual rows (sum of squared change, sum of |w|)
     int* health;
 };
@@ -141,6 +142,8 @@ constexpr int kFaceCoef = 32;
 // aL[4], aR[4], aT[4], the six aX[3] products of the UGKS flux, the reciprocal centre spacings of
 // the two cells (rL, rR each) and their half widths
 constexpr int kFaceC32 = 40;
+// values per cell record of the unstructured fused step
+constexpr int kUCellT = 16;
 // values per face record of the tiled step, and its tiles' columns
 constexpr int kFaceT = 24;
 constexpr int kCellT = 16;

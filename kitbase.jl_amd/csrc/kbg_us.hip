@@ -223,11 +223,12 @@ KBG_D UCell cell_chain(const SolveUS& S, int c, const double (&po)[4], const dou
 
 // the step's constants in the storage precision
 template <class T> struct UCellT {
-    T rT, inv, rds, A, l, U, V, kb, preu, prev, Ao, lo, Uo, Vo, kbo;
+    T rT, inv, rds, A, l, U, V, kb, preu, prev, Ao, lo, Uo, Vo, kbo, pad;
 };
+static_assert(sizeof(UCellT<double>) == kUCellT * 8 && sizeof(UCellT<float>) == kUCellT * 4, "UCellT");
 template <class T> KBG_D UCellT<T> to_t(const UCell& k) {
     return UCellT<T>{T(k.rT), T(k.inv), T(k.rds), T(k.A),  T(k.l),  T(k.U),  T(k.V),  T(k.kb),
-                     T(k.preu), T(k.prev), T(k.Ao), T(k.lo), T(k.Uo), T(k.Vo), T(k.kbo)};
+                     T(k.preu), T(k.prev), T(k.Ao), T(k.lo), T(k.Uo), T(k.Vo), T(k.kbo), T(0)};
 }
 
 // one velocity of the relaxation: h (b) from its old value, the dirc-weighted face fluxes
@@ -487,17 +488,39 @@ template <class T> __global__ __launch_bounds__(256) void k_usum(const SolveUS* 
     }
 }
 
+// The FP64 chains of the stepped cells, four lanes per cell (a moment each; the same values in all four).  Shakhov
+// solves, whose chain needs the cell's heat flux, run it in k_ustep.
+template <class T> __global__ __launch_bounds__(256) void k_uchain(const SolveUS* __restrict__ pS, int rows) {
+    const SolveUS& S = *pS;
+    const int c = blockIdx.x * 64 + (threadIdx.x >> 2), lane = threadIdx.x & 3;
+    if (c >= S.ncell || !stepped(to_global(S.ctype)[c])) return;
+    const double zero[4] = {0, 0, 0, 0};
+    double dw[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+        const gptr<const double> w = to_global(S.fws) + (size_t)to_global(S.cf)[(size_t)c * 3 + j] * 5;
+        const double d = to_global(S.dirc)[(size_t)c * 3 + j];
+#pragma unroll
+        for (int m = 0; m < 4; m++) dw[m] += w[m] * d;
+    }
+    const gptr<double> rrow = rows ? to_global(S.rcell) + (size_t)c * 8 : nullptr;
+    const UCell k = cell_chain(S, c, zero, zero, dw, true, lane, rrow);
+    if (lane == 0) ((UCellT<T>*)S.ucell)[c] = to_t<T>(k);
+}
+
 // The fused step's cells, one wavefront per cell, four cells per workgroup (no workgroup barrier): every lane
-// runs the FP64 chain (the same values in all lanes), then forms its velocities' fluxes from the upwind
-// cells and relaxes from one f buffer into the other.
-template <class T> __global__ __launch_bounds__(256) void k_ustep(const SolveUS* __restrict__ pS, int par, int rows, int chunk) {
+// forms its velocities' fluxes from the upwind cells and relaxes from one f buffer into the other.  CHAIN: every
+// lane first runs the FP64 chain (the same values in all lanes).  With the chain in k_uchain the wavefronts hold
+// fewer registers (FP32 68 against 102) and start with their loads: 41 -> 31.5 us at 8192 triangles x 28^2 velocities in
+// FP32, with 5 us for k_uchain.
+template <class T, bool CHAIN> __global__ __launch_bounds__(256) void k_ustep(const SolveUS* __restrict__ pS, int par, int rows, int chunk) {
     const SolveUS& S = *pS;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     // the wavefront's cell, a wavefront-uniform value: the cell's and its faces' data go to scalar registers
     const int c = __builtin_amdgcn_readfirstlane((int(blockIdx.x % kXcd) * chunk + int(blockIdx.x / kXcd)) * 4 + wave);
     if (c >= S.ncell) return;
     const int nv = S.nv, RS = S.nf * nv;
-    const bool two = S.nf == 2, shak = two && S.coll == SHAKHOV;
+    const bool two = S.nf == 2, shak = CHAIN && two && S.coll == SHAKHOV;
     const gptr<const T> fin = fbuf<T>(S, par);
     const gptr<T> fout = fbuf<T>(S, par + 1);
     const gptr<const T> fc = fin + (size_t)c * RS;
@@ -509,9 +532,11 @@ template <class T> __global__ __launch_bounds__(256) void k_ustep(const SolveUS*
         if (rrow && lane < 8) rrow[lane] = 0.0;
         return;
     }
-    double po[4];
+    double po[4] = {1, 0, 0, 1};
+    if constexpr (CHAIN) {
 #pragma unroll
-    for (int m = 0; m < 4; m++) po[m] = to_global(S.prim)[(size_t)c * 4 + m];
+        for (int m = 0; m < 4; m++) po[m] = to_global(S.prim)[(size_t)c * 4 + m];
+    }
     const gptr<const double> dr = to_global(S.dirc) + (size_t)c * 3;
     const gptr<const T> U = to_global((const T*)S.u), V = to_global((const T*)S.v), WT = to_global((const T*)S.wt);
     UFace F[3];
@@ -527,17 +552,25 @@ template <class T> __global__ __launch_bounds__(256) void k_ustep(const SolveUS*
         d[j] = T(dr[j]);
         const gptr<const double> w = to_global(S.fws) + (size_t)f * 5;
         A[j] = T(w[4]);
+        if constexpr (CHAIN) {
 #pragma unroll
-        for (int m = 0; m < 4; m++) dw[m] += w[m] * dr[j];
-    }
-    double q[4] = {0, 0, 0, 0};
-    if (shak) {
-        const T Uo = T(po[1]), Vo = T(po[2]);
-        for (int iv = lane; iv < nv; iv += 64) heat_vel(U[iv], V[iv], WT[iv], fc[iv], fc[nv + iv], Uo, Vo, q);
-        wave_allreduce<4>(q);
+            for (int m = 0; m < 4; m++) dw[m] += w[m] * dr[j];
+        }
     }
     const T dtT = T(S.dt), KT = T(S.K);
-    const UCellT<T> kt = to_t<T>(cell_chain(S, c, po, q, dw, true, lane, rrow));
+    UCellT<T> kt;
+    if constexpr (CHAIN) {
+        double q[4] = {0, 0, 0, 0};
+        if (shak) {
+            const T Uo = T(po[1]), Vo = T(po[2]);
+            for (int iv = lane; iv < nv; iv += 64) heat_vel(U[iv], V[iv], WT[iv], fc[iv], fc[nv + iv], Uo, Vo, q);
+            wave_allreduce<4>(q);
+        }
+        kt = to_t<T>(cell_chain(S, c, po, q, dw, true, lane, rrow));
+    } else {
+        const __attribute__((address_space(4))) T* r = (const __attribute__((address_space(4))) T*)S.ucell + (size_t)c * kUCellT;  // scalar loads
+        kt = UCellT<T>{r[0], r[1], r[2], r[3], r[4], r[5], r[6], r[7], r[8], r[9], r[10], r[11], r[12], r[13], r[14], T(0)};
+    }
     constexpr int NB = sizeof(T) == 4 ? 2 : 1;  // velocities per lane in flight
     for (int v0 = lane; v0 < nv; v0 += 64 * NB) {
         UVel<T> x[NB];
@@ -689,13 +722,21 @@ hipError_t launch_ustep(bool fp64, const SolveUS& S, const SolveUS* d_S, int par
     // four faces or cells per workgroup; workgroup b -> group (b % 8) chunk + b / 8 covers [0, 8 chunk) once
     // (each XCD a contiguous run); groups past the end exit
     const int fch = ((S.nface + 3) / 4 + kXcd - 1) / kXcd, cch = ((S.ncell + 3) / 4 + kXcd - 1) / kXcd;
-    const dim3 gf(unsigned(fch) * kXcd), gc(unsigned(cch) * kXcd), b(256);
+    const dim3 gf(unsigned(fch) * kXcd), gc(unsigned(cch) * kXcd), gk((S.ncell + 63) / 64), b(256);
+    // the chains in a launch of their own pay for it on large meshes.  us per step, in k_ustep / apart: 512
+    // triangles x 16^2 velocities FP32 12.1 / 14.2, 2048 x 28^2 (1.6 M) FP32 28.4 / 29.2, FP64 39.0 / 40.2, 8192 x 28^2
+    // (6.4 M) FP32 66 / 60, FP64 107 / 100, 18432 x 40^2 FP32 291 / 245, FP64 524 / 509
+    const bool chain = (S.nf == 2 && S.coll == SHAKHOV) || size_t(S.ncell) * S.nv < 4000000u;
     if (fp64) {
         if (S.nface > 0) hipLaunchKernelGGL(k_usum<double>, gf, b, 0, st, d_S, par, fch);
-        hipLaunchKernelGGL(k_ustep<double>, gc, b, 0, st, d_S, par, rows, cch);
+        if (!chain) hipLaunchKernelGGL(k_uchain<double>, gk, b, 0, st, d_S, rows);
+        if (chain) hipLaunchKernelGGL((k_ustep<double, true>), gc, b, 0, st, d_S, par, rows, cch);
+        else hipLaunchKernelGGL((k_ustep<double, false>), gc, b, 0, st, d_S, par, rows, cch);
     } else {
         if (S.nface > 0) hipLaunchKernelGGL(k_usum<float>, gf, b, 0, st, d_S, par, fch);
-        hipLaunchKernelGGL(k_ustep<float>, gc, b, 0, st, d_S, par, rows, cch);
+        if (!chain) hipLaunchKernelGGL(k_uchain<float>, gk, b, 0, st, d_S, rows);
+        if (chain) hipLaunchKernelGGL((k_ustep<float, true>), gc, b, 0, st, d_S, par, rows, cch);
+        else hipLaunchKernelGGL((k_ustep<float, false>), gc, b, 0, st, d_S, par, rows, cch);
     }
     return hipGetLastError();
 }

@@ -320,3 +320,19 @@ def test_us_fused_step_at_the_edges_of_its_velocity_batches(space, nu, nv):
         err = rel_max if precision == "fp64" else rel_l2
         assert err(sg.w, so.w) < tol
         assert err(sg.f, so.f) < tol
+
+
+@pytest.mark.parametrize("space,precision", [("2d2f2v", "fp64"), ("2d2f2v", "fp32"), ("2d1f2v", "fp64")])
+def test_us_chains_in_a_launch_of_their_own(space, precision):
+    """Above 4 M cells x velocities k_uchain runs the BGK cells' chains: residual rows, averaged cells and stored
+    faces as in the smaller solves; bounds as above."""
+    ks, ps, st, dt = case(space, n=28, nx=53, ny=50)
+    ps.cellType[boundary_cells(ps, 3)] = 3
+    st = kb.mesh.init_fvm_us(ks, ps)
+    assert ps.ncell * ks.vs.u.size > 4000000
+    sg, so, rg, ro = run_both(ks, ps, st, dt, 3, precision)
+    if precision == "fp64":
+        assert rel_max(sg.f, so.f) <= 1e-10 and rel_max(sg.w, so.w) <= 1e-10
+        assert rel_max(rg, ro) <= 1e-8
+    else:
+        assert rel_l2(sg.f, so.f) <= 1e-4 and rel_l2(sg.w, so.w) <= 1e-4
