@@ -974,10 +974,9 @@ size_t kbg_solve_bytes(const kbg_desc* d) {
             // spectrum, the transforms' products, kernel modes (all in the storage precision), Q (FP64);
             // hipFFT's own work area not counted
             const size_t nc = size_t(d->nx) - 2, n3 = size_t(d->nv), nd = size_t(d->fsm_nm) * (d->fsm_nm - 1);
-            const size_t cn = kbg::fsm_cube_size(d->fsm_shape[0], d->fsm_shape[1], d->fsm_shape[2], esz == 4, d->fsm_nm, d->fsm_phi, d->fsm_psi, d->fsm_phipsi);
-            fsm = nc * n3 * 2 * esz + nc * n3 * 8;
-            if (cn && esz == 8) fsm += ((nd + 2) * (nc + 2) * n3 + nd * (nc + 1) * 6 * cn * cn + 2 * cn) * 8;
-            else fsm += (cn ? nc * (nd + 1) * n3 * 4 : nc * (2 * nd + 2) * n3 * 2 * esz) + cn * 2 * esz + (2 * nd + 1) * n3 * esz;
+            const int cn = kbg::fsm_cube_size(d->fsm_shape[0], d->fsm_shape[1], d->fsm_shape[2]);
+            const size_t work = (cn && esz == 4 ? nc * (nd + 1) * n3 * 4 : nc * (2 * nd + 2) * n3 * 2 * esz) + size_t(cn) * 2 * esz;
+            fsm = nc * n3 * 2 * esz + work + (2 * nd + 1) * n3 * esz + nc * n3 * 8;
         }
         size_t w3 = 0;
         if (d->vdim == 3 && d->flux == KBG_KFVS && d->interp_order == 2) {
@@ -1139,42 +1138,28 @@ int kbg_solve_create(kbg_ctx* ctx, const kbg_desc* desc, kbg_solve** out) {
             P.c0 = 2;
             P.ncell = d.nx - 2;
             P.f32 = !s->fp64;
-            P.cube_n = kbg::fsm_cube_size(P.nu, P.nv, P.nw, P.f32, P.M, d.fsm_phi, d.fsm_psi, d.fsm_phipsi);
+            P.cube_n = kbg::fsm_cube_size(P.nu, P.nv, P.nw);
             const size_t n3 = size_t(d.nv), nd = size_t(P.M) * (P.M - 1), nc = size_t(P.ncell), re = P.f32 ? 4 : 8;
             if (S.fvs != 1) return bail(fail(KBG_ERR_STATE, ":fsm needs the velocity-contiguous f layout"));
-            // cubes keep one real product per pair (and, packed, the loss transforms and the Nyquist planes'
-            // transforms); other grids the transformed mode products
-            P.packed = P.cube_n > 0 && !P.f32;
-            const bool cube = P.cube_n > 0, packed = P.packed;
-            const size_t n2 = size_t(P.cube_n) * P.cube_n, np = packed ? nd + 2 : nd + 1;
+            // the FP32 LDS path keeps one FP32 product per pair instead of the transformed mode products
+            const bool lds = P.cube_n && P.f32;
+            const size_t work = lds ? 0 : nc * (2 * nd + 2) * n3 * 2 * re;
+            const size_t part = lds ? nc * (nd + 1) * n3 * 4 : 0, twb = size_t(P.cube_n) * 2 * re;
             struct {
                 void** dst;
                 size_t bytes;
-            } bufs[] = {{&P.spec, nc * n3 * 2 * re},
-                        {(void**)&P.Q, nc * n3 * 8},
-                        {&P.work, cube ? 0 : nc * (2 * nd + 2) * n3 * 2 * re},
-                        {&P.phi, packed ? 0 : nd * n3 * re},
-                        {&P.psi, packed ? 0 : nd * n3 * re},
-                        {&P.phipsi, packed ? 0 : n3 * re},
-                        {&P.ms, packed ? np * n3 * 2 * re : 0},
-                        {&P.mo, packed ? nd * 3 * n2 * 2 * re : 0},
-                        {&P.planes, packed ? nc * nd * 3 * n2 * 2 * re : 0},
-                        {&P.part, cube ? nc * np * n3 * re : 0},
-                        {&P.tw, size_t(P.cube_n) * 2 * re}};
+            } bufs[] = {{&P.spec, nc * n3 * 2 * re}, {&P.work, work},       {&P.phi, nd * n3 * re},
+                        {&P.psi, nd * n3 * re},      {&P.phipsi, n3 * re},  {(void**)&P.Q, nc * n3 * 8},
+                        {(void**)&P.part, part},     {&P.tw, twb}};
             for (auto& b : bufs) {
                 if (!b.bytes) continue;
                 if ((rc = dev_alloc(s, &p, b.bytes))) return bail(rc);
                 *b.dst = p;
             }
-            if (packed) {
-                std::vector<double> ms(np * n3 * 2), mo(nd * 3 * n2 * 2, 0.0);
-                kbg::fsm_pack_modes(P.cube_n, P.M, d.fsm_phi, d.fsm_psi, d.fsm_phipsi, ms.data(), mo.data());
-                if ((rc = put_f64(s, (double*)P.ms, ms.data(), ms.size())) || (rc = put_f64(s, (double*)P.mo, mo.data(), mo.size()))) return bail(rc);
-            } else if ((rc = put_real(s, P.phi, d.fsm_phi, nd * n3, P.f32)) || (rc = put_real(s, P.psi, d.fsm_psi, nd * n3, P.f32)) ||
-                       (rc = put_real(s, P.phipsi, d.fsm_phipsi, n3, P.f32))) {
+            if ((rc = put_real(s, P.phi, d.fsm_phi, nd * n3, P.f32)) || (rc = put_real(s, P.psi, d.fsm_psi, nd * n3, P.f32)) ||
+                (rc = put_real(s, P.phipsi, d.fsm_phipsi, n3, P.f32)))
                 return bail(rc);
-            }
-            if (cube) {
+            if (P.cube_n) {
                 std::vector<double> tw(2 * P.cube_n);
                 for (int j = 0; j < P.cube_n; j++) {
                     tw[2 * j] = std::cos(-2.0 * kbg::kPi * j / P.cube_n);
@@ -1183,7 +1168,7 @@ int kbg_solve_create(kbg_ctx* ctx, const kbg_desc* desc, kbg_solve** out) {
                 if ((rc = put_real(s, P.tw, tw.data(), tw.size(), P.f32))) return bail(rc);
             }
             HIPCHK(hipMemset(P.Q, 0, nc * n3 * 8));
-            if (kbg::fsm_plan_create(P) != hipSuccess) return bail(fail(KBG_ERR_HIP, "setting up the :fsm transforms failed"));
+            if (kbg::fsm_plan_create(P) != hipSuccess) return bail(fail(KBG_ERR_HIP, "hipfftPlanMany failed for the :fsm transforms"));
             s->has_fsm = true;
             S.fsmq = P.Q;
             S.fsm_c0 = P.c0;

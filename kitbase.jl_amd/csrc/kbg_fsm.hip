@@ -1,33 +1,24 @@
 // kbg_fsm.hip -- KitBase's fast spectral Boltzmann collision operator (boltzmann_fft!,
 // theory_fsm.jl:271-314) for the 1D1F3V step!(:fsm) (step_1f.jl:122-157), on gfx950.
 //
-// Per step, for the interior cells c0 .. c0 + ncell - 1 of a solve, with f_spec = fftshift(bfft(f)) / n3,
-//   Q = 4 pi^2 / Kn / M^2 Re(sum_d F[f_spec phi_d] F[f_spec psi_d] - F[f_spec phipsi] F[f_spec])
-// (d < M(M-1), F the forward 3D transform, sums in FP64).  The kernel modes phi, psi, phipsi
-// (kernel_mode, theory_fsm.jl:24-90) come from the host with the descriptor.  Arrays are [w][v][u]
-// with u fastest (KitBase's column-major f[i, j, k]); transforms, spectra and modes are FP64 for FP64
-// storage and FP32 for FP32 storage (R below).  The update kernel adds dt Q to the transport update.
-//
-// Cubic grids of side 8, 12, 16, 18 or 24 take the library's own pencil transforms (kbg_fft.h):
-//   FP64, modes even in the frequency (KitBase's are): one complex transform per pair of modes
-//     k_fsm_spec    f_spec of every cell
-//     k_fsm_slab    F of f_spec (a + i b) per (cell, pair), a and b the even parts of the pair's two modes
-//     k_fsm_planes  the 2D transforms of the modes' odd parts, which live on the Nyquist planes
-//     k_fsm_psum    Q from both
-//   FP32: two transforms per pair, all of a pair in LDS
-//     k_fsm_load, hipFFT backward, k_fsm_pair, k_fsm_sum
-// Other grids and modes go through hipFFT:
-//   k_fsm_load    f (storage precision) -> complex spec[cell][n3]
-//   hipFFT        batched 3D backward transforms (bfft, unnormalised), one per cell
-//   k_fsm_modes   the 2 M(M-1) + 2 products f_spec phi_d, f_spec psi_d, f_spec phipsi, f_spec -> work
-//   hipFFT        batched 3D forward transforms of all the products in place
-//   k_fsm_q       the sum of the products
+// Per step, for the interior cells c0 .. c0 + ncell - 1 of a solve:
+//   k_fsm_load   f (storage precision) -> complex spec[cell][n3]
+//   hipFFT       batched 3D backward transforms (bfft, unnormalised), one per cell
+//   k_fsm_modes  f_spec = fftshift(spec) / n3, then per cell the 2 M(M-1) + 2 products
+//                f_spec phi_d, f_spec psi_d (d < M(M-1)), f_spec phipsi, f_spec -> work
+//   hipFFT       batched 3D forward transforms of all the products in place
+//   k_fsm_q      Q = 4 pi^2 / Kn / M^2 Re(sum_d F[f_spec phi_d] F[f_spec psi_d]
+//                                      - F[f_spec phipsi] F[f_spec])   (sums in FP64)
+// The transforms, the spectra and the kernel modes are FP64 for FP64 storage and FP32 for FP32
+// storage (R below).  hipFFT's forward pass streams the 2 M(M-1) + 2 product arrays per cell through
+// HBM about a dozen times; on cubic grids of side 8, 12, 16, 18 or 24 the forward transforms are the
+// library's own pencil transforms instead (kbg_fft.h): FP32 entirely in LDS (k_fsm_pair), FP64
+// written once and read once (k_fsm_slab64, k_fsm_q).  Q is FP64 in all of them.  The kernel modes phi,
+// psi, phipsi (kernel_mode, theory_fsm.jl:24-90) come from the host with the descriptor.  Arrays are
+// [w][v][u] with u fastest (KitBase's column-major f[i, j, k]).  The update kernel then adds dt Q to
+// the transport update (k_update1d).
 #include <hip/hip_runtime.h>
 #include <hipfft/hipfft.h>
-
-#include <algorithm>
-#include <cmath>
-#include <type_traits>
 
 #include "kbg_device.h"
 #include "kbg_fft.h"
@@ -107,12 +98,6 @@ __global__ __launch_bounds__(256) void k_fsm_q(const cx_t<R>* __restrict__ work,
     Q[i] = scale * re;
 }
 
-KBG_D int fsm_xcd_item() {
-    const int G = gridDim.x, bx = blockIdx.x;
-    const int x8 = bx & 7, q8 = G >> 3, r8 = G & 7;
-    return x8 * q8 + (x8 < r8 ? x8 : r8) + (bx >> 3);
-}
-
 // ---- FP32 storage on a cubic grid of N^3 velocities (N from fsm_cube_size): the forward transforms
 // in LDS, no product array.  One workgroup per (cell, pair): pair p < nd transforms f_spec phi_p and
 // f_spec psi_p, pair nd transforms f_spec phipsi and f_spec; the product Re(A B) of the two
@@ -125,6 +110,12 @@ KBG_D int fsm_xcd_item() {
 //   2. transforms the u-pencil (v, w) = (ta, tb) in LDS;
 //   3. transforms the v-pencil (u, w) = (ta, tb) and keeps it in registers, where the second
 //      transform's pencil meets the first.
+KBG_D int fsm_xcd_item() {
+    const int G = gridDim.x, bx = blockIdx.x;
+    const int x8 = bx & 7, q8 = G >> 3, r8 = G & 7;
+    return x8 * q8 + (x8 < r8 ? x8 : r8) + (bx >> 3);
+}
+
 template <int N> constexpr int fsm_pair_threads() { return (N * N + 63) / 64 * 64; }
 // the first transform's kept v-pencil: its first KEEP values wait in LDS behind the array (registers
 // for the rest), which keeps the kernel within the register budget of 576-thread workgroups
@@ -202,6 +193,74 @@ __global__ __launch_bounds__(fsm_pair_threads<N>()) void k_fsm_pair(const float2
     }
 }
 
+// ---- FP64 storage on a cubic grid: the transforms of the products f_spec phi_d, f_spec psi_d,
+// f_spec phipsi, f_spec in the layout of k_fsm_modes (work[cell][2 M(M-1) + 2][n3]), each written
+// once by k_fsm_slab64, then k_fsm_q.  One workgroup per slab of S w-planes of one product array:
+//   1. every w-pencil (u, v) of the array: f_spec times the mode straight from the backward
+//      transform's output (the fftshift is an index map), transformed along w in registers; the S
+//      frequencies of the slab go to LDS (rows padded to an odd length).  The N / S slabs of an array
+//      each redo these transforms: arithmetic from L2-resident inputs instead of a pass over HBM;
+//   2. one thread per u-pencil of the slab, in LDS;
+//   3. one thread per v-pencil, whose transform goes straight to the array.
+template <int N> constexpr int fsm_slab() { return N % 8 == 0 ? 8 : 6; }
+template <int N> constexpr int fsm_slab_threads() { return (fsm_slab<N>() * N + 63) / 64 * 64; }
+template <int N> constexpr int fsm_slab_lds() { return fsm_slab<N>() * N * (N | 1) * 16; }
+
+template <int N>
+__global__ __launch_bounds__(fsm_slab_threads<N>()) void k_fsm_slab64(const double2* __restrict__ spec, const double* __restrict__ phi,
+                                                                    const double* __restrict__ psi, const double* __restrict__ phipsi,
+                                                                    const double2* __restrict__ tw, double2* __restrict__ work, int nd,
+                                                                    int ncell) {
+    constexpr int N2 = N * N, N3 = N2 * N, P = N | 1, H = N / 2, S = fsm_slab<N>(), NS = N / S;
+    constexpr int NTH = fsm_slab_threads<N>();
+    extern __shared__ double2 slab[];
+    const int na = 2 * nd + 2;
+    const int item = fsm_xcd_item();
+    if (item >= ncell * na * NS) return;
+    const int sl = item % NS, a = (item / NS) % na, ci = item / (NS * na);
+    const int p = a >> 1, h = a & 1;
+    const double* __restrict__ mode = p < nd ? (h ? psi : phi) + (size_t)p * N3 : (h ? nullptr : phipsi);
+    const double inv = 1.0 / double(N3);
+    const int t = threadIdx.x;
+    double2 x[N], X[N];
+    // 1. along w, every pencil of the array; the slab's planes kept
+    for (int pen = t; pen < N2; pen += NTH) {
+        const int ta = pen % N, tb = pen / N;
+        const double2* __restrict__ col = spec + (size_t)ci * N3 + (ta + N - H) % N + N * ((tb + N - H) % N);
+#pragma unroll
+        for (int k = 0; k < N; k++) {
+            const double2 z = col[N2 * ((k + N - H) % N)];
+            const double m = mode ? mode[pen + N2 * k] : 1.0;
+            x[k] = make_double2((z.x * inv) * m, (z.y * inv) * m);
+        }
+        fft_dit<N, N, 1, double2>(x, X, tw);
+#pragma unroll
+        for (int k = 0; k < N; k++)  // compile-time register indices, a uniform branch per plane
+            if (k / S == sl) slab[ta + P * (tb + N * (k % S))] = X[k];
+    }
+    __syncthreads();
+    const bool act = t < S * N;
+    const int ta = t % N, tb = t / N;
+    if (act) {  // 2. along u: pencil (v, w) = (ta, tb)
+        double2* r = slab + P * (ta + N * tb);
+#pragma unroll
+        for (int k = 0; k < N; k++) x[k] = r[k];
+        fft_dit<N, N, 1, double2>(x, X, tw);
+#pragma unroll
+        for (int k = 0; k < N; k++) r[k] = X[k];
+    }
+    __syncthreads();
+    if (act) {  // 3. along v: pencil (u, w) = (ta, tb), to the array
+        const double2* r = slab + ta + P * N * tb;
+#pragma unroll
+        for (int k = 0; k < N; k++) x[k] = r[P * k];
+        fft_dit<N, N, 1, double2>(x, X, tw);
+        double2* __restrict__ o = work + ((size_t)ci * na + a) * N3 + ta + N2 * (sl * S + tb);
+#pragma unroll
+        for (int k = 0; k < N; k++) o[N * k] = X[k];
+    }
+}
+
 // Q = scale (sum_{p < nd} part_p - part_nd), pairs in order
 __global__ __launch_bounds__(256) void k_fsm_sum(const float* __restrict__ part, double* __restrict__ Q, int n3, int nd,
                                                  int ncell, double scale) {
@@ -220,250 +279,23 @@ template <int N> hipError_t launch_pair(const FsmPlan& P, hipStream_t st) {
     const int nd = P.M * (P.M - 1);
     hipLaunchKernelGGL(k_fsm_pair<N>, dim3(P.ncell * (nd + 1)), dim3(fsm_pair_threads<N>()), fsm_pair_lds<N>(), st,
                        (const float2*)P.spec, (const float*)P.phi, (const float*)P.psi, (const float*)P.phipsi,
-                       (const float2*)P.tw, (float*)P.part, nd, P.ncell);
+                       (const float2*)P.tw, P.part, nd, P.ncell);
     return hipGetLastError();
 }
 
-// ---- FP64 storage on a cubic grid of N^3 velocities, even kernel modes ------------------------------
-//
-// f is real, so f_spec is Hermitian: f_spec(k') = conj f_spec(k), k' the index of the negated frequency
-// ((N - i) % N per axis in the shifted layout; index 0, the Nyquist frequency, is its own partner).  A
-// mode m splits into m_e(k) = (m(k) + m(k')) / 2 and m_o = m - m_e.  f_spec m_e is Hermitian, its transform
-// real; f_spec m_o is anti-Hermitian, its transform imaginary.  For a pair of modes (a, b) the transform
-// of f_spec (a_e + i b_e) is then A_r + i B_r -- both real transforms at once -- and that of
-// f_spec (a_o + i b_o) is -B_i + i A_i, so with Z and Zo the two transforms
-//   Re(F[f_spec a] F[f_spec b]) = A_r B_r - A_i B_i = Re Z Im Z + Re Zo Im Zo.
-// KitBase's modes are even functions of the frequency, so m_o vanishes except on the planes where one
-// index is 0 (there the partner negates only the other two axes): Zo(x, y, z) = P0(y, z) + P1(x, z) + P2(x, y),
-// three 2D transforms.  fsm_pack_modes forms (a_e, b_e) and the planes of (a_o, b_o) on the host,
-// scales a and b of a pair to the same size by powers of two (their product is unchanged), and
-// reports whether the modes are even off the planes.
-//
-// Pair p < nd is (phi_p, psi_p).  The loss term takes two transforms, F[f_spec phipsi] and F[f_spec]
-// (part[nd] and part[nd + 1] hold their real parts; F[f_spec] is real).  Packed as a pair (phipsi, 1) it
-// would lose digits, its two transforms differing by orders of magnitude over the velocity grid (4e-5 of
-// Q in FP32 on the 24^3 shock structure, against 3e-6); with F[f_spec] = (-1)^(x+y+z) f, exact, gain and
-// loss would no longer come from the same rounded spectrum, and their moments would not cancel.
-
-// w-planes per slab; the N / S slabs of an array take the frequencies congruent r mod N / S
-template <int N> constexpr int fsm_slab() { return N % 8 == 0 ? 8 : 6; }
-template <int N> constexpr int fsm_slab_threads() { return (fsm_slab<N>() * N + 63) / 64 * 64; }
-template <int N> constexpr int fsm_slab_lds() { return fsm_slab<N>() * N * (N | 1) * 16; }
-
-// The S frequencies NS q + r (q < S) of a length-N pencil x: one output of the radix-NS butterfly over
-// x[m], x[m + S], .. (decimation in frequency), a twiddle, and a length-S transform.  load(k) returns x[k].
-template <int N, int S, int RR, class F> KBG_D void fsm_pencil_part(F&& load, double2 (&X)[S], const double2* __restrict__ tw) {
-    constexpr int NS = N / S;
-    double2 y[S];
-#pragma unroll
-    for (int m = 0; m < S; m++) {
-        double2 a = load(m);
-        if constexpr (NS == 2) {
-            const double2 b = load(m + S);
-            a = RR ? fft_cx<double2>(a.x - b.x, a.y - b.y) : fft_cx<double2>(a.x + b.x, a.y + b.y);
-        } else if constexpr (NS == 3) {
-            const double2 b = load(m + S), c = load(m + 2 * S);
-            const double2 s = fft_cx<double2>(b.x + c.x, b.y + c.y);
-            if constexpr (RR == 0) {
-                a = fft_cx<double2>(a.x + s.x, a.y + s.y);
-            } else {
-                const double h = RR == 1 ? 0.86602540378443864676 : -0.86602540378443864676;
-                const double2 d = fft_cx<double2>(b.x - c.x, b.y - c.y);
-                a = fft_cx<double2>(a.x - 0.5 * s.x + h * d.y, a.y - 0.5 * s.y - h * d.x);
-            }
-        }
-        y[m] = fft_twiddle<N, double2>(a, m * RR, tw);
-    }
-    fft_dit<S, N, 1, double2>(y, X, tw);
-}
-
-// The slab r of the 3D transform of the array load(pen, k) (pen = u + N v, k the w index): w-pencils in
-// registers, the slab's S planes in LDS (rows padded to an odd length, so the pencils a wavefront reads
-// fall in different banks), u-pencils in LDS, v-pencils in registers, then store(u, v, q, X) for the
-// thread's (u, q) and every v; w frequency NS q + r.  Threads: fsm_slab_threads.
-template <int N, class L, class ST>
-KBG_D void fsm_slab_transform(int r, double2* __restrict__ slab, const double2* __restrict__ tw, L&& load, ST&& store) {
-    constexpr int N2 = N * N, P = N | 1, S = fsm_slab<N>(), NS = N / S, NTH = fsm_slab_threads<N>();
-    const int t = threadIdx.x;
-    for (int pen = t; pen < N2; pen += NTH) {
-        double2 X[S];
-        auto ld = [&](int k) { return load(pen, k); };
-        if constexpr (NS == 1) {
-            fsm_pencil_part<N, S, 0>(ld, X, tw);
-        } else {  // r is uniform over the workgroup
-            if (r == 0) fsm_pencil_part<N, S, 0>(ld, X, tw);
-            else if (r == 1) fsm_pencil_part<N, S, 1>(ld, X, tw);
-            else if constexpr (NS == 3) fsm_pencil_part<N, S, 2>(ld, X, tw);
-        }
-        double2* o = slab + pen % N + P * (pen / N);
-#pragma unroll
-        for (int q = 0; q < S; q++) o[P * N * q] = X[q];
-    }
-    __syncthreads();
-    const bool act = t < S * N;
-    const int ta = t % N, tb = t / N;
-    double2 x[N], X[N];
-    if (act) {  // u-pencil (v, q) = (ta, tb)
-        double2* row = slab + P * (ta + N * tb);
-#pragma unroll
-        for (int k = 0; k < N; k++) x[k] = row[k];
-        fft_dit<N, N, 1, double2>(x, X, tw);
-#pragma unroll
-        for (int k = 0; k < N; k++) row[k] = X[k];
-    }
-    __syncthreads();
-    if (act) {  // v-pencil (u, q) = (ta, tb)
-        const double2* col = slab + ta + P * N * tb;
-#pragma unroll
-        for (int k = 0; k < N; k++) x[k] = col[P * k];
-        fft_dit<N, N, 1, double2>(x, X, tw);
-#pragma unroll
-        for (int k = 0; k < N; k++) store(ta, k, tb, X[k]);
-    }
-}
-
-// f_spec = fftshift(bfft(f)) / N^3 of one slab of one cell: f is real, so bfft(f) = conj F[f]
-template <int N>
-__global__ __launch_bounds__(fsm_slab_threads<N>()) void k_fsm_spec(const double* __restrict__ f, long fcs, int k0, const double2* __restrict__ tw,
-                                                                   double2* __restrict__ spec) {
-    constexpr int N2 = N * N, N3 = N2 * N, H = N / 2, NS = N / fsm_slab<N>();
-    extern __shared__ char smem[];
-    const int r = blockIdx.x % NS, ci = blockIdx.x / NS;
-    const double* __restrict__ fc = f + (long)(k0 + ci) * fcs;
-    double2* __restrict__ o = spec + (size_t)ci * N3;
-    const double inv = 1.0 / double(N3);
-    fsm_slab_transform<N>(
-        r, (double2*)smem, tw, [&](int pen, int k) { return fft_cx<double2>(fc[pen + N2 * k], 0.0); },
-        [&](int u, int v, int q, double2 X) {
-            o[(u + H) % N + N * ((v + H) % N) + N2 * ((NS * q + r + H) % N)] = fft_cx<double2>(X.x * inv, -X.y * inv);
-        });
-}
-
-// The order of the slab work: each XCD (workgroup ids congruent mod 8) takes a contiguous run of
-// [cell group][pair][cell of the group][slab], groups of ceil(ncell / 8) cells, so a pair's modes are
-// read once into an XCD's L2 and reused by the group's cells, whose spectra stay there (FP64 24^3:
-// 6 cells x 221 KB + 221 KB of modes against 4.6 MB of modes in cell-major order).
-//
-// part[cell][pair] = Re Z Im Z, Z the transform of f_spec (a_e + i b_e), and part[cell][nd], [nd + 1] = Re Z for
-// the loss; one workgroup per (cell, pair, slab).  A slab keeps S/N of the array in LDS (77 KB of 24^3), so two workgroups share a CU.  For the
-// 48 cells x 21 pairs of 24^3: 81 us, and 37 us for k_fsm_psum (two transforms per pair, written and read
-// back as 446 MB of complex products, took 167 + 109 us).
-template <int N>
-__global__ __launch_bounds__(fsm_slab_threads<N>()) void k_fsm_slab(const double2* __restrict__ spec, const double2* __restrict__ ms,
-                                                                   const double2* __restrict__ tw, double* __restrict__ part, int np, int ncell,
-                                                                   int cg) {
-    constexpr int N2 = N * N, N3 = N2 * N, NS = N / fsm_slab<N>();
-    extern __shared__ char smem[];
-    const int item = fsm_xcd_item(), per = cg * np * NS, g = item / per;
-    const int in = item - g * per, ncg = min(cg, ncell - g * cg);
-    const int r = in % NS, ci = g * cg + (in / NS) % ncg, p = in / (NS * ncg);
-    const double2* __restrict__ sc = spec + (size_t)ci * N3;
-    const double2* __restrict__ mp = ms + (size_t)p * N3;
-    double* __restrict__ o = part + ((size_t)ci * np + p) * N3;
-    fsm_slab_transform<N>(
-        r, (double2*)smem, tw,
-        [&](int pen, int k) {
-            const double2 s = sc[pen + N2 * k], m = mp[pen + N2 * k];
-            return fft_cx<double2>(s.x * m.x - s.y * m.y, s.x * m.y + s.y * m.x);
-        },
-        [&](int u, int v, int q, double2 X) { o[u + N * v + N2 * (NS * q + r)] = p < np - 2 ? X.x * X.y : X.x; });
-}
-
-// The 2D transforms of f_spec (a_o + i b_o) on the planes u = 0 ([w][v]), v = 0 ([w][u]) and w = 0
-// ([v][u]) of each pair; kFsmPP pairs of one cell per workgroup (at most 64 KB of LDS), one pencil per thread
-constexpr int kFsmPP = 2;
-template <int N> constexpr int fsm_plane_threads() { return (3 * kFsmPP * N + 63) / 64 * 64; }
-template <int N>
-__global__ __launch_bounds__(fsm_plane_threads<N>()) void k_fsm_planes(const double2* __restrict__ spec, const double2* __restrict__ mo,
-                                                                      const double2* __restrict__ tw, double2* __restrict__ planes,
-                                                                      int np) {
-    constexpr int N2 = N * N, N3 = N2 * N, P = N | 1, PP = kFsmPP;
-    __shared__ double2 lds[3 * PP * N * P];
-    const int ng = (np + PP - 1) / PP, ci = blockIdx.x / ng;
-    const int t = threadIdx.x, ta = t % N, pl = (t / N) % 3, p = (blockIdx.x % ng) * PP + t / (3 * N);
-    const bool act = t < 3 * PP * N && p < np;
-    double2* a = lds + (t / N) * N * P;
-    double2 x[N], X[N];
-    if (act) {  // the pencil along the plane's slow axis at fast index ta
-        const double2* __restrict__ sc = spec + (size_t)ci * N3 + (pl == 0 ? N * ta : ta);
-        const double2* __restrict__ mp = mo + ((size_t)p * 3 + pl) * N2 + ta;
-        const int st = pl == 2 ? N : N2;
-#pragma unroll
-        for (int k = 0; k < N; k++) {
-            const double2 s = sc[st * k], m = mp[N * k];
-            x[k] = fft_cx<double2>(s.x * m.x - s.y * m.y, s.x * m.y + s.y * m.x);
-        }
-        fft_dit<N, N, 1, double2>(x, X, tw);
-#pragma unroll
-        for (int k = 0; k < N; k++) a[P * k + ta] = X[k];
-    }
-    __syncthreads();
-    if (act) {  // the fast axis at slow index ta
-#pragma unroll
-        for (int k = 0; k < N; k++) x[k] = a[P * ta + k];
-        fft_dit<N, N, 1, double2>(x, X, tw);
-        double2* __restrict__ o = planes + (((size_t)ci * np + p) * 3 + pl) * N2 + N * ta;
-#pragma unroll
-        for (int k = 0; k < N; k++) o[k] = X[k];
-    }
-}
-
-// Q = scale (sum_{p < nd} (part_p + Re Zo Im Zo) - part_nd part_{nd+1}), pairs in order
-template <int N>
-__global__ __launch_bounds__(256) void k_fsm_psum(const double* __restrict__ part, const double2* __restrict__ planes, double* __restrict__ Q,
-                                                 int nd, int ncell, double scale) {
-    constexpr int N2 = N * N, N3 = N2 * N;
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= ncell * N3) return;
-    const int ci = i / N3, q = i % N3;
-    const int x = q % N, y = (q / N) % N, z = q / N2;
-    const double* __restrict__ pp = part + (size_t)ci * (nd + 2) * N3 + q;
-    const double2* __restrict__ pl = planes + (size_t)ci * nd * 3 * N2;
-    double re = 0.0;
-#pragma unroll 4
-    for (int p = 0; p < nd; p++) {
-        const double2* __restrict__ a = pl + (size_t)p * 3 * N2;
-        const double2 c0 = a[y + N * z], c1 = a[N2 + x + N * z], c2 = a[2 * N2 + x + N * y];
-        const double gr = c0.x + c1.x + c2.x, gi = c0.y + c1.y + c2.y;
-        re += pp[(size_t)p * N3] + gr * gi;
-    }
-    re -= pp[(size_t)nd * N3] * pp[(size_t)(nd + 1) * N3];
-    Q[i] = scale * re;
-}
-
-template <int N> hipError_t fsm_run_packed(const FsmPlan& P, const double* f, long fcs, int k0, double scale, hipStream_t st) {
-    constexpr int NS = N / fsm_slab<N>(), TH = fsm_slab_threads<N>();
-    constexpr size_t lds = fsm_slab_lds<N>();
-    const int nd = P.M * (P.M - 1), np = nd + 2, cg = (P.ncell + 7) / 8;
-    double2* spec = (double2*)P.spec;
-    double2* planes = (double2*)P.planes;
-    double* part = (double*)P.part;
-    const double2* tw = (const double2*)P.tw;
-    hipLaunchKernelGGL(k_fsm_spec<N>, dim3(P.ncell * NS), dim3(TH), lds, st, f, fcs, k0, tw, spec);
-    hipLaunchKernelGGL(k_fsm_planes<N>, dim3(P.ncell * ((nd + kFsmPP - 1) / kFsmPP)), dim3(fsm_plane_threads<N>()), 0, st, spec,
-                       (const double2*)P.mo, tw, planes, nd);
-    hipLaunchKernelGGL(k_fsm_slab<N>, dim3(P.ncell * np * NS), dim3(TH), lds, st, spec, (const double2*)P.ms, tw, part, np, P.ncell, cg);
-    hipLaunchKernelGGL(k_fsm_psum<N>, dim3((P.ncell * N * N * N + 255) / 256), dim3(256), 0, st, part, planes, P.Q, nd, P.ncell, scale);
+template <int N> hipError_t launch_cube64(const FsmPlan& P, hipStream_t st) {
+    const int nd = P.M * (P.M - 1), na = 2 * nd + 2;
+    const unsigned blocks = unsigned(P.ncell * na * (N / fsm_slab<N>()));
+    hipLaunchKernelGGL(k_fsm_slab64<N>, dim3(blocks), dim3(fsm_slab_threads<N>()), fsm_slab_lds<N>(), st, (const double2*)P.spec,
+                       (const double*)P.phi, (const double*)P.psi, (const double*)P.phipsi, (const double2*)P.tw,
+                       (double2*)P.work, nd, P.ncell);
     return hipGetLastError();
 }
 
-template <int N> hipError_t cube_attr(bool f32) {
-    if (f32) return hipFuncSetAttribute((const void*)k_fsm_pair<N>, hipFuncAttributeMaxDynamicSharedMemorySize, fsm_pair_lds<N>());
-    const hipError_t e = hipFuncSetAttribute((const void*)k_fsm_spec<N>, hipFuncAttributeMaxDynamicSharedMemorySize, fsm_slab_lds<N>());
+template <int N> hipError_t cube_attr() {
+    hipError_t e = hipFuncSetAttribute((const void*)k_fsm_pair<N>, hipFuncAttributeMaxDynamicSharedMemorySize, fsm_pair_lds<N>());
     if (e != hipSuccess) return e;
-    return hipFuncSetAttribute((const void*)k_fsm_slab<N>, hipFuncAttributeMaxDynamicSharedMemorySize, fsm_slab_lds<N>());
-}
-
-// fn(std::integral_constant<int, N>) for the plan's side
-template <class F> hipError_t with_cube(int n, F&& fn) {
-    switch (n) {
-    case 8: return fn(std::integral_constant<int, 8>{});
-    case 12: return fn(std::integral_constant<int, 12>{});
-    case 16: return fn(std::integral_constant<int, 16>{});
-    case 18: return fn(std::integral_constant<int, 18>{});
-    case 24: return fn(std::integral_constant<int, 24>{});
-    default: return hipErrorInvalidValue;
-    }
+    return hipFuncSetAttribute((const void*)k_fsm_slab64<N>, hipFuncAttributeMaxDynamicSharedMemorySize, fsm_slab_lds<N>());
 }
 
 unsigned blocks_of(size_t n) { return unsigned((n + 255) / 256); }
@@ -474,12 +306,9 @@ hipfftResult exec(const FsmPlan& P, hipfftHandle_t* plan, void* data, int dir) {
 }
 
 template <class R> hipError_t fsm_run(const FsmPlan& P, bool fp64, const void* f, long fcs, int k0, hipStream_t st) {
-    const double scale = 4.0 * kPi * kPi / P.kn / (double(P.M) * P.M);
     const int n3 = P.nu * P.nv * P.nw, nd = P.M * (P.M - 1);
     const size_t cells = (size_t)P.ncell * n3;
     const dim3 g(blocks_of(cells)), b(256);
-    if (P.packed)
-        return with_cube(P.cube_n, [&](auto n) { return fsm_run_packed<decltype(n)::value>(P, (const double*)f, fcs, k0, scale, st); });
     cx_t<R>* spec = (cx_t<R>*)P.spec;
     cx_t<R>* work = (cx_t<R>*)P.work;
     if (fp64) hipLaunchKernelGGL((k_fsm_load<double, R>), g, b, 0, st, (const double*)f, fcs, k0, P.ncell, n3, spec);
@@ -488,64 +317,48 @@ template <class R> hipError_t fsm_run(const FsmPlan& P, bool fp64, const void* f
     if (e != hipSuccess) return e;
     if (hipfftSetStream(P.plan_b, st) != HIPFFT_SUCCESS) return hipErrorUnknown;
     if (exec(P, P.plan_b, spec, HIPFFT_BACKWARD) != HIPFFT_SUCCESS) return hipErrorUnknown;
-    if (P.cube_n) {  // FP32
-        e = with_cube(P.cube_n, [&](auto n) { return launch_pair<decltype(n)::value>(P, st); });
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(k_fsm_sum, g, b, 0, st, (const float*)P.part, P.Q, n3, nd, P.ncell, scale);
-        return hipGetLastError();
+    const double scale = 4.0 * kPi * kPi / P.kn / (double(P.M) * P.M);
+    if constexpr (sizeof(R) == 4) {
+        if (P.cube_n) {
+            switch (P.cube_n) {
+            case 8: e = launch_pair<8>(P, st); break;
+            case 12: e = launch_pair<12>(P, st); break;
+            case 16: e = launch_pair<16>(P, st); break;
+            case 18: e = launch_pair<18>(P, st); break;
+            default: e = launch_pair<24>(P, st); break;
+            }
+            if (e != hipSuccess) return e;
+            hipLaunchKernelGGL(k_fsm_sum, g, b, 0, st, P.part, P.Q, n3, nd, P.ncell, scale);
+            return hipGetLastError();
+        }
     }
-    if (hipfftSetStream(P.plan_f, st) != HIPFFT_SUCCESS) return hipErrorUnknown;
-    hipLaunchKernelGGL(k_fsm_modes<R>, g, b, 0, st, spec, work, (const R*)P.phi, (const R*)P.psi, (const R*)P.phipsi, P.nu,
-                       P.nv, P.nw, nd, P.ncell);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    if (exec(P, P.plan_f, work, HIPFFT_FORWARD) != HIPFFT_SUCCESS) return hipErrorUnknown;
+    if (P.cube_n) {
+        switch (P.cube_n) {
+        case 8: e = launch_cube64<8>(P, st); break;
+        case 12: e = launch_cube64<12>(P, st); break;
+        case 16: e = launch_cube64<16>(P, st); break;
+        case 18: e = launch_cube64<18>(P, st); break;
+        default: e = launch_cube64<24>(P, st); break;
+        }
+        if (e != hipSuccess) return e;
+    } else {
+        if (hipfftSetStream(P.plan_f, st) != HIPFFT_SUCCESS) return hipErrorUnknown;
+        hipLaunchKernelGGL(k_fsm_modes<R>, g, b, 0, st, spec, work, (const R*)P.phi, (const R*)P.psi, (const R*)P.phipsi, P.nu,
+                           P.nv, P.nw, nd, P.ncell);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+        if (exec(P, P.plan_f, work, HIPFFT_FORWARD) != HIPFFT_SUCCESS) return hipErrorUnknown;
+    }
     hipLaunchKernelGGL(k_fsm_q<R>, g, b, 0, st, work, P.Q, n3, nd, P.ncell, scale);
     return hipGetLastError();
 }
 
 }  // namespace
 
-int fsm_cube_size(int nu, int nv, int nw, bool f32, int nm, const double* phi, const double* psi, const double* phipsi) {
+int fsm_cube_size(int nu, int nv, int nw) {
     if (nu != nv || nu != nw) return 0;
     for (int n : {8, 12, 16, 18, 24})
-        if (n == nu) return f32 || !phi || !psi || !phipsi || fsm_pack_modes(n, nm, phi, psi, phipsi, nullptr, nullptr) ? n : 0;
+        if (n == nu) return n;
     return 0;
-}
-
-bool fsm_pack_modes(int N, int nm, const double* phi, const double* psi, const double* phipsi, double* ms, double* mo) {
-    const int nd = nm * (nm - 1), N2 = N * N, N3 = N2 * N;
-    if (ms)  // the loss: phipsi as it is, odd part included, and 1
-        for (int i = 0; i < N3; i++) {
-            ms[((size_t)nd * N3 + i) * 2] = phipsi[i];
-            ms[((size_t)(nd + 1) * N3 + i) * 2] = 1.0;
-            ms[((size_t)nd * N3 + i) * 2 + 1] = ms[((size_t)(nd + 1) * N3 + i) * 2 + 1] = 0.0;
-        }
-    for (int p = 0; p < nd; p++) {
-        const double* ab[2] = {phi + (size_t)p * N3, psi + (size_t)p * N3};
-        double mx[2] = {0.0, 0.0};
-        for (int h = 0; h < 2; h++)
-            for (int i = 0; i < N3; i++) mx[h] = std::max(mx[h], std::fabs(ab[h][i]));
-        if (!std::isfinite(mx[0]) || !std::isfinite(mx[1])) return false;
-        // a 2^e and b 2^-e of about the same size: the transforms share one complex array, whose rounding
-        // follows the larger of the two
-        const int e = mx[0] > 0.0 && mx[1] > 0.0 ? int(std::lround(0.5 * std::log2(mx[1] / mx[0]))) : 0;
-        for (int i = 0; i < N3; i++) {
-            const int x = i % N, y = (i / N) % N, z = i / N2;
-            const int j = (N - x) % N + N * ((N - y) % N) + N2 * ((N - z) % N);
-            for (int h = 0; h < 2; h++) {
-                const double a = ab[h][i], b = ab[h][j], odd = 0.5 * (a - b), sc = std::ldexp(1.0, h ? -e : e);
-                const bool plane = x == 0 || y == 0 || z == 0;
-                if (!(std::fabs(odd) <= (plane ? mx[h] : 1e-14 * mx[h]))) return false;  // a NaN, or not even (45 FP64 ulp)
-                if (!ms) continue;
-                ms[((size_t)p * N3 + i) * 2 + h] = 0.5 * (a + b) * sc;
-                if (!plane) continue;
-                // one plane per element: u = 0 first, then v = 0, then w = 0
-                const int pl = x == 0 ? 0 : (y == 0 ? 1 : 2), at = pl == 0 ? y + N * z : (pl == 1 ? x + N * z : x + N * y);
-                mo[(((size_t)p * 3 + pl) * N2 + at) * 2 + h] = odd * sc;
-            }
-        }
-    }
-    return true;
 }
 
 hipError_t fsm_collision(const FsmPlan& P, bool fp64, const void* f, long fcs, int k0, hipStream_t st) {
@@ -555,12 +368,19 @@ hipError_t fsm_collision(const FsmPlan& P, bool fp64, const void* f, long fcs, i
 
 hipError_t fsm_plan_create(FsmPlan& P) {
     const int n3 = P.nu * P.nv * P.nw, nd = P.M * (P.M - 1);
-    if (P.cube_n) {
-        const hipError_t e = with_cube(P.cube_n, [&](auto n) { return cube_attr<decltype(n)::value>(P.f32); });
-        if (e != hipSuccess || P.packed) return e;
-    }
     int n[3] = {P.nw, P.nv, P.nu};
     const hipfftType t = P.f32 ? HIPFFT_C2C : HIPFFT_Z2Z;
+    if (P.cube_n) {
+        hipError_t e;
+        switch (P.cube_n) {
+        case 8: e = cube_attr<8>(); break;
+        case 12: e = cube_attr<12>(); break;
+        case 16: e = cube_attr<16>(); break;
+        case 18: e = cube_attr<18>(); break;
+        default: e = cube_attr<24>(); break;
+        }
+        if (e != hipSuccess) return e;
+    }
     if (hipfftPlanMany(&P.plan_b, 3, n, nullptr, 1, n3, nullptr, 1, n3, t, P.ncell) != HIPFFT_SUCCESS) return hipErrorUnknown;
     if (!P.cube_n &&
         hipfftPlanMany(&P.plan_f, 3, n, nullptr, 1, n3, nullptr, 1, n3, t, P.ncell * (2 * nd + 2)) != HIPFFT_SUCCESS) {

@@ -232,22 +232,16 @@ struct FsmPlan {
     double kn = 0.0;
     bool f32 = false;           // transforms, spectra and modes in FP32 (FP32 storage), else FP64
     void* spec = nullptr;       // complex [ncell][n3]
-    void* work = nullptr;       // complex [ncell][2 M(M-1) + 2][n3] (hipFFT path)
-    void* phi = nullptr;        // real [M(M-1)][n3] (not packed; psi and phipsi too)
+    void* work = nullptr;       // complex [ncell][2 M(M-1) + 2][n3]
+    void* phi = nullptr;        // real [M(M-1)][n3]
     void* psi = nullptr;        // real [M(M-1)][n3]
     void* phipsi = nullptr;     // real [n3]
     double* Q = nullptr;        // [ncell][n3]
-    // cubic grids of side cube_n (fsm_cube_size, else 0) take the in-house transforms, with twiddles
-    // tw[cube_n] = exp(-2 pi i j / cube_n).  FP32: products part, [ncell][M(M-1) + 1][n3], from phi, psi,
-    // phipsi.  FP64 (packed): the pairs' even modes and the loss modes ms, complex [M(M-1) + 2][n3], the
-    // pairs' odd parts on the Nyquist planes mo, complex [M(M-1)][3][n2], the planes' transforms, complex
-    // [ncell][M(M-1)][3][n2], the products and the loss transforms part, [ncell][M(M-1) + 2][n3]
+    // cubic grids of side cube_n (fsm_cube_size, else 0) take the in-house forward transforms, with
+    // twiddles tw[cube_n] = exp(-2 pi i j / cube_n) in the plan's precision: FP32 in LDS per direction
+    // pair (products part [ncell][M(M-1) + 1][n3], no work), FP64 through work in three passes
     int cube_n = 0;
-    bool packed = false;
-    void* ms = nullptr;
-    void* mo = nullptr;
-    void* planes = nullptr;
-    void* part = nullptr;
+    float* part = nullptr;
     void* tw = nullptr;
     struct hipfftHandle_t* plan_b = nullptr;
     struct hipfftHandle_t* plan_f = nullptr;
@@ -256,13 +250,8 @@ struct FsmPlan {
 // Q of the plan's cells from the f buffer f (cell stride fcs, storage index of cell c0 = k0)
 hipError_t fsm_collision(const FsmPlan& P, bool fp64, const void* f, long fcs, int k0, hipStream_t st);
 hipError_t fsm_plan_create(FsmPlan& P);
-// side of the cubic velocity grids whose transforms are the library's own (8, 12, 16, 18, 24; in FP64 with
-// modes even in the frequency off the Nyquist planes, NULL modes counting as even), else 0
-int fsm_cube_size(int nu, int nv, int nw, bool f32, int nm, const double* phi, const double* psi, const double* phipsi);
-// the even parts of the mode pairs and the loss modes (phipsi, 1), ms [nm(nm-1) + 2][N^3], and the pairs' odd parts on
-// the planes, mo [nm(nm-1)][3][N^2] (zeroed by the caller), (a, b) interleaved; false when the modes are not even off the planes.
-// ms NULL: only the check
-bool fsm_pack_modes(int N, int nm, const double* phi, const double* psi, const double* phipsi, double* ms, double* mo);
+// side of the cubic velocity grids whose forward transforms are the library's own (8, 12, 16, 18, 24), else 0
+int fsm_cube_size(int nu, int nv, int nw);
 void fsm_plan_destroy(FsmPlan& P);
 hipError_t launch_resid1d(const Solve1D& S, const double* d_rcell, int nrows, int boundary_split, double* d_res,
                           hipStream_t st);

@@ -178,17 +178,3 @@ def test_fsm_refusals():
     assert rc == -4 and b"fast spectral" in lib.kbg_last_error()  # KBG_ERR_STATE
     dev.close()
     ctx.close()
-
-
-@pytest.mark.parametrize("n", [8, 12, 16])
-def test_fsm_modes_that_are_not_even(n):
-    """The FP64 cubes pack two modes into one transform, which needs modes even in the frequency; a
-    descriptor with other modes (phi of one direction changed at one interior frequency) takes the
-    general path.  Against the oracle at the bar of the FP64 tests above."""
-    ks, ctr, face, dt = fsm_case(n=n, nx=6)
-    homogeneous_bimodal(ks, ctr)
-    phi = ks.gas.fsm.phi.copy()
-    phi[1, n // 2 + 1, n // 2, n // 2 + 1] *= 1.5
-    ks.gas.fsm = kb.fsm.FsmKernel(ks.gas.fsm.Kn, ks.gas.fsm.nm, phi, ks.gas.fsm.psi, ks.gas.fsm.phipsi)
-    cg, co = run_both(ks, ctr, face, dt, 1, "fp64")
-    assert rel_l2(cg.f[1:-1] - ctr.f[1:-1], co.f[1:-1] - ctr.f[1:-1]) <= 1e-10
