@@ -975,7 +975,7 @@ size_t kbg_solve_bytes(const kbg_desc* d) {
             // hipFFT's own work area not counted
             const size_t nc = size_t(d->nx) - 2, n3 = size_t(d->nv), nd = size_t(d->fsm_nm) * (d->fsm_nm - 1);
             const int cn = kbg::fsm_cube_size(d->fsm_shape[0], d->fsm_shape[1], d->fsm_shape[2]);
-            const size_t work = (cn && esz == 4 ? nc * (nd + 1) * n3 * 4 : nc * (2 * nd + 2) * n3 * 2 * esz) + size_t(cn) * 2 * esz;
+            const size_t work = nc * (nd + 1) * n3 * (cn ? esz : 4 * esz) + size_t(cn) * 2 * esz;
             fsm = nc * n3 * 2 * esz + work + (2 * nd + 1) * n3 * esz + nc * n3 * 8;
         }
         size_t w3 = 0;
@@ -1141,16 +1141,15 @@ int kbg_solve_create(kbg_ctx* ctx, const kbg_desc* desc, kbg_solve** out) {
             P.cube_n = kbg::fsm_cube_size(P.nu, P.nv, P.nw);
             const size_t n3 = size_t(d.nv), nd = size_t(P.M) * (P.M - 1), nc = size_t(P.ncell), re = P.f32 ? 4 : 8;
             if (S.fvs != 1) return bail(fail(KBG_ERR_STATE, ":fsm needs the velocity-contiguous f layout"));
-            // the FP32 LDS path keeps one FP32 product per pair instead of the transformed mode products
-            const bool lds = P.cube_n && P.f32;
-            const size_t work = lds ? 0 : nc * (2 * nd + 2) * n3 * 2 * re;
-            const size_t part = lds ? nc * (nd + 1) * n3 * 4 : 0, twb = size_t(P.cube_n) * 2 * re;
+            // cubes keep one real product per pair instead of the transformed mode products
+            const size_t work = P.cube_n ? 0 : nc * (2 * nd + 2) * n3 * 2 * re;
+            const size_t part = P.cube_n ? nc * (nd + 1) * n3 * re : 0, twb = size_t(P.cube_n) * 2 * re;
             struct {
                 void** dst;
                 size_t bytes;
             } bufs[] = {{&P.spec, nc * n3 * 2 * re}, {&P.work, work},       {&P.phi, nd * n3 * re},
                         {&P.psi, nd * n3 * re},      {&P.phipsi, n3 * re},  {(void**)&P.Q, nc * n3 * 8},
-                        {(void**)&P.part, part},     {&P.tw, twb}};
+                        {&P.part, part},             {&P.tw, twb}};
             for (auto& b : bufs) {
                 if (!b.bytes) continue;
                 if ((rc = dev_alloc(s, &p, b.bytes))) return bail(rc);

@@ -12,8 +12,8 @@
 // The transforms, the spectra and the kernel modes are FP64 for FP64 storage and FP32 for FP32
 // storage (R below).  hipFFT's forward pass streams the 2 M(M-1) + 2 product arrays per cell through
 // HBM about a dozen times; on cubic grids of side 8, 12, 16, 18 or 24 the forward transforms are the
-// library's own pencil transforms instead (kbg_fft.h): FP32 entirely in LDS (k_fsm_pair), FP64
-// written once and read once (k_fsm_slab64, k_fsm_q).  Q is FP64 in all of them.  The kernel modes phi,
+// library's own pencil transforms instead (kbg_fft.h), whole arrays in LDS in FP32 (k_fsm_pair), slabs
+// of them in FP64 (k_fsm_slab64); each writes one real product per pair, which k_fsm_sum adds.  Q is FP64 in all of them.  The kernel modes phi,
 // psi, phipsi (kernel_mode, theory_fsm.jl:24-90) come from the host with the descriptor.  Arrays are
 // [w][v][u] with u fastest (KitBase's column-major f[i, j, k]).  The update kernel then adds dt Q to
 // the transport update (k_update1d).
@@ -193,40 +193,58 @@ __global__ __launch_bounds__(fsm_pair_threads<N>()) void k_fsm_pair(const float2
     }
 }
 
-// ---- FP64 storage on a cubic grid: the transforms of the products f_spec phi_d, f_spec psi_d,
-// f_spec phipsi, f_spec in the layout of k_fsm_modes (work[cell][2 M(M-1) + 2][n3]), each written
-// once by k_fsm_slab64, then k_fsm_q.  One workgroup per slab of S w-planes of one product array:
+// ---- FP64 storage on a cubic grid: the same products per pair, in slabs (a 24^3 array of 16 bytes does
+// not fit a CU's LDS).  One workgroup per (cell, pair, slab of S w-frequencies); each of the pair's two
+// transforms:
 //   1. every w-pencil (u, v) of the array: f_spec times the mode straight from the backward
 //      transform's output (the fftshift is an index map), transformed along w in registers; the S
 //      frequencies of the slab go to LDS (rows padded to an odd length).  The N / S slabs of an array
-//      each redo these transforms: arithmetic from L2-resident inputs instead of a pass over HBM;
+//      each redo these transforms: arithmetic from L2-resident inputs instead of a pass over HBM.  A
+//      slab's frequencies are those whose butterflies share the most (fsm_slab_class), and the code of
+//      each class is its own, so the compiler drops the butterflies of the others;
 //   2. one thread per u-pencil of the slab, in LDS;
-//   3. one thread per v-pencil, whose transform goes straight to the array.
+//   3. one thread per v-pencil; the first transform's pencil stays in registers until the second's
+//      meets it, and the product is stored.
+// Bound by VALU and L2 latency at two
+// workgroups per CU (77 KB of LDS).  48 cells x 21 pairs
+// of 24^3: 147 us + 21 us of k_fsm_sum; with both transforms of every pair written (446 MB), whole
+// w-transforms and the sum of products in a kernel of its own, 167 + 109 us.
 template <int N> constexpr int fsm_slab() { return N % 8 == 0 ? 8 : 6; }
 template <int N> constexpr int fsm_slab_threads() { return (fsm_slab<N>() * N + 63) / 64 * 64; }
 template <int N> constexpr int fsm_slab_lds() { return fsm_slab<N>() * N * (N | 1) * 16; }
+// slab of frequency k: with N = R M (fft_radix), the last radix-R stage joins the frequencies k % M; slabs are
+// whole such sets where M allows it, every other output k / M of the last stage for N = 12 (M = 3, two slabs)
+template <int N> constexpr int fsm_slab_class(int k) {
+    constexpr int M = N / fft_radix(N), NS = N / fsm_slab<N>();
+    return M % NS == 0 ? k % M / (M / NS) : k / M % NS;
+}
+template <int N> constexpr int fsm_slab_index(int k) {  // position of k among its slab's frequencies
+    int j = 0;
+    for (int i = 0; i < k; i++) j += fsm_slab_class<N>(i) == fsm_slab_class<N>(k);
+    return j;
+}
+template <int N> constexpr int fsm_slab_freq(int sl, int j) {  // the j-th frequency of slab sl
+    constexpr int M = N / fft_radix(N), NS = N / fsm_slab<N>(), C = M / NS;
+    if constexpr (M % NS == 0) return sl * C + j % C + j / C * M;
+    else return (sl + j / M * NS) * M + j % M;
+}
+template <int N> constexpr bool fsm_slab_maps() {
+    for (int k = 0; k < N; k++)
+        if (fsm_slab_freq<N>(fsm_slab_class<N>(k), fsm_slab_index<N>(k)) != k || fsm_slab_index<N>(k) >= fsm_slab<N>()) return false;
+    return true;
+}
+static_assert(fsm_slab_maps<8>() && fsm_slab_maps<12>() && fsm_slab_maps<16>() && fsm_slab_maps<18>() && fsm_slab_maps<24>());
 
-template <int N>
-__global__ __launch_bounds__(fsm_slab_threads<N>()) void k_fsm_slab64(const double2* __restrict__ spec, const double* __restrict__ phi,
-                                                                    const double* __restrict__ psi, const double* __restrict__ phipsi,
-                                                                    const double2* __restrict__ tw, double2* __restrict__ work, int nd,
-                                                                    int ncell) {
-    constexpr int N2 = N * N, N3 = N2 * N, P = N | 1, H = N / 2, S = fsm_slab<N>(), NS = N / S;
-    constexpr int NTH = fsm_slab_threads<N>();
-    extern __shared__ double2 slab[];
-    const int na = 2 * nd + 2;
-    const int item = fsm_xcd_item();
-    if (item >= ncell * na * NS) return;
-    const int sl = item % NS, a = (item / NS) % na, ci = item / (NS * na);
-    const int p = a >> 1, h = a & 1;
-    const double* __restrict__ mode = p < nd ? (h ? psi : phi) + (size_t)p * N3 : (h ? nullptr : phipsi);
-    const double inv = 1.0 / double(N3);
-    const int t = threadIdx.x;
+// 1. of slab SL: every w-pencil of the array, the slab's frequencies to LDS
+template <int N, int SL>
+KBG_D void fsm_slab_w(const double2* __restrict__ spec, const double* __restrict__ mode, const double2* __restrict__ tw, double2* slab,
+                      int t) {
+    constexpr int N2 = N * N, P = N | 1, H = N / 2, NTH = fsm_slab_threads<N>();
+    const double inv = 1.0 / double(N2 * N);
     double2 x[N], X[N];
-    // 1. along w, every pencil of the array; the slab's planes kept
     for (int pen = t; pen < N2; pen += NTH) {
         const int ta = pen % N, tb = pen / N;
-        const double2* __restrict__ col = spec + (size_t)ci * N3 + (ta + N - H) % N + N * ((tb + N - H) % N);
+        const double2* __restrict__ col = spec + (ta + N - H) % N + N * ((tb + N - H) % N);
 #pragma unroll
         for (int k = 0; k < N; k++) {
             const double2 z = col[N2 * ((k + N - H) % N)];
@@ -235,39 +253,70 @@ __global__ __launch_bounds__(fsm_slab_threads<N>()) void k_fsm_slab64(const doub
         }
         fft_dit<N, N, 1, double2>(x, X, tw);
 #pragma unroll
-        for (int k = 0; k < N; k++)  // compile-time register indices, a uniform branch per plane
-            if (k / S == sl) slab[ta + P * (tb + N * (k % S))] = X[k];
+        for (int k = 0; k < N; k++)
+            if (fsm_slab_class<N>(k) == SL) slab[ta + P * (tb + N * fsm_slab_index<N>(k))] = X[k];
     }
-    __syncthreads();
+}
+
+template <int N>
+__global__ __launch_bounds__(fsm_slab_threads<N>(), 2) void k_fsm_slab64(const double2* __restrict__ spec, const double* __restrict__ phi,
+                                                                       const double* __restrict__ psi,
+                                                                       const double* __restrict__ phipsi,
+                                                                       const double2* __restrict__ tw, double* __restrict__ part, int nd,
+                                                                       int ncell) {
+    constexpr int N2 = N * N, N3 = N2 * N, P = N | 1, S = fsm_slab<N>(), NS = N / S;
+    extern __shared__ double2 slab[];
+    const int np = nd + 1;
+    const int item = fsm_xcd_item();
+    if (item >= ncell * np * NS) return;
+    const int sl = item % NS, p = (item / NS) % np, ci = item / (NS * np);
+    const int t = threadIdx.x;
     const bool act = t < S * N;
     const int ta = t % N, tb = t / N;
-    if (act) {  // 2. along u: pencil (v, w) = (ta, tb)
-        double2* r = slab + P * (ta + N * tb);
+    const double2* __restrict__ sc = spec + (size_t)ci * N3;
+    double2 x[N], X[N], A[N];
+#pragma unroll 1
+    for (int h = 0; h < 2; h++) {
+        const double* __restrict__ mode = p < nd ? (h ? psi : phi) + (size_t)p * N3 : (h ? nullptr : phipsi);
+        if (h) __syncthreads();  // the first transform's v-pencils have been read
+        if (NS == 1 || sl == 0) fsm_slab_w<N, 0>(sc, mode, tw, slab, t);
+        else if (NS == 2 || sl == 1) fsm_slab_w<N, 1>(sc, mode, tw, slab, t);
+        else fsm_slab_w<N, 2>(sc, mode, tw, slab, t);
+        __syncthreads();
+        if (act) {  // 2. along u: pencil (v, w) = (ta, tb)
+            double2* r = slab + P * (ta + N * tb);
 #pragma unroll
-        for (int k = 0; k < N; k++) x[k] = r[k];
-        fft_dit<N, N, 1, double2>(x, X, tw);
+            for (int k = 0; k < N; k++) x[k] = r[k];
+            fft_dit<N, N, 1, double2>(x, X, tw);
 #pragma unroll
-        for (int k = 0; k < N; k++) r[k] = X[k];
-    }
-    __syncthreads();
-    if (act) {  // 3. along v: pencil (u, w) = (ta, tb), to the array
-        const double2* r = slab + ta + P * N * tb;
+            for (int k = 0; k < N; k++) r[k] = X[k];
+        }
+        __syncthreads();
+        if (act) {  // 3. along v: pencil (u, w) = (ta, tb)
+            const double2* r = slab + ta + P * N * tb;
 #pragma unroll
-        for (int k = 0; k < N; k++) x[k] = r[P * k];
-        fft_dit<N, N, 1, double2>(x, X, tw);
-        double2* __restrict__ o = work + ((size_t)ci * na + a) * N3 + ta + N2 * (sl * S + tb);
+            for (int k = 0; k < N; k++) x[k] = r[P * k];
+            fft_dit<N, N, 1, double2>(x, X, tw);
+            if (h == 0) {
 #pragma unroll
-        for (int k = 0; k < N; k++) o[N * k] = X[k];
+                for (int k = 0; k < N; k++) A[k] = X[k];
+            } else {
+                double* __restrict__ o = part + ((size_t)ci * np + p) * N3 + ta + N2 * fsm_slab_freq<N>(sl, tb);
+#pragma unroll
+                for (int k = 0; k < N; k++) o[N * k] = A[k].x * X[k].x - A[k].y * X[k].y;
+            }
+        }
     }
 }
 
 // Q = scale (sum_{p < nd} part_p - part_nd), pairs in order
-__global__ __launch_bounds__(256) void k_fsm_sum(const float* __restrict__ part, double* __restrict__ Q, int n3, int nd,
+template <class R>
+__global__ __launch_bounds__(256) void k_fsm_sum(const R* __restrict__ part, double* __restrict__ Q, int n3, int nd,
                                                  int ncell, double scale) {
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= (size_t)ncell * n3) return;
     const int ci = int(i / n3), q = int(i % n3);
-    const float* __restrict__ pp = part + (size_t)ci * (nd + 1) * n3 + q;
+    const R* __restrict__ pp = part + (size_t)ci * (nd + 1) * n3 + q;
     double re = 0.0;
 #pragma unroll 10  // ten loads in flight per thread: 10.9 us for the 56 MB of 48 cells of 24^3, 15.7 without
     for (int d = 0; d < nd; d++) re += double(pp[(size_t)d * n3]);
@@ -279,17 +328,21 @@ template <int N> hipError_t launch_pair(const FsmPlan& P, hipStream_t st) {
     const int nd = P.M * (P.M - 1);
     hipLaunchKernelGGL(k_fsm_pair<N>, dim3(P.ncell * (nd + 1)), dim3(fsm_pair_threads<N>()), fsm_pair_lds<N>(), st,
                        (const float2*)P.spec, (const float*)P.phi, (const float*)P.psi, (const float*)P.phipsi,
-                       (const float2*)P.tw, P.part, nd, P.ncell);
+                       (const float2*)P.tw, (float*)P.part, nd, P.ncell);
     return hipGetLastError();
 }
 
-template <int N> hipError_t launch_cube64(const FsmPlan& P, hipStream_t st) {
-    const int nd = P.M * (P.M - 1), na = 2 * nd + 2;
-    const unsigned blocks = unsigned(P.ncell * na * (N / fsm_slab<N>()));
-    hipLaunchKernelGGL(k_fsm_slab64<N>, dim3(blocks), dim3(fsm_slab_threads<N>()), fsm_slab_lds<N>(), st, (const double2*)P.spec,
-                       (const double*)P.phi, (const double*)P.psi, (const double*)P.phipsi, (const double2*)P.tw,
-                       (double2*)P.work, nd, P.ncell);
+template <int N> hipError_t launch_slab64(const FsmPlan& P, hipStream_t st) {
+    const int nd = P.M * (P.M - 1);
+    hipLaunchKernelGGL(k_fsm_slab64<N>, dim3(P.ncell * (nd + 1) * (N / fsm_slab<N>())), dim3(fsm_slab_threads<N>()), fsm_slab_lds<N>(),
+                       st, (const double2*)P.spec, (const double*)P.phi, (const double*)P.psi, (const double*)P.phipsi,
+                       (const double2*)P.tw, (double*)P.part, nd, P.ncell);
     return hipGetLastError();
+}
+
+template <int N, class R> hipError_t launch_cube(const FsmPlan& P, hipStream_t st) {
+    if constexpr (sizeof(R) == 4) return launch_pair<N>(P, st);
+    else return launch_slab64<N>(P, st);
 }
 
 template <int N> hipError_t cube_attr() {
@@ -318,36 +371,23 @@ template <class R> hipError_t fsm_run(const FsmPlan& P, bool fp64, const void* f
     if (hipfftSetStream(P.plan_b, st) != HIPFFT_SUCCESS) return hipErrorUnknown;
     if (exec(P, P.plan_b, spec, HIPFFT_BACKWARD) != HIPFFT_SUCCESS) return hipErrorUnknown;
     const double scale = 4.0 * kPi * kPi / P.kn / (double(P.M) * P.M);
-    if constexpr (sizeof(R) == 4) {
-        if (P.cube_n) {
-            switch (P.cube_n) {
-            case 8: e = launch_pair<8>(P, st); break;
-            case 12: e = launch_pair<12>(P, st); break;
-            case 16: e = launch_pair<16>(P, st); break;
-            case 18: e = launch_pair<18>(P, st); break;
-            default: e = launch_pair<24>(P, st); break;
-            }
-            if (e != hipSuccess) return e;
-            hipLaunchKernelGGL(k_fsm_sum, g, b, 0, st, P.part, P.Q, n3, nd, P.ncell, scale);
-            return hipGetLastError();
-        }
-    }
     if (P.cube_n) {
         switch (P.cube_n) {
-        case 8: e = launch_cube64<8>(P, st); break;
-        case 12: e = launch_cube64<12>(P, st); break;
-        case 16: e = launch_cube64<16>(P, st); break;
-        case 18: e = launch_cube64<18>(P, st); break;
-        default: e = launch_cube64<24>(P, st); break;
+        case 8: e = launch_cube<8, R>(P, st); break;
+        case 12: e = launch_cube<12, R>(P, st); break;
+        case 16: e = launch_cube<16, R>(P, st); break;
+        case 18: e = launch_cube<18, R>(P, st); break;
+        default: e = launch_cube<24, R>(P, st); break;
         }
         if (e != hipSuccess) return e;
-    } else {
-        if (hipfftSetStream(P.plan_f, st) != HIPFFT_SUCCESS) return hipErrorUnknown;
-        hipLaunchKernelGGL(k_fsm_modes<R>, g, b, 0, st, spec, work, (const R*)P.phi, (const R*)P.psi, (const R*)P.phipsi, P.nu,
-                           P.nv, P.nw, nd, P.ncell);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
-        if (exec(P, P.plan_f, work, HIPFFT_FORWARD) != HIPFFT_SUCCESS) return hipErrorUnknown;
+        hipLaunchKernelGGL(k_fsm_sum<R>, g, b, 0, st, (const R*)P.part, P.Q, n3, nd, P.ncell, scale);
+        return hipGetLastError();
     }
+    if (hipfftSetStream(P.plan_f, st) != HIPFFT_SUCCESS) return hipErrorUnknown;
+    hipLaunchKernelGGL(k_fsm_modes<R>, g, b, 0, st, spec, work, (const R*)P.phi, (const R*)P.psi, (const R*)P.phipsi, P.nu,
+                       P.nv, P.nw, nd, P.ncell);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    if (exec(P, P.plan_f, work, HIPFFT_FORWARD) != HIPFFT_SUCCESS) return hipErrorUnknown;
     hipLaunchKernelGGL(k_fsm_q<R>, g, b, 0, st, work, P.Q, n3, nd, P.ncell, scale);
     return hipGetLastError();
 }

@@ -232,16 +232,16 @@ struct FsmPlan {
     double kn = 0.0;
     bool f32 = false;           // transforms, spectra and modes in FP32 (FP32 storage), else FP64
     void* spec = nullptr;       // complex [ncell][n3]
-    void* work = nullptr;       // complex [ncell][2 M(M-1) + 2][n3]
+    void* work = nullptr;       // complex [ncell][2 M(M-1) + 2][n3] (no cube)
     void* phi = nullptr;        // real [M(M-1)][n3]
     void* psi = nullptr;        // real [M(M-1)][n3]
     void* phipsi = nullptr;     // real [n3]
     double* Q = nullptr;        // [ncell][n3]
     // cubic grids of side cube_n (fsm_cube_size, else 0) take the in-house forward transforms, with
-    // twiddles tw[cube_n] = exp(-2 pi i j / cube_n) in the plan's precision: FP32 in LDS per direction
-    // pair (products part [ncell][M(M-1) + 1][n3], no work), FP64 through work in three passes
+    // twiddles tw[cube_n] = exp(-2 pi i j / cube_n) and one product per direction pair, part
+    // [ncell][M(M-1) + 1][n3], both in the plan's precision
     int cube_n = 0;
-    float* part = nullptr;
+    void* part = nullptr;
     void* tw = nullptr;
     struct hipfftHandle_t* plan_b = nullptr;
     struct hipfftHandle_t* plan_f = nullptr;
