@@ -623,28 +623,23 @@ bool tiled2d(const kbg_desc& d) {
     return true;
 }
 
-// buffers of the tiled step; a solve they do not fit beside (S.g stays NULL) is stepped by the other kernels
+// buffers of the tiled step
 int alloc_tiled2d(kbg_solve* s) {
     const kbg_desc& d = s->d;
     Solve2D& S = s->h2;
     const size_t C = s->N, FX = size_t(d.nx + 1) * d.ny, FY = size_t(d.nx) * (d.ny + 1), nch = (size_t(d.nv) + 255) / 256;
-    void *rds, *perm, *g;
+    void *rds, *perm;
     struct {
         void** dst;
         size_t bytes;
     } tb[] = {{&S.xrec, FX * kbg::kFaceT * s->esz}, {&S.yrec, FY * kbg::kFaceT * s->esz}, {(void**)&S.xfrec, FX * 64},
               {(void**)&S.yfrec, FY * 64},         {(void**)&S.psum, nch * (FX + FY) * 32}, {&S.crec, C * kbg::kCellT * s->esz},
-              {&rds, C * s->esz},                  {&perm, size_t(d.nv) * 4},              {&g, C * 2 * d.nv * s->esz}};
-    const size_t kept = s->allocs.size();
-    for (auto& b : tb) {
-        if (dev_alloc(s, b.dst, b.bytes) == KBG_OK) continue;
-        (void)hipGetLastError();
-        for (size_t k = kept; k < s->allocs.size(); k++) (void)hipFree(s->allocs[k]);
-        s->allocs.resize(kept);
-        return KBG_OK;
-    }
-    for (auto& b : tb) HIPCHK(hipMemset(*b.dst, 0, b.bytes));
+              {&rds, C * s->esz},                  {&perm, size_t(d.nv) * 4}};
     int rc;
+    for (auto& b : tb) {
+        if ((rc = dev_alloc(s, b.dst, b.bytes))) return rc;
+        HIPCHK(hipMemset(*b.dst, 0, b.bytes));
+    }
     std::vector<double> r(C);
     for (size_t c = 0; c < C; c++) r[c] = 1.0 / (d.dx[c] * d.dy[c]);
     if ((rc = put_real(s, rds, r.data(), C, !s->fp64))) return rc;
@@ -655,7 +650,6 @@ int alloc_tiled2d(kbg_solve* s) {
     HIPCHK(hipMemcpy(perm, order.data(), size_t(d.nv) * 4, hipMemcpyHostToDevice));
     S.rds = rds;
     S.vperm = static_cast<const int*>(perm);
-    S.g = g;
     return KBG_OK;
 }
 
@@ -1004,8 +998,8 @@ size_t kbg_solve_bytes(const kbg_desc* d) {
     if (d->flux != KBG_KFVS) b += F * kbg::kFaceCoef * 8 + (esz == 4 ? F * kbg::kFaceC32 * 4 : 0);
     if (kbg::step2d_threads(d->precision == KBG_FP64, d->nv) == 0) b += C * 8 * 8 + C * 4 * nv * esz;  // slopes
     else if (esz == 4) b += 2 * nv * 4 + F * 8;  // departure form: reference Maxwellian, per-face coefficients
-    if (tiled2d(*d))  // G, face records, moment sums
-        b += C * (2 * nv + 1 + kbg::kCellT) * esz + F * (kbg::kFaceT * esz + 64 + (nv + 255) / 256 * 32) + nv * 4;
+    if (tiled2d(*d))  // face and cell records, moment sums
+        b += C * (1 + kbg::kCellT) * esz + F * (kbg::kFaceT * esz + 64 + (nv + 255) / 256 * 32) + nv * 4;
     return b;
 }
 
@@ -1890,7 +1884,7 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
     {
         std::map<std::tuple<int, int, int, int>, std::vector<int>> groups;
         for (int i : fused2)
-            groups[{solves[i]->fp64 ? 1 : 0, solves[i]->d.flux, solves[i]->h2.g ? 0 : solves[i]->thr2, solves[i]->h2.g ? 1 : 0}].push_back(i);
+            groups[{solves[i]->fp64 ? 1 : 0, solves[i]->d.flux, solves[i]->h2.xrec ? 0 : solves[i]->thr2, solves[i]->h2.xrec ? 1 : 0}].push_back(i);
         for (auto& kv : groups) {
             Launch2 L{std::get<0>(kv.first) == 1, std::get<1>(kv.first), std::get<2>(kv.first), (int)kv.second.size(), 0, 0, 0,
                       descs2.size(), 0, 0, 0, 0.0, 0, {0, 0, 0, 0}};
@@ -2262,9 +2256,8 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
             const Solve2D* dd = d_descs2 + L.desc0;
             hipStream_t ss = sst[stream2[g]];
             if (L.ty) {
-                const int w = last || capturing ? 1 : 0;
                 HIPCHK(kbg::launch_tile2d(L.fp64, L.flux, L.ty, dd, d_pref2 + L.fpref0, L.n, L.totals, (last && residuals) ? 1 : 0,
-                                          first || capturing ? 1 : 0, w, w, ss));
+                                          first || capturing ? 1 : 0, last || capturing ? 1 : 0, ss));
                 continue;
             }
             HIPCHK(kbg::launch_face2d(true, L.flux, dd, d_pref2 + L.ipref0, L.n, L.ninterior, ss));

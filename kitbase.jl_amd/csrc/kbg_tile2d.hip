@@ -6,9 +6,10 @@
 //
 //   k_tile2d   one thread per velocity, a workgroup of 256 over a tile of kTX cells along x and up to
 //              kTile2dRows rows, marching up the rows: every distribution value is loaded once per tile, each
-//              cell's slopes are formed once, and the transport update G = f + sum of face fluxes / ds goes
-//              to the second buffer, so the interior face fluxes never go to memory (they do in the
-//              last step of a call, which leaves them where evolve! does).  The tile's face records sit in
+//              cell's slopes are formed once, and the interior face fluxes never go to memory: their
+//              places in the flux arrays hold the transport update G = f + sum of face fluxes / ds (g_face).
+//              The last step of a call leaves the fluxes there instead, as evolve! does, and k_relax2d
+//              forms G from f and them, with the same operations.  The tile's face records sit in
 //              LDS: as scalar loads their waits and the spills of scalar registers took a third of the
 //              kernel.  Faces between tiles are evaluated by both, with the same operations; the tile to
 //              their right (above) adds up their moments: over 8 lanes in the storage type, then in FP64.
@@ -303,6 +304,11 @@ KBG_D int cell_at(int nx, int ny, int k) {
 }
 KBG_HD int interior_faces(int nx, int ny) { return (nx - 1) * ny + nx * (ny - 1); }
 
+// The interior face whose place in the flux arrays holds G of cell (i, j) (from 0): the x-face to its left, in
+// the first column the y-face below it, and for the first cell the y-face below cell (1, 1), which no other
+// cell takes.
+KBG_D int g_face(int nx, int i, int j) { return i > 0 ? i + (nx + 1) * j : j > 0 ? nx * j : nx + 1; }
+
 }  // namespace
 
 // A call's first step: walls and interface chains.  pstart: prefix sums of ceil(interior faces / 256) + cells
@@ -461,7 +467,6 @@ KBG_D void tile_march(const Solve2D& S, int i0, int j0, int j1, int iv, bool liv
     const TL W{make_rsrc(S.f, unsigned(long(nx) * ny * RSE)), iv * E, ohb, RSE, {xx, xy}, yy, {xx * xx + yx * yx, xy * xy + yy * yy}, wq,
                T(0.5) * wq, yx, u >= T(0), v >= T(0)};
     const int voff = iv * E, vst = live ? voff : 0x7fffffff;  // stores of lanes past nv fall outside the buffers
-    const rsrc_t gout = make_rsrc(S.g, unsigned(long(nx) * ny * RSE));
     const rsrc_t xff = make_rsrc(S.xff, unsigned(long(nx + 1) * ny * RSE)), yff = make_rsrc(S.yff, unsigned(long(nx) * (ny + 1) * RSE));
     auto ldf = [&](rsrc_t r, int f) __attribute__((always_inline)) {
         return H2{bload((T*)0, r, voff, f * RSE), bload((T*)0, r, voff, f * RSE + ohb)};
@@ -569,7 +574,11 @@ KBG_D void tile_march(const Solve2D& S, int i0, int j0, int j1, int iv, bool liv
         }
         static_for<kTX>([&](auto t) {
             const T r = RD[row * kTX + t];
-            stf(gout, cj + t, H2{fB[t].x + D[t].x * r, fB[t].y + D[t].y * r});
+            if constexpr (!KEEP) {
+                const H2 g{fB[t].x + D[t].x * r, fB[t].y + D[t].y * r};
+                if (t == 0 && !inL) stf(yff, g_face(nx, 0, j), g);
+                else stf(xff, g_face(nx, i0 + t, j), g);
+            }
             fB[t] = fC[t];
             fC[t] = fN[t];
         });
@@ -749,9 +758,10 @@ __global__ __launch_bounds__(256) void k_chain2d(const Solve2D* __restrict__ sol
 }
 
 // update!'s relaxation f = (G + (dt / tau) M) / (1 + dt / tau): a workgroup per cell and 1024 velocities (next
-// to a wall: per cell).  next: workgroups before them form the next step's interface chains, and those next
-// to a wall its wall fluxes.  Bound by memory: 604 MB in 124 us at 16384 cells x 48^2 velocities in FP32.
-template <class T, int FLUX, bool NEXT>
+// to a wall: per cell).  NEXT: workgroups before them form the next step's interface chains, and those next
+// to a wall its wall fluxes.  KEEP: the flux arrays hold the face fluxes, from which G is formed here.  Bound by
+// memory: 604 MB in 124 us at 16384 cells x 48^2 velocities in FP32.
+template <class T, int FLUX, bool NEXT, bool KEEP>
 __global__ __launch_bounds__(256, NEXT ? 4 : 6) void k_relax2d(const Solve2D* __restrict__ solves, const int* __restrict__ rstart, int nsolves) {
     constexpr int VPT = 4;
     __shared__ double red[NEXT ? 36 : 1];
@@ -772,8 +782,21 @@ __global__ __launch_bounds__(256, NEXT ? 4 : 6) void k_relax2d(const Solve2D* __
     const bool wall = b < nw;
     const int c = cell_at(nx, ny, wall ? b : nw + (b - nw) / per);
     const bool del = sizeof(T) == 4 && S.delta;
-    const T* __restrict__ G = (const T*)S.g + (size_t)c * 2 * nv;
+    const int i = c % nx, j = c / nx;
+    const T* __restrict__ G = (const T*)(i > 0 ? S.xff : S.yff) + (size_t)g_face(nx, i, j) * 2 * nv;
+    const T* __restrict__ xl = (const T*)S.xff + (size_t)(i + (nx + 1) * j) * 2 * nv;
+    const T* __restrict__ yd = (const T*)S.yff + (size_t)(i + nx * j) * 2 * nv;
+    const T rds = KEEP ? ((const T*)S.rds)[c] : T(0);
     T* h = (T*)S.f + (size_t)c * 2 * nv;
+    auto g_of = [&](int o) {
+        if constexpr (KEEP) {
+            T d = xl[o] - xl[2 * nv + o];
+            d += yd[o] - yd[size_t(nx) * 2 * nv + o];
+            return h[o] + d * rds;
+        } else {
+            return G[o];
+        }
+    };
     const T* __restrict__ U = (const T*)S.u;
     const T* __restrict__ V = (const T*)S.v;
     const float* __restrict__ R = S.mref;
@@ -783,8 +806,8 @@ __global__ __launch_bounds__(256, NEXT ? 4 : 6) void k_relax2d(const Solve2D* __
 #pragma unroll
         for (int k = 0; k < VPT; k++) {
             const int iv = min(v0 + tid + 256 * k, nv - 1);
-            gh[k] = G[iv];
-            gb[k] = G[nv + iv];
+            gh[k] = g_of(iv);
+            gb[k] = g_of(nv + iv);
             u[k] = U[iv];
             v[k] = V[iv];
             if constexpr (sizeof(T) == 4) {
@@ -827,7 +850,7 @@ int tile2d_rows(bool fp64, long one_row) {
 }
 
 template <class T, int FLUX>
-static hipError_t launch_tile_t(int ty, const Solve2D* d_solves, const int* d_pref, int n, const int* totals, int rows, int first, int last, int keep,
+static hipError_t launch_tile_t(int ty, const Solve2D* d_solves, const int* d_pref, int n, const int* totals, int rows, int first, int last,
                                 hipStream_t st) {
     // k_relax2d with the next step's walls and chains holds 4 wavefronts per SIMD, alone 8: sharing the launch
     // pays while the launch is short (us per step, shared / not: 64 x 64 x 32^2 FP32 60 / 66, FP64 95 / 105, 100 x
@@ -835,18 +858,21 @@ static hipError_t launch_tile_t(int ty, const Solve2D* d_solves, const int* d_pr
     const bool share = totals[3] <= 32768;
     if (first || !share) hipLaunchKernelGGL((k_pre2d<T, FLUX>), dim3(totals[0]), dim3(256), 0, st, d_solves, d_pref, n);
     const size_t lds = (size_t(ty) * (kTX + 3) + size_t(ty + 3) * kTX) * sizeof(FaceRec<T>) + size_t(ty) * kTX * (1 + 4 * 64) * sizeof(T);
-    if (keep) hipLaunchKernelGGL((k_tile2d<T, FLUX, true>), dim3(totals[1]), dim3(256), lds, st, d_solves, d_pref + (n + 1), n);
+    if (last) hipLaunchKernelGGL((k_tile2d<T, FLUX, true>), dim3(totals[1]), dim3(256), lds, st, d_solves, d_pref + (n + 1), n);
     else hipLaunchKernelGGL((k_tile2d<T, FLUX, false>), dim3(totals[1]), dim3(256), lds, st, d_solves, d_pref + (n + 1), n);
-    hipLaunchKernelGGL(k_chain2d<T>, dim3((totals[2] + 15) / 16), dim3(256), 0, st, d_solves, d_pref + 2 * (n + 1), n, rows, keep);
-    if (share && !last) hipLaunchKernelGGL((k_relax2d<T, FLUX, true>), dim3(totals[3]), dim3(256), 0, st, d_solves, d_pref + 3 * (n + 1), n);
-    else hipLaunchKernelGGL((k_relax2d<T, KFVS, false>), dim3(totals[3]), dim3(256), 0, st, d_solves, d_pref + 3 * (n + 1), n);
+    hipLaunchKernelGGL(k_chain2d<T>, dim3((totals[2] + 15) / 16), dim3(256), 0, st, d_solves, d_pref + 2 * (n + 1), n, rows, last);
+    const dim3 gr(totals[3]), b(256);
+    const int* rstart = d_pref + 3 * (n + 1);
+    if (last) hipLaunchKernelGGL((k_relax2d<T, KFVS, false, true>), gr, b, 0, st, d_solves, rstart, n);
+    else if (share) hipLaunchKernelGGL((k_relax2d<T, FLUX, true, false>), gr, b, 0, st, d_solves, rstart, n);
+    else hipLaunchKernelGGL((k_relax2d<T, KFVS, false, false>), gr, b, 0, st, d_solves, rstart, n);
     return hipGetLastError();
 }
 
 hipError_t launch_tile2d(bool fp64, int flux, int ty, const Solve2D* d_solves, const int* d_pref, int n, const int* totals, int rows, int first,
-                         int last, int keep, hipStream_t st) {
+                         int last, hipStream_t st) {
     if (ty < 1 || ty > kTile2dRows) return hipErrorInvalidValue;
-#define KBG_T(T, FL) return launch_tile_t<T, FL>(ty, d_solves, d_pref, n, totals, rows, first, last, keep, st)
+#define KBG_T(T, FL) return launch_tile_t<T, FL>(ty, d_solves, d_pref, n, totals, rows, first, last, st)
     if (fp64) {
         if (flux == KFVS) KBG_T(double, KFVS);
         if (flux == KCU) KBG_T(double, KCU);

@@ -93,7 +93,6 @@ struct Solve2D {
     // the tiled step (kbg_tile2d.hip; NULL where the solve does not take it)
     int ty;                                        // rows per tile
     const void* rds;                               // [nx*ny] 1 / (dx dy), storage type
-    void* g;                                       // [nx*ny][2][nv] f + sum of face fluxes / ds
     void* xrec;                                    // [(nx+1)*ny][kFaceT] interior faces' flux coefficients
     void* yrec;                                    // [nx*(ny+1)][kFaceT]
     double* xfrec;                                 // [(nx+1)*ny][8] fw0 len, Mr's coefficient, n1, n2
@@ -293,10 +292,10 @@ hipError_t launch_cell2d(bool fp64, int threads, const Solve2D* d_solves, const 
 // The tiled 2D step of n solves of one precision and flux, ty rows per tile (at most kTile2dRows).  d_pref:
 // four prefix arrays of n + 1 (workgroups of k_pre2d, pre2d_wgs; of k_tile2d, ceil(nx / kTile2dX) ceil(ny / ty)
 // ceil(nv / 256); cells; workgroups of k_relax2d, relax2d_wgs), totals their last entries.  first: the walls'
-// fluxes and the interface records of this step are not there yet; last: leave the next step's out; keep:
-// also leave the face fluxes, moments and coefficients of Mr where the other kernels do
+// fluxes and the interface records of this step are not there yet; last: leave the next step's out, and the
+// face fluxes, moments and coefficients of Mr where the other kernels do
 hipError_t launch_tile2d(bool fp64, int flux, int ty, const Solve2D* d_solves, const int* d_pref, int n, const int* totals, int rows, int first,
-                         int last, int keep, hipStream_t st);
+                         int last, hipStream_t st);
 int tile2d_rows(bool fp64, long one_row);  // rows per tile for a group of `one_row` workgroups of one row
 int pre2d_wgs(int nx, int ny);
 int relax2d_wgs(int nx, int ny, int nv);

@@ -60,3 +60,12 @@ def test_version_and_footprint_without_gpu():
     ks = kb.SolverSet(kb.configs.sod_1d1f1v())
     n32, n64 = kb.solve_bytes(ks, "fp32"), kb.solve_bytes(ks, "fp64")
     assert n64 > n32 > 2 * 100 * 64 * 4
+
+
+@pytest.mark.parametrize("flux,precision", [("ugks", "fp32"), ("kfvs", "fp32"), ("ugks", "fp64"), ("kfvs", "fp64")])
+def test_a_2d_solve_holds_f_and_two_flux_arrays(flux, precision):
+    """What a large cavity solve holds beside f and the two face-flux arrays does not follow its velocities: about
+    2 kB of records per cell, less than a tenth of them at 32^2 velocities (a third such array is 33 %)."""
+    ks = kb.SolverSet(kb.configs.cavity_2d2f2v(nx=64, ny=60, nu=32, nv=32, flux=flux))
+    arrays = (64 * 60 + 65 * 60 + 64 * 61) * 2 * 32 * 32 * (4 if precision == "fp32" else 8)
+    assert arrays < kb.solve_bytes(ks, precision) < 1.1 * arrays
