@@ -762,10 +762,10 @@ __global__ __launch_bounds__(256) void k_chain2d(const Solve2D* __restrict__ sol
 // to a wall its wall fluxes.  KEEP: the flux arrays hold the face fluxes, from which G is formed here.  Bound by
 // memory: 604 MB in 124 us at 16384 cells x 48^2 velocities in FP32.
 template <class T, int FLUX, bool NEXT, bool KEEP>
-__global__ __launch_bounds__(256, NEXT ? 4 : 6) void k_relax2d(const Solve2D* __restrict__ solves, const int* __restrict__ rstart, int nsolves) {
+__global__ __launch_bounds__(256, NEXT || KEEP ? 4 : 6) void k_relax2d(const Solve2D* __restrict__ solves, const int* __restrict__ rstart, int nsolves) {
     constexpr int VPT = 4;
     __shared__ double red[NEXT ? 36 : 1];
-    const int g = blockIdx.x;
+    const int g = KEEP ? xcd_order() : int(blockIdx.x);  // KEEP: neighbouring cells' shared faces from one L2
     if (g >= rstart[nsolves]) return;
     const int si = owner(rstart, nsolves, g);
     const Solve2D& S = solves[si];
