@@ -113,11 +113,12 @@ int kbg_ctx_set_graphs(kbg_ctx *ctx, int enable);
 int kbg_ctx_set_sweep_steps(kbg_ctx *ctx, int steps);
 /* Most velocities per wavefront of the fused 1D sweep: 0 (default) takes the kernel's full width
  * (64 FP32 velocities of one distribution), or 8 velocities on up to 16 wavefronts in KFVS batches too
- * small to fill the chip; 8, 16 or 32 spread each segment's velocity grid over more wavefronts (at most 8
- * in large batches), which shortens the pass of latency-bound batches (serving) at some cost in
- * throughput on large ones; 64 always takes the full width.  The order of a solve's sums depends only on
- * its velocity count and this setting, so its results are the same in any batch.  No counterpart in
- * KitBase. */
+ * small to fill the chip; 8 does the same (and 8 velocities on up to 8 wavefronts in any batch for solves
+ * that have no such choice: KCU, UGKS, many velocities); 16 or 32 spread each segment's velocity grid over
+ * more wavefronts (at most 8, in small KFVS batches 16), which shortens the pass of latency-bound batches
+ * (serving) at some cost in throughput on large ones; 64 always takes the full width.  The order of a
+ * solve's sums depends only on its velocity count and this setting (one order for 0 and 64), so its
+ * results are the same in any batch.  No counterpart in KitBase. */
 int kbg_ctx_set_sweep_vw(kbg_ctx *ctx, int vw);
 /* HIP events on the context stream, for timing: record slot (0..15), elapsed ms between slots.
  * kbg_step / kbg_batch_step record slots KBG_EV_STEPS_BEGIN and KBG_EV_STEPS_END around their

@@ -3,14 +3,15 @@
 The knobs, searched one after another on the caller's own batch:
   1. the context's schedule (kbg_ctx_set_schedule): cells per sweep workgroup (segment length,
      1..60) and the number of concurrent streams the batch is spread over (1..4);
-  2. the most velocities per sweep wavefront (kbg_ctx_set_sweep_vw: 0 = the kernel's full width,
-     64 FP32 / 32 FP64 for one distribution; 32 or 16 put more wavefronts on each work item);
+  2. the most velocities per sweep wavefront (kbg_ctx_set_sweep_vw: 0 = by the size of the batch, the
+     kernel's full width, 64 FP32 / 32 FP64 for one distribution, or 8; 32 or 16 put more wavefronts
+     on each work item);
   3. HIP graph replay of the step rounds against launching them one by one (kbg_ctx_set_graphs).
 Each candidate is timed with the library's step-loop events (kbg_batch_step records
 KBG_EV_STEPS_BEGIN / END around its steps); the fastest is kept and left set on the context.
 Trials advance the solves like any other steps; tune() returns how many steps it took, so a
-caller can count them as warm-up.  Results do not depend on the knobs (a solve's arithmetic and
-sums keep their order in any schedule).
+caller can count them as warm-up.  Results do not depend on the schedule and the replay; a cap of 32
+or 16 velocities adds a solve's FP64 moment sums in another order.
 
 Results are cached per batch signature (solve count, cells, velocity counts, precision and flux
 mix) in a JSON file when `cache` is given, so a serving process tunes a shape once.

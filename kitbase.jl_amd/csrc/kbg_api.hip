@@ -1953,17 +1953,25 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
     // velocities, about 55 wavefronts each at full width): n = 4 19.2 / 9.4, 24 21.2 / 13.1, 36 22.9 / 19.1,
     // 48 26.2 / 24.9, 64 30.5 / 32.3, 96 33.1 / 47.1, 256 85.2 / 131.
     // A solve's results do not depend on the width (kbg_sweep.h), so the rule may look at the whole batch.
-    constexpr long kNarrowWaves = 2700;
+    // A cap of 16 or 32 velocities per wavefront sets the order of a solve's sums too, that of k_sweep1d's
+    // wavefronts under it, whichever kernel steps it; with a cap of 8 solves that may take the narrow sweep add in
+    // the full width's order and take the full width in large batches.  Under the cap of 16 the other side is
+    // k_sweep1d at 16 velocities, us per step it / narrow: n = 16 14.8 / 10.2, 32 17.9 / 18.3, 48 23.3 / 27.1.
+    constexpr long kNarrowWaves = 2700, kNarrowWavesCap = 1600;
+    const int sum_cap = ctx->sweep_vw == 16 || ctx->sweep_vw == 32 ? ctx->sweep_vw : 0;
     long waves0 = 0;
     for (int i : fused) {
         const Solve1D& S = solves[i]->h1;
         waves0 += long(S.upd_hi - S.upd_lo + kbg::sweep_out(2)) / kbg::sweep_out(2) * solves[i]->sweep_nw;
     }
-    std::vector<int> narrow_nw(n, 0);  // wavefronts per item of the narrow sweep, 0: the full-width sweep
+    std::vector<int> narrow_nw(n, 0);  // wavefronts per item of the narrow sweep, 0: k_sweep1d
+    std::vector<int> wide_nw(n, 0);    // and of k_sweep1d: the kernel's width, or more under a cap
     for (int i : fused) {
         const kbg_solve* s = solves[i];
         const int nv = s->d.nv, most = kbg::sweep_vw_narrow(s->d.nf);
-        if (s->d.flux != KBG_KFVS || nv > kbg::kSweepNarrowWaves * most || waves0 > kNarrowWaves || ctx->sweep_vw > most) continue;
+        const bool may = s->d.flux == KBG_KFVS && nv <= kbg::kSweepNarrowWaves * most && ctx->sweep_vw <= most;
+        wide_nw[i] = kbg::sweep_cap_nw(s->fp64, s->d.nf, nv, may ? sum_cap : ctx->sweep_vw);
+        if (!may || waves0 > (sum_cap ? kNarrowWavesCap : kNarrowWaves)) continue;
         const int vw = ctx->sweep_vw > 0 ? ctx->sweep_vw : kbg::kVChunk;
         int nw = 1;
         while (nw < kbg::kSweepNarrowWaves && kbg::sweep_item_vw(nv, nw) > vw) nw *= 2;
@@ -2069,15 +2077,13 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
             desc_of[i] = (int)descs.size();
             descs.push_back(s->h1);
             const size_t i0 = items.size();
-            // wavefronts per item: the kernel's width, or more when the context caps the velocities
-            // per wavefront (a function of the solve and the context only, so a solve's sums keep
-            // their order in any batch)
-            int nw = narrow_nw[i] ? narrow_nw[i] : s->sweep_nw;
+            // wide_nw is a function of the solve and the context only, so a solve's sums keep their order
+            // in any batch
+            const int nw = narrow_nw[i] ? narrow_nw[i] : wide_nw[i];
             if (narrow_nw[i] || split[i]) {
                 if (!split[i]) L.narrow = std::max(L.narrow, nw);
                 L.rows = std::max(L.rows, (s->d.nv + kbg::kVChunk - 1) / kbg::kVChunk);
-            } else if (ctx->sweep_vw > 0)
-                while (nw < kbg::kSweepMaxWaves && (s->d.nv + nw - 1) / nw > ctx->sweep_vw) nw *= 2;
+            }
             build_items(s, seg_of(i), desc_of[i], nw, items);
             for (size_t it = i0; it < items.size(); it++) by_nw[nw].push_back((int)it);
             L.wg_waves = std::max(L.wg_waves, nw);
@@ -2241,7 +2247,7 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
                 } else if (L.narrow) {
                     double* rp = keep ? d_rpart + L.item0 * 12 : nullptr;
                     HIPCHK((L.fp64 ? kbg::launch_sweep1d_narrow64 : kbg::launch_sweep1d_narrow32)(
-                        L.nf, L.narrow, L.rows, d_descs, d_items + L.item0, (int)L.nitems, par, rp, per, sst[L.stream]));
+                        L.nf, L.narrow, L.rows, d_descs, d_items + L.item0, (int)L.nitems, par, sum_cap, rp, per, sst[L.stream]));
                 } else {
                     HIPCHK(kbg::launch_sweep1d(L.fp64, L.nf, L.flux, L.wg_waves, d_descs, d_items, d_packs + L.pack0, (int)L.npacks,
                                                par, keep ? d_rpart : nullptr, per, sst[L.stream]));
@@ -2303,6 +2309,7 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
         auto put = [&](const void* p, size_t b) { sig.append(static_cast<const char*>(p), b); };
         auto puti = [&](long long v) { put(&v, sizeof v); };
         puti(nstreams);
+        puti(sum_cap);
         const void* bufs[] = {d_descs, d_items, d_packs, d_descs2, d_pref2};
         put(bufs, sizeof bufs);
         for (Solve1D d : descs) {

@@ -188,14 +188,21 @@ constexpr int sweep_nw(bool fp64, int nf, int nv) {
          : (nv + sweep_vw(fp64, nf) - 1) / sweep_vw(fp64, nf) <= 2 ? 2
          : (nv + sweep_vw(fp64, nf) - 1) / sweep_vw(fp64, nf) <= 4 ? 4 : 8;
 }
+// and under a cap of `cap` velocities per wavefront (0: none)
+constexpr int sweep_cap_nw(bool fp64, int nf, int nv, int cap) {
+    int nw = sweep_nw(fp64, nf, nv);
+    while (cap > 0 && nw < kSweepMaxWaves && (nv + nw - 1) / nw > cap) nw *= 2;
+    return nw;
+}
 // The narrow KFVS sweep of small launches: nstep 1, 2 or 4, items of nw <= kSweepNarrowWaves wavefronts of at
-// most sweep_vw_narrow velocities, wg_waves the largest nw, rows the most 8-velocity chunks of the solves
+// most sweep_vw_narrow velocities, wg_waves the largest nw, rows the most 8-velocity chunks of the solves; the
+// sums run in the order of k_sweep1d's items of sweep_cap_nw(.., cap) wavefronts
 constexpr int kSweepNarrowWaves = 16;
 constexpr int sweep_vw_narrow(int nf) { return 16 / nf; }
 hipError_t launch_sweep1d_narrow32(int nf, int wg_waves, int rows, const Solve1D* d_solves, const WorkItem* d_items, int nitems,
-                                   int par, double* d_rpart, int nstep, hipStream_t st);
+                                   int par, int cap, double* d_rpart, int nstep, hipStream_t st);
 hipError_t launch_sweep1d_narrow64(int nf, int wg_waves, int rows, const Solve1D* d_solves, const WorkItem* d_items, int nitems,
-                                   int par, double* d_rpart, int nstep, hipStream_t st);
+                                   int par, int cap, double* d_rpart, int nstep, hipStream_t st);
 hipError_t sweep_narrow_attr32();
 hipError_t sweep_narrow_attr64();
 // The FP64 KCU / UGKS step of small launches (kbg_split1d.hip), one step per launch; items of at most kSplitOut

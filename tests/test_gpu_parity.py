@@ -445,6 +445,41 @@ def test_sweep_velocity_cap(gpu_ctx, vw):
         gpu_ctx.set_sweep_vw(0)
 
 
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("vw", [8, 16, 32])
+def test_sweep_velocity_cap_in_a_batch_that_fills_the_chip(gpu_ctx, vw, precision):
+    """Under a velocity cap a solve steps to the same bits alone and beside 40 tubes of 4000 cells, a batch beyond
+    the narrow sweep's rule: one distribution at velocity counts whose capped, uncapped and 8-velocity widths all
+    differ, and two distributions."""
+    rng = np.random.default_rng(vw)
+    cfgs = [kb.configs.sod_1d1f1v(nx=120, nu=nv) for nv in (9, 64, 101, 256)]
+    cfgs += [kb.configs.shock_1d2f1v(nx=70, nu=nv, flux="kfvs") for nv in (64, 128)]
+    made = []
+    for cfg in cfgs + [kb.configs.sod_1d1f1v(nx=4000, nu=64)]:
+        ks = kb.SolverSet(cfg)
+        ctr, face = kb.init_fvm(ks)
+        ctr.f *= 1.0 + 0.01 * rng.random(ctr.f.shape)
+        made.append((ks, ctr, face, kb.timestep(ks, ctr)))
+    try:
+        gpu_ctx.set_sweep_vw(vw)
+        small, tube = made[:-1], made[-1]
+        batch = [kb.DeviceSolve(ks, ctr, face, precision, gpu_ctx) for ks, ctr, face, dt in small + [tube] * 40]
+        kb.batch_step(batch, [m[3] for m in small + [tube] * 40], 7, ctx=gpu_ctx)
+        for (ks, ctr, face, dt), b in zip(small, batch):
+            alone = kb.DeviceSolve(ks, ctr, face, precision, gpu_ctx)
+            alone.step(dt, 7)
+            ca, cb = copy.deepcopy(ctr), copy.deepcopy(ctr)
+            alone.download(ca)
+            b.download(cb)
+            alone.close()
+            for x, y in ((ca.f, cb.f), (ca.w, cb.w), (ca.prim, cb.prim)):
+                np.testing.assert_array_equal(x, y, err_msg=f"{ks.vs.nv} velocities")
+        for d in batch:
+            d.close()
+    finally:
+        gpu_ctx.set_sweep_vw(0)
+
+
 def test_residual_fused_matches_oracle(gpu_ctx):
     ks = kb.SolverSet(kb.configs.sod_1d1f1v(nx=64))
     ctr, face = kb.init_fvm(ks)
