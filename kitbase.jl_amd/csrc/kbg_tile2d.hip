@@ -12,7 +12,7 @@
 //              forms G from f and them, with the same operations.  The tile's face records sit in
 //              LDS: as scalar loads their waits and the spills of scalar registers took a third of the
 //              kernel.  Faces between tiles are evaluated by both, with the same operations; the tile to
-//              their right (above) adds up their moments: over 8 lanes in the storage type, then in FP64.
+//              their right (above) adds up their moments in FP64.
 //   k_chain2d  16 lanes per cell: the four faces' moments (the workgroups' sums in order) and the FP64 cell
 //              chain (w, prim, the relaxation's coefficients).
 //   k_relax2d  one workgroup per cell: f = (G + (dt / tau) M) / (1 + dt / tau), and for a cell next to a wall
@@ -55,27 +55,31 @@ constexpr int kTX = kTile2dX;
 
 // An interior face's flux coefficients in the storage type, the length folded in.  With x, y the normal and
 // tangential velocity, h, b the upwind face values and sh, sb their slopes, H = exp(nl |c - U|^2):
-//   UGKS  fh = x (H (P + x R) + M3 h - M4 x sh),  P, R polynomials 1, x, y, x^2 + y^2 (R of the upwind side);
-//         fb = x (H (kb (P + x R) + e0 + x e1) + M3 b - M4 x sb)   (flux_ugks.jl:209-245 factored)
+//   UGKS  fh = x (H (P + x R) + M3 eh), eh = h - rho x sh,  P, R polynomials 1, x, y, x^2 + y^2 (R of the upwind
+//         side), rho = M4 / M3; fb = x (H (kb (P + x R) + x2 (P3 + x R3)) + M3 eb)   (flux_ugks.jl:209-245 factored)
 //   KCU   fh = x (H P0 + M3 h), fb = x (H kb P0 + M3 b)             (flux_kcu.jl:898-967)
-//   KFVS  fh = x (M3 h - M4 x sh), fb alike                         (flux_kfvs.jl:654-697)
+//   KFVS  fh = x M3 eh, fb alike                                    (flux_kfvs.jl:654-697)
+// The moment sums run over w x eh, and M3 multiplies them in FP64 (frec).  FP32 carries rho in two parts: a
+// coefficient's own rounding is the same for all velocities and does not cancel in the sums as theirs do.
 template <class T> struct alignas(16) FaceRec {
-    T nl, U, V, kb, M3, M4, e0, r, P[4];  // r: 1 / centre distance
+    T nl, U, V, kb, M3, rho, x2, r, P[4];  // x2: <xi^4> - <xi^2>^2; r: 1 / centre distance
     struct {
-        T q[4], e1, d;  // R, and the signed half width of the side's cell
-    } s[2];            // left, right
+        T q[4], d;  // R, and the signed half width of the side's cell
+    } s[2];        // left, right
+    T rhol, pad;    // rho + rhol
 };
 static_assert(sizeof(FaceRec<float>) == kFaceT * 4 && sizeof(FaceRec<double>) == kFaceT * 8, "FaceRec");
 
 template <class T> KBG_D T nl_of(double lam);
 template <> KBG_D float nl_of<float>(double lam) { return float(-lam * 1.4426950408889634074); }
 template <> KBG_D double nl_of<double>(double lam) { return -lam; }
-// 1 / x for the limiter's denominators (about one rounding more than a division)
-KBG_D float recip(float x) { return __builtin_amdgcn_rcpf(x); }
-KBG_D double recip(double x) {
+// the limiter's quotient (about one rounding more than a division in FP64)
+KBG_D float quot(float a, float x) { return a * __builtin_amdgcn_rcpf(x); }
+KBG_D double quot(double a, double x) {
     double r = __builtin_amdgcn_rcp(x);
     r = __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
-    return __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
+    r = __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
+    return a * r;
 }
 KBG_D float gauss(float x) { return __builtin_amdgcn_exp2f(x); }
 KBG_D double gauss(double x) { return exp(x); }
@@ -109,7 +113,8 @@ template <class T, int FLUX> KBG_D void face_chain(const Solve2D& S, int b) {
     o.s[1].d = T(-dxR);
     if constexpr (FLUX == KFVS) {
         o.M3 = T(dt * len);
-        o.M4 = T(0.5 * dt * dt * len);
+        o.rho = T(0.5 * dt);
+        o.rhol = T(0.5 * dt - double(o.rho));
         for (int m = 0; m < 4; m++) fr[m] = 0.0;
         fr[4] = dt * len;
     } else {
@@ -144,7 +149,9 @@ template <class T, int FLUX> KBG_D void face_chain(const Solve2D& S, int b) {
             o.V = T(F.prim[2]);
             o.kb = T(kb);
             o.M3 = T(F.Mt[3] * len);
-            o.M4 = T(F.Mt[4] * len);
+            const double rho = F.Mt[3] != 0.0 ? F.Mt[4] / F.Mt[3] : 0.0;  // both 0 there
+            o.rho = T(rho);
+            o.rhol = T(rho - double(o.rho));
             o.P[0] = T(a0 + a2 * (F.aT[0] + 0.5 * F.aT[3] * kb));
             o.P[1] = T(a2 * F.aT[1]);
             o.P[2] = T(a2 * F.aT[2]);
@@ -157,10 +164,7 @@ template <class T, int FLUX> KBG_D void face_chain(const Solve2D& S, int b) {
             o.s[1].q[1] = T(a1 * F.aR[1]);
             o.s[1].q[2] = T(a1 * F.aR[2]);
             o.s[1].q[3] = T(a1 * 0.5 * F.aR[3]);
-            const double x2 = F.Mxi2 - kb * kb;  // <xi^4> - <xi^2>^2
-            o.e0 = T(a2 * 0.5 * F.aT[3] * x2);
-            o.s[0].e1 = T(a1 * 0.5 * F.aL[3] * x2);
-            o.s[1].e1 = T(a1 * 0.5 * F.aR[3] * x2);
+            o.x2 = T(F.Mxi2 - kb * kb);
             for (int m = 0; m < 4; m++) fr[m] = F.fw0[m] * len;
             fr[4] = F.Mt[3] * len;
         }
@@ -341,18 +345,22 @@ template <int CTRL> KBG_D double dppx(double x) {
     return __builtin_bit_cast(double, ((long long)hi << 32) | (long long)(unsigned)lo);
 }
 // keep + the partner's send, where up lanes keep b and send a, the others keep a and send b
-template <int CTRL, class T> KBG_D T fold(bool up, T a, T b) {
+template <int CTRL, class T, class S = T> KBG_D S fold(bool up, T a, T b) {
     // pinned, or the selects become one load through a selected address and the sums go to scratch
     asm volatile("" : "+v"(a), "+v"(b));
-    return (up ? b : a) + dppx<CTRL>(up ? a : b);
+    return S(up ? b : a) + S(dppx<CTRL>(up ? a : b));
 }
-// sums of 8 values over 8 lanes in the storage type: lane l ends with value l & 7 of its group of 8
-template <class T> KBG_D T sum8(int lane, T (&v)[8]) {
-    T a[4], b[2];
+// Sums of 8 values over 8 lanes, in FP64: lane l ends with value l & 7 of its group of 8.  Neighbouring lanes hold
+// velocities of one sign, whose terms of the mass flux do not cancel: added in FP32 they left 1.4 to 1.7 times the
+// error in rho of k_flux2d, whose lanes each add 8 velocities apart by 64 in FP32 (KFVS, one step of 61 x 60 cells
+// x 600 velocities); in FP64 0.6 to 0.8 times.  UGKS FP32 64 x 64 cells x 32^2 velocities 61 us per step either way
+// with the rows per tile chosen for each; 45 x 45 x 28^2 46.5 in FP32, 47.7 here.
+template <class T> KBG_D double sum8(int lane, T (&v)[8]) {
+    double a[4], b[2];
 #pragma unroll
-    for (int m = 0; m < 4; m++) a[m] = fold<0x141>((lane & 4) != 0, v[m], v[m + 4]);  // row_half_mirror
+    for (int m = 0; m < 4; m++) a[m] = fold<0x141, T, double>((lane & 4) != 0, v[m], v[m + 4]);  // row_half_mirror
 #pragma unroll
-    for (int m = 0; m < 2; m++) b[m] = fold<0x4e>((lane & 2) != 0, a[m], a[m + 2]);   // quad_perm 2 3 0 1
+    for (int m = 0; m < 2; m++) b[m] = fold<0x4e>((lane & 2) != 0, a[m], a[m + 2]);  // quad_perm 2 3 0 1
     return fold<0xb1>((lane & 1) != 0, b[0], b[1]);                                  // quad_perm 1 0 3 2
 }
 
@@ -380,7 +388,7 @@ template <class T, int FLUX, int SX, int SY> struct Tile {
     // van Leer: (sL |sR| + |sL| sR) / (|sL| + |sR| + 1e-7), by reciprocal
     static KBG_D T lim1(T sL, T sR) {
         const T aL = fabs(sL), aR = fabs(sR);
-        return (sL * aR + aL * sR) * recip(aL + aR + T(1e-7));
+        return quot(sL * aR + aL * sR, aL + aR + T(1e-7));
     }
     static KBG_D H2 lim(H2 l, H2 r) { return H2{lim1(l.x, r.x), lim1(l.y, r.y)}; }
     // one-sided where c
@@ -400,36 +408,36 @@ template <class T, int FLUX, int SX, int SY> struct Tile {
             const T dr = R->s[1].d;
             d = dd ? d : dr;
         }
-        const T h = (dd ? fa.x : fc.x) + sh * d, b = (dd ? fa.y : fc.y) + sb * d;
-        T eh = M3 * h, eb = M3 * b, Fh, Fb;
+        T eh = (dd ? fa.x : fc.x) + sh * d, eb = (dd ? fa.y : fc.y) + sb * d, Fh, Fb;
         if constexpr (FLUX == KCU) {
             const T cu = x - R->U, cv = y - R->V;
             const T g = gauss(R->nl * (cu * cu + cv * cv)) * R->P[0];
-            Fh = x * (g + eh);
-            Fb = x * (g * R->kb + eb);
+            Fh = x * (g + M3 * eh);
+            Fb = x * (g * R->kb + M3 * eb);
         } else {
-            const T m4x = R->M4 * x;
-            eh -= m4x * sh;
-            eb -= m4x * sb;
+            const T rx = sizeof(T) == 4 ? R->rho * x + R->rhol * x : R->rho * x;
+            eh -= rx * sh;
+            eb -= rx * sb;
             if constexpr (FLUX == KFVS) {
-                Fh = x * eh;
-                Fb = x * eb;
+                Fh = x * (M3 * eh);
+                Fb = x * (M3 * eb);
             } else {
                 const T cu = x - R->U, cv = y - R->V;
                 const T H = gauss(R->nl * (cu * cu + cv * cv));
                 T q = R->s[sd].q[0] + x * R->s[sd].q[1] + y * R->s[sd].q[2] + q2 * R->s[sd].q[3];
-                T xe = x * R->s[sd].e1;
+                T q3 = R->s[sd].q[3];
                 if constexpr (SD == 2) {
                     const T qR = R->s[1].q[0] + x * R->s[1].q[1] + y * R->s[1].q[2] + q2 * R->s[1].q[3];
-                    const T xr = x * R->s[1].e1;
+                    const T r3 = R->s[1].q[3];
                     q = dd ? q : qR;
-                    xe = dd ? xe : xr;
+                    q3 = dd ? q3 : r3;
                 }
                 const T p = R->P[0] + x * R->P[1] + y * R->P[2] + q2 * R->P[3];
                 const T g = p + x * q;
-                const T gb = R->kb * g + (R->e0 + xe);
-                Fh = x * (H * g + eh);
-                Fb = x * (H * gb + eb);
+                const T t3 = R->P[3] + x * q3;
+                const T gb = R->kb * g + R->x2 * t3;
+                Fh = x * (H * g + M3 * eh);
+                Fb = x * (H * gb + M3 * eb);
             }
         }
         if constexpr (SUMS) {
@@ -455,7 +463,7 @@ namespace {
 // [row][pair of faces][8 groups of 8 lanes][8 values]
 template <class T, int FLUX, bool KEEP, int SX, int SY>
 KBG_D void tile_march(const Solve2D& S, int i0, int j0, int j1, int iv, bool live, T u, T v, int lane, const FaceRec<T>* XR, const FaceRec<T>* YR,
-                      const T* RD, T* sums) {
+                      const T* RD, double* sums) {
     constexpr int E = sizeof(T);
     using H2 = HB<T>;
     using TL = Tile<T, FLUX, SX, SY>;
@@ -492,7 +500,7 @@ KBG_D void tile_march(const Solve2D& S, int i0, int j0, int j1, int iv, bool liv
             sB[t] = qB[t];
             FD[t] = ldf(yff, i0 + t);
         });
-        sums[2 * 64 + lane] = sums[3 * 64 + lane] = T(0);
+        sums[2 * 64 + lane] = sums[3 * 64 + lane] = 0.0;
     } else {
         static_for<kTX>([&](auto t) {
             constexpr int o = (t & 1) * 4;
@@ -609,8 +617,8 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 4 : 2) void k_tile2d(const So
     FaceRec<T>* XR = reinterpret_cast<FaceRec<T>*>(tile_lds);
     FaceRec<T>* YR = XR + ty * (kTX + 3);
     T* RD = reinterpret_cast<T*>(YR + (ty + 3) * kTX);
-    T* sums = RD + ty * kTX;
-    T* ws = sums + (size_t)wave * nws;
+    double* sums = reinterpret_cast<double*>(RD + ty * kTX);
+    double* ws = sums + (size_t)wave * nws;
     {
         constexpr int P = sizeof(FaceRec<T>) / 16;
         const int nX = rows * (kTX + 3), nR = nX + (rows + 3) * kTX;
@@ -640,7 +648,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 4 : 2) void k_tile2d(const So
         else KBG_M(1, 1);
 #undef KBG_M
     } else {
-        for (int k = lane; k < nws; k += 64) ws[k] = T(0);
+        for (int k = lane; k < nws; k += 64) ws[k] = 0.0;
     }
     __syncthreads();
     const size_t FX = size_t(nx + 1) * ny, F = FX + size_t(nx) * (ny + 1);
@@ -649,9 +657,9 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 4 : 2) void k_tile2d(const So
         const int m = k & 3, sl = k >> 2, t = sl % kTX, ydir = (sl / kTX) & 1, j = j0 + sl / (2 * kTX);
         double q = 0.0;
         for (int w = 0; w < 4; w++) {
-            const T* p = sums + (size_t)w * nws + (sl >> 1) * 64 + (sl & 1) * 4 + m;
+            const double* p = sums + (size_t)w * nws + (sl >> 1) * 64 + (sl & 1) * 4 + m;
 #pragma unroll
-            for (int g8 = 0; g8 < 8; g8++) q += double(p[g8 * 8]);
+            for (int g8 = 0; g8 < 8; g8++) q += p[g8 * 8];
         }
         const size_t f = ydir ? FX + (i0 + t) + size_t(nx) * j : size_t(i0 + t) + size_t(nx + 1) * j;
         S.psum[(size_t(chunk) * F + f) * 4 + m] = q;
@@ -697,7 +705,6 @@ __global__ __launch_bounds__(256) void k_chain2d(const Solve2D* __restrict__ sol
         const int nch = (S.nv + 255) / 256;
 #pragma unroll 4
         for (int k = 0; k < nch; k++) q += ps[size_t(k) * F * 4];
-        q += fr[m];
         if (del) {
             // the sums ran over departures: the reference Maxwellian's share from its moments
             const double* mm = S.mmom;
@@ -706,8 +713,9 @@ __global__ __launch_bounds__(256) void k_chain2d(const Solve2D* __restrict__ sol
             else if (m == 1) r = n1 * n1 * mm[2] + 2.0 * n1 * n2 * mm[3] + n2 * n2 * mm[4];
             else if (m == 2) r = (n1 * n1 - n2 * n2) * mm[3] + n1 * n2 * (mm[4] - mm[2]);
             else r = 0.5 * (n1 * (mm[5] + mm[7]) + n2 * (mm[6] + mm[8]) + n1 * mm[9] + n2 * mm[10]);
-            q += cf * r;
+            q += r;
         }
+        q = fr[m] + cf * q;
     }
     const double o = __shfl_xor(q, 3, 64);  // moments 1 and 2 change places
     const double fw = wall ? q : m == 1 ? q * n1 - o * n2 : (m == 2 ? o * n2 + q * n1 : q);
@@ -840,13 +848,20 @@ __global__ __launch_bounds__(256, NEXT || KEEP ? 4 : 6) void k_relax2d(const Sol
 int pre2d_wgs(int nx, int ny) { return (interior_faces(nx, ny) + 255) / 256 + wall_cells(nx, ny); }
 int relax2d_wgs(int nx, int ny, int nv) { return pre2d_wgs(nx, ny) + (nx * ny - wall_cells(nx, ny)) * ((nv + 1023) / 1024); }
 // Fewer rows repeat the two faces' and slopes' work of the rows around a tile more often, more rows leave too few
-// workgroups to overlap one's waits with another's work.  us per step at 1 / 2 / 3 / 4 / 6 rows: FP32 KCU 24 x 24
-// cells x 16^2 velocities 24.7 / 25.6 / 27.5 / 29.3 / 33, UGKS 45 x 45 x 28^2 50 / 47 / 45 / 48 / 50, 100 x 100 x
-// 28^2 128 / 110 / 109 / 110 / 115, 128 x 128 x 48^2 601 / 504 / 491 / 484 / 485; FP64 (2 workgroups per CU) UGKS
-// 64 x 64 x 32^2 121 / 102 / 103 / 95 / 103, 100 x 100 x 40^2 583 / 500 / 464 / 451 / 435.
+// workgroups to overlap one's waits with another's work; FP32 holds 4 workgroups per CU, and between 3072 and 4096
+// of one row three rows per tile are a few more than the chip holds at once.  us per step at 1 / 2 / 3 / 4 / 6 rows:
+// FP32 UGKS 24 x 24 cells x 16^2 velocities 28 / 30 / 33 / 36 / 41, 45 x 45 x 28^2 53 / 50 / 48 / 51 / 54, 64 x 64 x
+// 24^2 59 / 54 / 58 / 53 / 72, 64 x 64 x 32^2 69 / 61 / 64 / 61 / 74, 100 x 100 x 40^2 247 / 218 / 214 / 218 / 237,
+// 128 x 128 x 48^2 605 / 510 / 496 / 488 / 544; FP64 (2 workgroups per CU) UGKS 64 x 64 x 32^2 121 / 102 / 103 / 95 /
+// 103, 100 x 100 x 40^2 583 / 500 / 464 / 451 / 435.
 int tile2d_rows(bool fp64, long one_row) {
     if (fp64) return one_row <= 256 ? 1 : one_row <= 1024 ? 2 : one_row <= 3072 ? 3 : one_row <= 12288 ? 4 : 6;
-    return one_row <= 1024 ? 1 : one_row <= 16384 ? 3 : 6;
+    return one_row <= 1024 ? 1 : one_row <= 2560 ? 3 : one_row <= 5120 ? 4 : one_row <= 24576 ? 3 : 4;
+}
+
+// records, 1 / (dx dy) and sums of a tile of ty rows
+template <class T> constexpr size_t tile2d_lds(int ty) {
+    return (size_t(ty) * (kTX + 3) + size_t(ty + 3) * kTX) * sizeof(FaceRec<T>) + size_t(ty) * kTX * (sizeof(T) + 4 * 64 * sizeof(double));
 }
 
 template <class T, int FLUX>
@@ -857,7 +872,7 @@ static hipError_t launch_tile_t(int ty, const Solve2D* d_solves, const int* d_pr
     // 100 x 40^2 FP64 439 / 451, 128 x 128 x 48^2 FP32 502 / 487)
     const bool share = totals[3] <= 32768;
     if (first || !share) hipLaunchKernelGGL((k_pre2d<T, FLUX>), dim3(totals[0]), dim3(256), 0, st, d_solves, d_pref, n);
-    const size_t lds = (size_t(ty) * (kTX + 3) + size_t(ty + 3) * kTX) * sizeof(FaceRec<T>) + size_t(ty) * kTX * (1 + 4 * 64) * sizeof(T);
+    const size_t lds = tile2d_lds<T>(ty);
     if (last) hipLaunchKernelGGL((k_tile2d<T, FLUX, true>), dim3(totals[1]), dim3(256), lds, st, d_solves, d_pref + (n + 1), n);
     else hipLaunchKernelGGL((k_tile2d<T, FLUX, false>), dim3(totals[1]), dim3(256), lds, st, d_solves, d_pref + (n + 1), n);
     hipLaunchKernelGGL(k_chain2d<T>, dim3((totals[2] + 15) / 16), dim3(256), 0, st, d_solves, d_pref + 2 * (n + 1), n, rows, last);
@@ -886,8 +901,7 @@ hipError_t launch_tile2d(bool fp64, int flux, int ty, const Solve2D* d_solves, c
 
 // above the 64 KB of dynamic LDS a kernel may use without asking
 hipError_t tile2d_attr() {
-    constexpr int R = kTile2dRows;
-    constexpr size_t lds = (size_t(R) * (kTX + 3) + size_t(R + 3) * kTX) * sizeof(FaceRec<double>) + size_t(R) * kTX * (1 + 4 * 64) * sizeof(double);
+    constexpr size_t lds = tile2d_lds<double>(kTile2dRows);
     hipError_t e = hipSuccess;
     for (const void* k : {(const void*)k_tile2d<double, KFVS, false>, (const void*)k_tile2d<double, KFVS, true>,
                           (const void*)k_tile2d<double, KCU, false>, (const void*)k_tile2d<double, KCU, true>,

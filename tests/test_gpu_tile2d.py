@@ -129,3 +129,36 @@ def test_tiled_step_under_graph_replay(gpu_ctx):
             gpu_ctx.set_graphs(False)
     np.testing.assert_array_equal(got[0].f, got[1].f)
     np.testing.assert_array_equal(got[0].w, got[1].w)
+
+
+@pytest.mark.parametrize("space,flux", [("2d2f2v", "ugks"), ("2d2f2v", "kcu"), ("2d2f2v", "kfvs"), ("2d1f2v", "kfvs")])
+def test_tiled_fp32_moments_are_no_less_accurate_than_the_face_parallel_ones(gpu_ctx, space, flux):
+    """One FP32 step's error in w against the oracle's step from the same stored state: the tiled kernels beside
+    k_flux2d / k_cell2d, to which a normal one rounding off another sends the solve.  The tiled moments add no more
+    terms in FP32 than those (8 per lane) and weight them in FP64 as they do, so the rms error over the 3660 cells
+    may exceed theirs by its scatter only: 1.1 for every conserved variable."""
+    mk = kb.configs.cavity_2d2f2v if space == "2d2f2v" else kb.configs.cavity_2d1f2v
+    ks = kb.SolverSet(mk(nx=61, ny=60, nu=25, nv=24, knudsen=0.05, flux=flux, vMeshType="rectangle"))
+    ctr, face = kb.init_fvm(ks)
+    dt = kb.timestep(ks, ctr)
+    dev = kb.DeviceSolve(ks, ctr, face, "fp64", gpu_ctx)
+    dev.step(dt, 100)
+    dev.download(ctr)
+    dev.close()
+    ctr.f *= 1.0 + 0.02 * np.random.default_rng(3).random(ctr.f.shape)
+    err, n1 = [], ks.ps.n[0, 0, 1, 0]
+    for tiled in (True, False):
+        ks.ps.n[0, 0, 1, 0] = n1 if tiled else np.nextafter(n1, 0.0)
+        dev = kb.DeviceSolve(ks, ctr, copy.deepcopy(face), "fp32", gpu_ctx)
+        got, ref = copy.deepcopy(ctr), copy.deepcopy(ctr)
+        dev.download(ref)
+        dev.step(dt, 1)
+        dev.download(got)
+        dev.close()
+        o = oracle.OracleSolve(ks, ref, copy.deepcopy(face))
+        o.reconstruct()
+        o.evolve(dt)
+        o.update(dt)
+        err.append(np.sqrt(np.mean((got.w - ref.w).reshape(-1, 4) ** 2, axis=0)))
+    ks.ps.n[0, 0, 1, 0] = n1
+    assert np.all(err[0] <= 1.1 * err[1]), (err[0] / err[1])
