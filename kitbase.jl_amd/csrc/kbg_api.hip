@@ -623,33 +623,28 @@ bool tiled2d(const kbg_desc& d) {
     return true;
 }
 
+size_t tile2d_bytes(const kbg_desc& d) {
+    const kbg::Tile2D t = kbg::tile2d_at(nullptr, d.nx, d.ny, d.nv, d.precision == KBG_FP64 ? 8 : 4);
+    return size_t(t.end - t.xrec);
+}
+
 // buffers of the tiled step
 int alloc_tiled2d(kbg_solve* s) {
     const kbg_desc& d = s->d;
     Solve2D& S = s->h2;
-    const size_t C = s->N, FX = size_t(d.nx + 1) * d.ny, FY = size_t(d.nx) * (d.ny + 1), nch = (size_t(d.nv) + 255) / 256;
-    void *rds, *perm;
-    struct {
-        void** dst;
-        size_t bytes;
-    } tb[] = {{&S.xrec, FX * kbg::kFaceT * s->esz}, {&S.yrec, FY * kbg::kFaceT * s->esz}, {(void**)&S.xfrec, FX * 64},
-              {(void**)&S.yfrec, FY * 64},         {(void**)&S.psum, nch * (FX + FY) * 32}, {&S.crec, C * kbg::kCellT * s->esz},
-              {&rds, C * s->esz},                  {&perm, size_t(d.nv) * 4}};
+    const size_t C = s->N, bytes = tile2d_bytes(d);
     int rc;
-    for (auto& b : tb) {
-        if ((rc = dev_alloc(s, b.dst, b.bytes))) return rc;
-        HIPCHK(hipMemset(*b.dst, 0, b.bytes));
-    }
+    if ((rc = dev_alloc(s, &S.tile, bytes))) return rc;
+    HIPCHK(hipMemset(S.tile, 0, bytes));
+    const kbg::Tile2D t = kbg::tile2d_at(S.tile, d.nx, d.ny, d.nv, int(s->esz));
     std::vector<double> r(C);
     for (size_t c = 0; c < C; c++) r[c] = 1.0 / (d.dx[c] * d.dy[c]);
-    if ((rc = put_real(s, rds, r.data(), C, !s->fp64))) return rc;
+    if ((rc = put_real(s, t.rds, r.data(), C, !s->fp64))) return rc;
     std::vector<int> order(d.nv);
     for (int k = 0; k < d.nv; k++) order[k] = k;
     auto quadrant = [&](int k) { return (d.v[k] >= 0.0 ? 2 : 0) + (d.u[k] >= 0.0 ? 1 : 0); };
     std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return quadrant(a) < quadrant(b); });
-    HIPCHK(hipMemcpy(perm, order.data(), size_t(d.nv) * 4, hipMemcpyHostToDevice));
-    S.rds = rds;
-    S.vperm = static_cast<const int*>(perm);
+    HIPCHK(hipMemcpy(t.vperm, order.data(), size_t(d.nv) * 4, hipMemcpyHostToDevice));
     return KBG_OK;
 }
 
@@ -796,6 +791,7 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
 // stand-in, not a device address): kbg_ctx_create looks up each device's address once, with that
 // device current, and every use goes through scratch_ptr(device).
 constexpr size_t kNoallocScratchBytes = KBG_NOALLOC_SCRATCH_BYTES;
+static_assert(sizeof(Solve1D) <= 344 && sizeof(Solve2D) <= 400, "descriptors the staging array holds a batch of");
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
 void* g_scratch_addr[kMaxDevices] = {};
@@ -998,8 +994,7 @@ size_t kbg_solve_bytes(const kbg_desc* d) {
     if (d->flux != KBG_KFVS) b += F * kbg::kFaceCoef * 8 + (esz == 4 ? F * kbg::kFaceC32 * 4 : 0);
     if (kbg::step2d_threads(d->precision == KBG_FP64, d->nv) == 0) b += C * 8 * 8 + C * 4 * nv * esz;  // slopes
     else if (esz == 4) b += 2 * nv * 4 + F * 8;  // departure form: reference Maxwellian, per-face coefficients
-    if (tiled2d(*d))  // face and cell records, moment sums
-        b += C * (1 + kbg::kCellT) * esz + F * (kbg::kFaceT * esz + 64 + (nv + 255) / 256 * 32) + nv * 4;
+    if (tiled2d(*d)) b += tile2d_bytes(*d);  // face and cell records, moment sums
     return b;
 }
 
@@ -1238,12 +1233,9 @@ int kbg_solve_create(kbg_ctx* ctx, const kbg_desc* desc, kbg_solve** out) {
             HIPCHK(hipMemset(p, 0, 2 * size_t(d.nv) * 4));
             S.mref = (const float*)p;
             s->mref.assign(2 * size_t(d.nv), 0.0f);
-            if ((rc = dev_alloc(s, &p, FX * 8))) return bail(rc);
-            HIPCHK(hipMemset(p, 0, FX * 8));
-            S.xcref = (double*)p;
-            if ((rc = dev_alloc(s, &p, FY * 8))) return bail(rc);
-            HIPCHK(hipMemset(p, 0, FY * 8));
-            S.ycref = (double*)p;
+            if ((rc = dev_alloc(s, &p, (FX + FY) * 8))) return bail(rc);
+            HIPCHK(hipMemset(p, 0, (FX + FY) * 8));
+            S.cref = (double*)p;
         }
         if (tiled2d(d) && (rc = alloc_tiled2d(s))) return bail(rc);
         if ((rc = dev_alloc(s, &p, 8 * 8))) return bail(rc);
@@ -1508,8 +1500,7 @@ int kbg_upload(kbg_solve* s, const double* w, const double* prim, const double* 
     if ((rc = stage_up(s, static_cast<float*>(S.f), N * RS, [fs, mr, RS](size_t i) { return float(fs[i] - double(mr[i % RS])); })))
         return rc;
     HIPCHK(hipMemcpyAsync((void*)S.mref, s->mref.data(), RS * 4, hipMemcpyHostToDevice, s->ctx->stream));
-    HIPCHK(hipMemsetAsync(S.xcref, 0, FX * 8, s->ctx->stream));
-    HIPCHK(hipMemsetAsync(S.ycref, 0, FY * 8, s->ctx->stream));
+    HIPCHK(hipMemsetAsync(S.cref, 0, (FX + FY) * 8, s->ctx->stream));
     HIPCHK(hipStreamSynchronize(s->ctx->stream));
     s->rep_full = false;
     return push2d(s);
@@ -1626,8 +1617,7 @@ int kbg_upload_faces(kbg_solve* s, const double* fw, const double* ff) {
     const size_t FX = size_t(s->d.nx + 1) * s->d.ny, FY = size_t(s->d.nx) * (s->d.ny + 1), RS = 2 * s->d.nv;
     if (ff && s->h2.delta && !s->rep_full) {
         // uploaded face fluxes are full values: none leaves out the reference Maxwellian's part
-        HIPCHK(hipMemsetAsync(s->h2.xcref, 0, FX * 8, s->ctx->stream));
-        HIPCHK(hipMemsetAsync(s->h2.ycref, 0, FY * 8, s->ctx->stream));
+        HIPCHK(hipMemsetAsync(s->h2.cref, 0, (FX + FY) * 8, s->ctx->stream));
     }
     if (fw) {
         if ((rc = put_f64(s, s->h2.xfw, fw, FX * 4))) return rc;
@@ -1679,7 +1669,7 @@ int kbg_download_faces(kbg_solve* s, double* fw, double* ff) {
         if (s->h2.delta && !s->rep_full) {
             // the fused step's face fluxes leave out c x Mr: add it back (FP64, on the host)
             std::vector<double> c(FX + FY);
-            if ((rc = get_f64(s, c.data(), s->h2.xcref, FX)) || (rc = get_f64(s, c.data() + FX, s->h2.ycref, FY))) return rc;
+            if ((rc = get_f64(s, c.data(), s->h2.cref, FX + FY))) return rc;
             const kbg_desc& d = s->d;
             for (size_t fc = 0; fc < FX + FY; fc++) {
                 if (c[fc] == 0.0) continue;
@@ -1884,7 +1874,7 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
     {
         std::map<std::tuple<int, int, int, int>, std::vector<int>> groups;
         for (int i : fused2)
-            groups[{solves[i]->fp64 ? 1 : 0, solves[i]->d.flux, solves[i]->h2.xrec ? 0 : solves[i]->thr2, solves[i]->h2.xrec ? 1 : 0}].push_back(i);
+            groups[{solves[i]->fp64 ? 1 : 0, solves[i]->d.flux, solves[i]->h2.tile ? 0 : solves[i]->thr2, solves[i]->h2.tile ? 1 : 0}].push_back(i);
         for (auto& kv : groups) {
             Launch2 L{std::get<0>(kv.first) == 1, std::get<1>(kv.first), std::get<2>(kv.first), (int)kv.second.size(), 0, 0, 0,
                       descs2.size(), 0, 0, 0, 0.0, 0, {0, 0, 0, 0}};
@@ -1897,7 +1887,6 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
                 for (int i : kv.second) {
                     kbg_solve* s = solves[i];
                     s->h2.dt = dts[i];
-                    s->h2.ty = L.ty;
                     descs2.push_back(s->h2);
                     const long nx = s->d.nx, ny = s->d.ny;
                     const long k[4] = {kbg::pre2d_wgs(s->d.nx, s->d.ny),

@@ -485,7 +485,7 @@ __global__ __launch_bounds__(flux2d_max_threads<T>()) void k_flux2d(const Solve2
                     r[4] += Sy;
                     r[6] += Sq + Sb;
                 }
-                (dir == 0 ? S.xcref : S.ycref)[fi] = cf;
+                S.cref[(dir == 0 ? 0 : size_t(nx + 1) * ny) + fi] = cf;
             }
             double l0, l1, l2, l3;
             if constexpr (FLUX == KFVS) {
@@ -606,7 +606,7 @@ __global__ __launch_bounds__(flux2d_max_threads<T>()) void k_flux2d(const Solve2
         fwout[1] = l1 * n1 - l2 * n2;
         fwout[2] = l1 * n2 + l2 * n1;
         fwout[3] = (0.5 * m3 + 0.5 * m4) * len * dt;
-        if (del) (dir == 0 ? S.xcref : S.ycref)[fi] = len * dt;
+        if (del) S.cref[(dir == 0 ? 0 : size_t(nx + 1) * ny) + fi] = len * dt;
     }
 }
 
@@ -712,7 +712,8 @@ __global__ __launch_bounds__(step2d_max_threads<T>()) void k_cell2d(const Solve2
                 // the reference Maxwellian's share of the four face fluxes: sum of +-c (n1 u + n2 v) / ds
                 const double *gL = S.xgeo + (size_t)L * 3, *gR = S.xgeo + (size_t)R * 3;
                 const double *gD = S.ygeo + (size_t)D * 3, *gU = S.ygeo + (size_t)Up * 3;
-                const double cL = S.xcref[L], cR = S.xcref[R], cD = S.ycref[D], cU = S.ycref[Up];
+                const double* yc = S.cref + size_t(nx + 1) * ny;
+                const double cL = S.cref[L], cR = S.cref[R], cD = yc[D], cU = yc[Up];
                 cst[C_CU] = (cL * gL[0] - cR * gR[0] + cD * gD[0] - cU * gU[0]) / ds;
                 cst[C_CV] = (cL * gL[1] - cR * gR[1] + cD * gD[1] - cU * gU[1]) / ds;
             }
@@ -813,7 +814,7 @@ __global__ __launch_bounds__(256) void k_delta2d(const Solve2D* __restrict__ pS,
     for (int dir = 0; dir < 2; dir++) {
         const long nfc = dir == 0 ? FX : FY;
         float* ff = (float*)(dir == 0 ? S.xff : S.yff);
-        double* cr = dir == 0 ? S.xcref : S.ycref;
+        double* cr = S.cref + (dir == 0 ? 0 : FX);
         const double* geo = dir == 0 ? S.xgeo : S.ygeo;
         if (mode == 2) {
             for (long e = t0; e < nfc * RS; e += stride) {

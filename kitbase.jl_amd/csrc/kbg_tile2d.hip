@@ -70,6 +70,8 @@ template <class T> struct alignas(16) FaceRec {
 };
 static_assert(sizeof(FaceRec<float>) == kFaceT * 4 && sizeof(FaceRec<double>) == kFaceT * 8, "FaceRec");
 
+template <class T> KBG_D Tile2D bufs(const Solve2D& S) { return tile2d_at(S.tile, S.nx, S.ny, S.nv, sizeof(T)); }
+
 template <class T> KBG_D T nl_of(double lam);
 template <> KBG_D float nl_of<float>(double lam) { return float(-lam * 1.4426950408889634074); }
 template <> KBG_D double nl_of<double>(double lam) { return -lam; }
@@ -110,8 +112,9 @@ template <class T, int FLUX> KBG_D void face_chain(const Solve2D& S, int b) {
     const double n1 = geo[0], n2 = geo[1], len = geo[2], dt = S.dt;
     const double* d = dir == 0 ? S.dx : S.dy;
     const double dxL = 0.5 * d[cL], dxR = 0.5 * d[cR];
-    FaceRec<T>& o = ((FaceRec<T>*)(dir == 0 ? S.xrec : S.yrec))[fi];
-    double* fr = (dir == 0 ? S.xfrec : S.yfrec) + (size_t)fi * 8;
+    const Tile2D B = bufs<T>(S);
+    FaceRec<T>& o = ((FaceRec<T>*)(dir == 0 ? B.xrec : B.yrec))[fi];
+    double* fr = (dir == 0 ? B.xfrec : B.yfrec) + (size_t)fi * 8;
     o.r = T(1.0 / (0.5 * (d[cL] + d[cR])));
     o.s[0].d = T(dxL);
     o.s[1].d = T(-dxR);
@@ -279,7 +282,7 @@ template <class T> KBG_D void wall2d(const Solve2D& S, int dir, int fi, int side
         fwout[1] = l1 * n1 - l2 * n2;
         fwout[2] = l1 * n2 + l2 * n1;
         fwout[3] = (0.5 * m3 + 0.5 * m4) * len * dt;
-        if (del) (dir == 0 ? S.xcref : S.ycref)[fi] = len * dt;
+        if (del) S.cref[(dir == 0 ? 0 : size_t(S.nx + 1) * S.ny) + fi] = len * dt;
     }
 }
 
@@ -604,7 +607,8 @@ KBG_D void tile_march(const Solve2D& S, int i0, int j0, int j1, int iv, bool liv
 // tile column ends at the last cell, where nx is no multiple of kTX overlapping its neighbour (both compute
 // the shared cells, with the same results).
 template <class T, int FLUX, bool KEEP>
-__global__ __launch_bounds__(256, sizeof(T) == 4 ? 4 : 2) void k_tile2d(const Solve2D* __restrict__ solves, const int* __restrict__ tstart, int nsolves) {
+__global__ __launch_bounds__(256, sizeof(T) == 4 ? 4 : 2) void k_tile2d(const Solve2D* __restrict__ solves, const int* __restrict__ tstart, int nsolves,
+                                                                                int ty) {
     // face records of the tile (x-faces i0 - 1 .. i0 + kTX + 1 of its rows, y-faces of rows j0 - 1 .. j1 + 1), 1 / (dx dy),
     // sums [4 wavefronts][rows][kTX pairs of faces][64]
     extern __shared__ double tile_lds[];
@@ -612,7 +616,8 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 4 : 2) void k_tile2d(const So
     if (g >= tstart[nsolves]) return;
     const int si = owner(tstart, nsolves, g);
     const Solve2D& S = solves[si];
-    const int nx = S.nx, ny = S.ny, nv = S.nv, ty = S.ty;
+    const int nx = S.nx, ny = S.ny, nv = S.nv;
+    const Tile2D B = bufs<T>(S);
     const int ntx = (nx + kTX - 1) / kTX, nty = (ny + ty - 1) / ty;
     const int b = g - tstart[si], tile = b % (ntx * nty), chunk = b / (ntx * nty);
     const int i0 = min(tile % ntx * kTX, nx - kTX), j0 = tile / ntx * ty, j1 = min(j0 + ty, ny);
@@ -630,17 +635,17 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 4 : 2) void k_tile2d(const So
             const int rec = k / P, part = k % P;
             if (rec < nX) {
                 const int r = rec / (kTX + 3), i = min(max(i0 + rec % (kTX + 3) - 1, 0), nx);
-                ((uint4*)XR)[k] = ((const uint4*)S.xrec)[((size_t)i + size_t(nx + 1) * (j0 + r)) * P + part];
+                ((uint4*)XR)[k] = ((const uint4*)B.xrec)[((size_t)i + size_t(nx + 1) * (j0 + r)) * P + part];
             } else {
                 const int q = rec - nX, j = min(max(j0 - 1 + q / kTX, 0), ny);
-                ((uint4*)YR)[q * P + part] = ((const uint4*)S.yrec)[((size_t)(i0 + q % kTX) + size_t(nx) * j) * P + part];
+                ((uint4*)YR)[q * P + part] = ((const uint4*)B.yrec)[((size_t)(i0 + q % kTX) + size_t(nx) * j) * P + part];
             }
         }
-        for (int k = tid; k < rows * kTX; k += 256) RD[k] = ((const T*)S.rds)[i0 + k % kTX + nx * (j0 + k / kTX)];
+        for (int k = tid; k < rows * kTX; k += 256) RD[k] = ((const T*)B.rds)[i0 + k % kTX + nx * (j0 + k / kTX)];
     }
     __syncthreads();
     if (chunk * 256 + wave * 64 < nv) {
-        const int iv0 = chunk * 256 + tid, iv = S.vperm[min(iv0, nv - 1)];
+        const int iv0 = chunk * 256 + tid, iv = B.vperm[min(iv0, nv - 1)];
         const T u = ((const T*)S.u)[iv], v = ((const T*)S.v)[iv];
         const unsigned long long bx = __ballot(u >= T(0)), by = __ballot(v >= T(0));
         const bool mixed = (bx != 0ull && ~bx != 0ull) || (by != 0ull && ~by != 0ull), live = iv0 < nv;
@@ -666,7 +671,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? 4 : 2) void k_tile2d(const So
             for (int g8 = 0; g8 < 8; g8++) q += p[g8 * 8];
         }
         const size_t f = ydir ? FX + (i0 + t) + size_t(nx) * j : size_t(i0 + t) + size_t(nx + 1) * j;
-        S.psum[(size_t(chunk) * F + f) * 4 + m] = q;
+        B.psum[(size_t(chunk) * F + f) * 4 + m] = q;
     }
 }
 
@@ -696,16 +701,17 @@ __global__ __launch_bounds__(256) void k_chain2d(const Solve2D* __restrict__ sol
     const bool xf = fc < 2;
     const int fi = fc == 0 ? i + (nx + 1) * j : fc == 1 ? i + 1 + (nx + 1) * j : fc == 2 ? i + nx * j : i + nx * (j + 1);
     const bool wall = fc == 0 ? i == 0 : fc == 1 ? i == nx - 1 : fc == 2 ? j == 0 : j == ny - 1;
-    const double* fr = (xf ? S.xfrec : S.yfrec) + (size_t)fi * 8;
+    const Tile2D B = bufs<T>(S);
+    const double* fr = (xf ? B.xfrec : B.yfrec) + (size_t)fi * 8;
     const double* geo = (xf ? S.xgeo : S.ygeo) + (size_t)fi * 3;
     const double n1 = geo[0], n2 = geo[1];
     double q = 0.0, cf;
     if (wall) {
         q = (xf ? S.xfw : S.yfw)[(size_t)fi * 4 + m];
-        cf = del ? (xf ? S.xcref : S.ycref)[fi] : 0.0;
+        cf = del ? S.cref[(xf ? 0 : FX) + fi] : 0.0;
     } else {
         cf = fr[4];
-        const double* ps = S.psum + ((xf ? size_t(fi) : FX + fi)) * 4 + m;
+        const double* ps = B.psum + ((xf ? size_t(fi) : FX + fi)) * 4 + m;
         const int nch = (S.nv + 255) / 256;
 #pragma unroll 4
         for (int k = 0; k < nch; k++) q += ps[size_t(k) * F * 4];
@@ -725,7 +731,7 @@ __global__ __launch_bounds__(256) void k_chain2d(const Solve2D* __restrict__ sol
     const double fw = wall ? q : m == 1 ? q * n1 - o * n2 : (m == 2 ? o * n2 + q * n1 : q);
     if (act && keep && !wall && (fc == 0 || fc == 2)) {
         (xf ? S.xfw : S.yfw)[(size_t)fi * 4 + m] = fw;
-        if (del && m == 0) (xf ? S.xcref : S.ycref)[fi] = cf;
+        if (del && m == 0) S.cref[(xf ? 0 : FX) + fi] = cf;
     }
     const double ds = S.dx[c] * S.dy[c];
     // sum over the faces of a quantity of this lane's moment: L - R + D - U
@@ -743,7 +749,7 @@ __global__ __launch_bounds__(256) void k_chain2d(const Solve2D* __restrict__ sol
     if (!act) return;
     if ((lane & 15) == 0) {
         flag_health(S.health, prim_health<4>(pn));
-        CellRec<T>& k = ((CellRec<T>*)S.crec)[c];
+        CellRec<T>& k = ((CellRec<T>*)B.crec)[c];
         k.rT = T(r);
         k.inv = T(1.0 / (1.0 + r));
         k.An = T(pn[0] * (pn[3] / kPi));
@@ -798,7 +804,8 @@ __global__ __launch_bounds__(256, NEXT || KEEP ? 4 : 6) void k_relax2d(const Sol
     const T* __restrict__ G = (const T*)(i > 0 ? S.xff : S.yff) + (size_t)g_face(nx, i, j) * 2 * nv;
     const T* __restrict__ xl = (const T*)S.xff + (size_t)(i + (nx + 1) * j) * 2 * nv;
     const T* __restrict__ yd = (const T*)S.yff + (size_t)(i + nx * j) * 2 * nv;
-    const T rds = KEEP ? ((const T*)S.rds)[c] : T(0);
+    const Tile2D B = bufs<T>(S);
+    const T rds = KEEP ? ((const T*)B.rds)[c] : T(0);
     T* h = (T*)S.f + (size_t)c * 2 * nv;
     auto g_of = [&](int o) {
         if constexpr (KEEP) {
@@ -812,7 +819,7 @@ __global__ __launch_bounds__(256, NEXT || KEEP ? 4 : 6) void k_relax2d(const Sol
     const T* __restrict__ U = (const T*)S.u;
     const T* __restrict__ V = (const T*)S.v;
     const float* __restrict__ R = S.mref;
-    const CellRec<T> K = ((const CellRec<T>*)S.crec)[c];
+    const CellRec<T> K = ((const CellRec<T>*)B.crec)[c];
     for (int v0 = wall ? 0 : (b - nw) % per * 1024; v0 < nv; v0 += 1024) {
         T gh[VPT], gb[VPT], u[VPT], v[VPT], rh[VPT], rb[VPT];
 #pragma unroll
@@ -877,8 +884,8 @@ static hipError_t launch_tile_t(int ty, const Solve2D* d_solves, const int* d_pr
     const bool share = totals[3] <= 32768;
     if (first || !share) hipLaunchKernelGGL((k_pre2d<T, FLUX>), dim3(totals[0]), dim3(256), 0, st, d_solves, d_pref, n);
     const size_t lds = tile2d_lds<T>(ty);
-    if (last) hipLaunchKernelGGL((k_tile2d<T, FLUX, true>), dim3(totals[1]), dim3(256), lds, st, d_solves, d_pref + (n + 1), n);
-    else hipLaunchKernelGGL((k_tile2d<T, FLUX, false>), dim3(totals[1]), dim3(256), lds, st, d_solves, d_pref + (n + 1), n);
+    if (last) hipLaunchKernelGGL((k_tile2d<T, FLUX, true>), dim3(totals[1]), dim3(256), lds, st, d_solves, d_pref + (n + 1), n, ty);
+    else hipLaunchKernelGGL((k_tile2d<T, FLUX, false>), dim3(totals[1]), dim3(256), lds, st, d_solves, d_pref + (n + 1), n, ty);
     hipLaunchKernelGGL(k_chain2d<T>, dim3((totals[2] + 15) / 16), dim3(256), 0, st, d_solves, d_pref + 2 * (n + 1), n, rows, last);
     const dim3 gr(totals[3]), b(256);
     const int* rstart = d_pref + 3 * (n + 1);

@@ -17,6 +17,8 @@
 
 namespace kbg {
 
+// A batch stages one descriptor per solve, in kbg_batch_step_noalloc's fixed array: growing one lowers the number
+// of solves that fit there (kbg_api.hip asserts the sizes).
 struct Solve1D {
     int nx, ng, nv, nf, vdim, nw;
     int flux, coll, limiter, interp2;
@@ -48,15 +50,18 @@ struct Solve1D {
     const double* bcprim;                          // [2][nw]  wall primitive vectors
     const void* vtab;                              // [nv + 8] per-velocity constants (swept path)
     int* health;                                   // failure flags (kbg_device.h prim_health)
-    const double* fsmq;                            // collision :fsm: Q of the cells fsm_c0 .. [ncell][nv]
+    union {
+        const double* fsmq;                        // collision :fsm (1D1F3V): Q of the cells fsm_c0 .. [ncell][nv]
+        double* psum;                              // swept solves: k_split1d's moment sums of two steps, or NULL
+    };
     int fsm_c0;                                    // first physical cell of fsmq
-    double* psum;                                  // k_split1d: moment sums of two steps (kbg_split1d.hip; or NULL)
 };
 
 struct Solve2D {
     int nx, ny, nv;
     int flux, coll, limiter, interp2;
     int bc[4];                                     // left, right, down, up: 0 fix, 1 Maxwell
+    int delta;                                     // f holds departures (below)
     double K, gam, mu, om, Pr, dt;
     const double* dx;                              // [nx*ny]
     const double* dy;
@@ -85,21 +90,10 @@ struct Solve2D {
     // FP32 solves of the fused step store f - Mr, Mr a per-solve reference Maxwellian (h and b), and
     // the face fluxes of the fused step without Mr's part c x Mr, where x is the normal velocity and c
     // the face's coefficient of the distribution in its flux (0 for a stored :fix face)
-    int delta;
     const float* mref;                             // [2][nv] Mr (h, b) as stored in FP32
     double mmom[11];                               // sum w u^a v^b Mr_h: (a,b) = 10 01 20 11 02 30 21 12 03; Mr_b: 10 01
-    double* xcref;                                 // [(nx+1)*ny] c of each x-face
-    double* ycref;                                 // [nx*(ny+1)]
-    // the tiled step (kbg_tile2d.hip; NULL where the solve does not take it)
-    int ty;                                        // rows per tile
-    const void* rds;                               // [nx*ny] 1 / (dx dy), storage type
-    void* xrec;                                    // [(nx+1)*ny][kFaceT] interior faces' flux coefficients
-    void* yrec;                                    // [nx*(ny+1)][kFaceT]
-    double* xfrec;                                 // [(nx+1)*ny][8] fw0 len, Mr's coefficient, n1, n2
-    double* yfrec;                                 // [nx*(ny+1)][8]
-    double* psum;                                  // [chunks of 256 velocities][faces][4] moment sums
-    void* crec;                                    // [nx*ny][kCellT] relaxation coefficients, storage type
-    const int* vperm;                              // [nv] velocities sorted by the signs of v and u
+    double* cref;                                  // [(nx+1)*ny + nx*(ny+1)] c of each x-face, then each y-face
+    void* tile;                                    // the tiled step's buffers (Tile2D; NULL where the solve does not take it)
 };
 
 // An unstructured triangle solve (2D1F2V / 2D2F2V, KFVS): faces with their two cells, normal (from
@@ -147,6 +141,30 @@ constexpr int kUCellT = 16;
 constexpr int kFaceT = 24;
 constexpr int kCellT = 16;
 constexpr int kTile2dX = 4, kTile2dRows = 6;
+// The tiled step's buffers (kbg_tile2d.hip), one after another in Solve2D::tile
+struct Tile2D {
+    char *xrec, *yrec;      // [(nx+1)*ny], [nx*(ny+1)][kFaceT] interior faces' flux coefficients, storage type
+    double *xfrec, *yfrec;  // [..][8] fw0 len, Mr's coefficient, n1, n2
+    double* psum;           // [chunks of 256 velocities][faces][4] moment sums
+    char* crec;             // [nx*ny][kCellT] relaxation coefficients, storage type
+    char* rds;              // [nx*ny] 1 / (dx dy), storage type
+    int* vperm;             // [nv] velocities sorted by the signs of v and u
+    char* end;
+};
+inline __host__ __device__ Tile2D tile2d_at(void* tile, int nx, int ny, int nv, int esz) {
+    const size_t FX = size_t(nx + 1) * ny, FY = size_t(nx) * (ny + 1), C = size_t(nx) * ny;
+    Tile2D t;
+    t.xrec = (char*)tile;
+    t.yrec = t.xrec + FX * kFaceT * esz;
+    t.xfrec = (double*)(t.yrec + FY * kFaceT * esz);
+    t.yfrec = t.xfrec + FX * 8;
+    t.psum = t.yfrec + FY * 8;
+    t.crec = (char*)(t.psum + size_t((nv + 255) / 256) * (FX + FY) * 4);
+    t.rds = t.crec + C * kCellT * esz;
+    t.vperm = (int*)(t.rds + C * esz);
+    t.end = (char*)(t.vperm + nv);
+    return t;
+}
 // Threads per workgroup of the fused 2D step (one face or cell per workgroup): 64 ceil(nv / 256), 4
 // velocities per thread, at most 1024 in FP32 and 512 in FP64 (the register budget of an FP64
 // thread); 0 when the velocity grid is larger (the phase kernels then step the solve)

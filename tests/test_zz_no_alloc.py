@@ -93,3 +93,34 @@ def test_noalloc_refusals(gpu_ctx):
         gpu_ctx.set_schedule(seg, streams)
     for r in runs + ref + big:
         r[4].close()
+
+
+def test_a_solve_takes_no_more_of_the_staging_array(gpu_ctx):
+    """The 8 MiB hold as many solves as they did when a 1D descriptor had 344 bytes and a 2D one 408 beside three
+    prefix sums: what a refused batch says it needs grows by no more per solve (each of the six arrays is rounded
+    up to 256 bytes).  256 1D solves of two work items each (112 bytes an item, 16 per pack of four), and 32 2D
+    solves of the tiled step."""
+    import re
+
+    big = _solves([kb.configs.riemann_1d1f1v(dict(kb.configs.batch_instances(1)[0], nx=2048, nu=32))] * 40, gpu_ctx)
+    one = _solves([kb.configs.sod_1d1f1v(nx=4, nu=8)], gpu_ctx)[0]
+    tubes = [one] + [(*one[:4], kb.DeviceSolve(one[0], one[1], one[2], "fp32", gpu_ctx)) for _ in range(255)]
+    cav = _solves([kb.configs.cavity_2d2f2v(nx=20, ny=20, nu=16, nv=16)] * 32, gpu_ctx)
+    seg, streams = gpu_ctx.schedule()
+    gpu_ctx.set_schedule(1, 1)
+    gpu_ctx.set_sweep_vw(64)
+
+    def need(runs):
+        with pytest.raises(kb._lib.KbgError, match="staging") as e:
+            _call(gpu_ctx, "kbg_batch_step_noalloc", runs, 1, False)
+        return int(re.search(r"needs (\d+) bytes", str(e.value))[1])
+
+    try:
+        n0 = need(big)
+        assert need(big + tubes) - n0 <= 256 * (344 + 2 * 112) + 128 * 16 + 6 * 256
+        assert need(big + cav) - n0 <= 32 * (408 + 12) + 12 + 6 * 256
+    finally:
+        gpu_ctx.set_sweep_vw(0)
+        gpu_ctx.set_schedule(seg, streams)
+    for r in big + tubes + cav:
+        r[4].close()
