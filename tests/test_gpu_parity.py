@@ -793,6 +793,43 @@ def test_split_sweep_equals_the_sweep(gpu_ctx, space, flux, collision, nv):
         gpu_ctx.set_sweep_vw(0)
 
 
+@pytest.mark.parametrize("seg", [60, 20])
+def test_split_sweep_in_batches(gpu_ctx, seg):
+    """k_split1d with several solves per launch, of 7, 64 and 128 velocities (grid rows of the shorter ones left
+    empty) and both fluxes, with whole and with shortened segments: the bits a solve has alone with the sweep, also
+    beside a solve that takes the batch past the split's 1024 wavefronts."""
+    made = []
+    for nx, nv, flux in ((61, 7, "ugks"), (30, 64, "kcu"), (130, 128, "ugks"), (64, 64, "ugks"), (3700, 128, "ugks")):
+        ks = kb.SolverSet(kb.configs.shock_1d2f1v(nx=nx, nu=nv, flux=flux, vMeshType="rectangle"))
+        ctr, face = kb.init_fvm(ks)
+        ctr.f *= 1.0 + 0.01 * np.random.default_rng(nx).random(ctr.f.shape)
+        made.append((ks, ctr, face, kb.timestep(ks, ctr)))
+
+    def run(group):
+        devs = [kb.DeviceSolve(ks, ctr, face, "fp64", gpu_ctx) for ks, ctr, face, dt in group]
+        kb.batch_step(devs, [m[3] for m in group], 5, ctx=gpu_ctx)
+        out = [copy.deepcopy(m[1]) for m in group]
+        for d, c in zip(devs, out):
+            d.download(c)
+            d.close()
+        return out
+
+    cells, streams = gpu_ctx.schedule()
+    try:
+        gpu_ctx.set_sweep_vw(64)
+        ref = [run([m])[0] for m in made[:4]]
+        gpu_ctx.set_sweep_vw(0)
+        gpu_ctx.set_schedule(seg, streams)
+        for got in ([run([m])[0] for m in made[:4]], run(made[:4]), run(made)[:4]):
+            for g, r in zip(got, ref):
+                np.testing.assert_array_equal(g.f, r.f)
+                np.testing.assert_array_equal(g.w, r.w)
+                np.testing.assert_array_equal(g.prim, r.prim)
+    finally:
+        gpu_ctx.set_sweep_vw(0)
+        gpu_ctx.set_schedule(cells, streams)
+
+
 @pytest.mark.parametrize("space,flux", [("2d2f2v", "ugks"), ("2d2f2v", "kcu"), ("2d2f2v", "kfvs"), ("2d1f2v", "kfvs")])
 @pytest.mark.parametrize("nu,nv", [(9, 7), (8, 8), (13, 5), (16, 16), (13, 20), (24, 24), (17, 33)])
 def test_phase_calls_at_the_edges_of_their_workgroups(gpu_ctx, space, flux, nu, nv):
