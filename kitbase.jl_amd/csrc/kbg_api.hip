@@ -770,14 +770,15 @@ int sync_boundary_faces(kbg_solve* s) {
 }
 
 // segments of the stepped cells, in order along x (neighbouring segments share halo rows)
-void build_items(kbg_solve* s, int seg, int solve_index, int nw, std::vector<WorkItem>& out) {
+void build_items(kbg_solve* s, int seg, int solve_index, int nw, int gch, std::vector<WorkItem>& out) {
     const Solve1D& S = s->h1;
     for (int c0 = S.upd_lo; c0 <= S.upd_hi; c0 += seg) {
         WorkItem wi;
         wi.solve = solve_index;
         wi.c0 = c0;
         wi.c1 = std::min(c0 + seg - 1, S.upd_hi);
-        wi.nw = nw;
+        wi.nw = short(nw);
+        wi.gch = short(gch);
         out.push_back(wi);
     }
 }
@@ -1944,14 +1945,29 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
     // A solve's results do not depend on the width (kbg_sweep.h), so the rule may look at the whole batch.
     // A cap of 16 or 32 velocities per wavefront sets the order of a solve's sums too, that of k_sweep1d's
     // wavefronts under it, whichever kernel steps it; with a cap of 8 solves that may take the narrow sweep add in
-    // the full width's order and take the full width in large batches.  Under the cap of 16 the other side is
-    // k_sweep1d at 16 velocities, us per step it / narrow: n = 16 14.8 / 10.2, 32 17.9 / 18.3, 48 23.3 / 27.1.
-    constexpr long kNarrowWaves = 2700, kNarrowWavesCap = 1600;
+    // the full width's order and take the full width in large batches.
     const int sum_cap = ctx->sweep_vw == 16 || ctx->sweep_vw == 32 ? ctx->sweep_vw : 0;
+    // FP64, two distributions and many velocities each make the narrow passes dearer against the full ones
+    // (narrow_weight).  us per step, full / narrow, solves of 2000 cells, at k wavefronts: FP32 2F 128 velocities 1.7 k
+    // 17.7 / 16.2, 2.2 k 18.9 / 20.2; FP64 1F 64 velocities 1.8 k 18.8 / 18.2, 2.6 k 21.6 / 25.2, 128 velocities 1.3 k
+    // 17.9 / 16.0, 1.7 k 18.4 / 20.0, 2.6 k 21.6 / 29.7; FP64 2F 32 velocities 1.4 k 17.2 / 16.7, 1.8 k 18.3 / 19.0, 64
+    // velocities 0.9 k 16.5 / 16.4, 2.6 k 21.5 / 25.3, 128 velocities 0.6 k 17.0 / 17.7, 2.6 k 24.3 / 29.0.
+    // Under the cap of 16 the other side is k_sweep1d at 16 velocities, us per step it / narrow: n tubes of the kind
+    // above 16 14.9 / 10.7, 28 16.2 / 16.9, 40 19.7 / 24.1; FP32 64 velocities 1.8 k 16.8 / 13.8, 2.6 k 23.0 / 18.9, 128
+    // velocities 2.6 k 23.1 / 20.2, 250 velocities 1.3 k 15.1 / 13.2, 1.7 k 17.0 / 16.4; FP64 64 velocities 2.6 k 24.2 / 19.4,
+    // 250 velocities 1.7 k 19.8 / 19.0, 2.6 k 23.1 / 23.8, but 64 velocities 0.9 k 11.8 / 12.8, 128 velocities 0.9 k 12.3 / 15.1.
+    constexpr long kNarrowWaves = 27000;  // weighted, in tenths
+    auto narrow_weight = [&](const kbg_solve* s) -> long {
+        const int nv = s->d.nv;
+        if (sum_cap) return nv <= 128 ? 10 : s->fp64 ? 12 : 22;
+        if (!s->fp64) return s->d.nf == 2 && nv > 64 ? 14 : 10;
+        if (s->d.nf == 1) return nv > 64 ? 18 : 14;
+        return nv > 64 ? 65 : nv > 32 ? 30 : 18;
+    };
     long waves0 = 0;
     for (int i : fused) {
         const Solve1D& S = solves[i]->h1;
-        waves0 += long(S.upd_hi - S.upd_lo + kbg::sweep_out(2)) / kbg::sweep_out(2) * solves[i]->sweep_nw;
+        waves0 += long(S.upd_hi - S.upd_lo + kbg::sweep_out(2)) / kbg::sweep_out(2) * solves[i]->sweep_nw * narrow_weight(solves[i]);
     }
     std::vector<int> narrow_nw(n, 0);  // wavefronts per item of the narrow sweep, 0: k_sweep1d
     std::vector<int> wide_nw(n, 0);    // and of k_sweep1d: the kernel's width, or more under a cap
@@ -1960,7 +1976,7 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
         const int nv = s->d.nv, most = kbg::sweep_vw_narrow(s->d.nf);
         const bool may = s->d.flux == KBG_KFVS && nv <= kbg::kSweepNarrowWaves * most && ctx->sweep_vw <= most;
         wide_nw[i] = kbg::sweep_cap_nw(s->fp64, s->d.nf, nv, may ? sum_cap : ctx->sweep_vw);
-        if (!may || waves0 > (sum_cap ? kNarrowWavesCap : kNarrowWaves)) continue;
+        if (!may || waves0 > kNarrowWaves || (sum_cap && s->fp64 && nv <= 128 && waves0 < 15000)) continue;
         const int vw = ctx->sweep_vw > 0 ? ctx->sweep_vw : kbg::kVChunk;
         int nw = 1;
         while (nw < kbg::kSweepNarrowWaves && kbg::sweep_item_vw(nv, nw) > vw) nw *= 2;
@@ -2073,7 +2089,7 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
                 if (!split[i]) L.narrow = std::max(L.narrow, nw);
                 L.rows = std::max(L.rows, (s->d.nv + kbg::kVChunk - 1) / kbg::kVChunk);
             }
-            build_items(s, seg_of(i), desc_of[i], nw, items);
+            build_items(s, seg_of(i), desc_of[i], nw, kbg::sweep_item_vw(s->d.nv, wide_nw[i]) / kbg::kVChunk, items);
             for (size_t it = i0; it < items.size(); it++) by_nw[nw].push_back((int)it);
             L.wg_waves = std::max(L.wg_waves, nw);
         }
@@ -2236,7 +2252,7 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
                 } else if (L.narrow) {
                     double* rp = keep ? d_rpart + L.item0 * 12 : nullptr;
                     HIPCHK((L.fp64 ? kbg::launch_sweep1d_narrow64 : kbg::launch_sweep1d_narrow32)(
-                        L.nf, L.narrow, L.rows, d_descs, d_items + L.item0, (int)L.nitems, par, sum_cap, rp, per, sst[L.stream]));
+                        L.nf, L.narrow, L.rows, d_descs, d_items + L.item0, (int)L.nitems, par, rp, per, sst[L.stream]));
                 } else {
                     HIPCHK(kbg::launch_sweep1d(L.fp64, L.nf, L.flux, L.wg_waves, d_descs, d_items, d_packs + L.pack0, (int)L.npacks,
                                                par, keep ? d_rpart : nullptr, per, sst[L.stream]));
@@ -2298,7 +2314,6 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
         auto put = [&](const void* p, size_t b) { sig.append(static_cast<const char*>(p), b); };
         auto puti = [&](long long v) { put(&v, sizeof v); };
         puti(nstreams);
-        puti(sum_cap);
         const void* bufs[] = {d_descs, d_items, d_packs, d_descs2, d_pref2};
         put(bufs, sizeof bufs);
         for (Solve1D d : descs) {

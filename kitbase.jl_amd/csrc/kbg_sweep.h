@@ -211,9 +211,9 @@ template <class T> struct SFace {
 //
 // VW: most velocities per wavefront.  NARROW (small launches, k_sweep1d_narrow): more wavefronts per item
 // than k_sweep1d takes, and every chunk's sums get an LDS row of their own, which wavefront 0 adds in the
-// order of the chunk sums of k_sweep1d's sweep_cap_nw(.., cap) wavefronts -- the same values whatever the width.
+// order of k_sweep1d's wavefronts (groups of wi.gch chunks) -- the same values whatever the width.
 template <class T, int NF, int FLUX, int LIMK, bool SHAK, int NSTEP, int VW, bool NARROW>
-KBG_D void sweep1d(const Solve1D& S, const WorkItem& wi, int par, int cap, int lane, int wave, int NW, double* lds,
+KBG_D void sweep1d(const Solve1D& S, const WorkItem& wi, int par, int lane, int wave, int NW, double* lds,
                    double* rrow) {
     static_assert(NSTEP == 1 || FLUX == KFVS, "several steps per pass are built for KFVS");
     using C = SweepCfg<T, NF, FLUX>;
@@ -541,21 +541,40 @@ KBG_D void sweep1d(const Solve1D& S, const WorkItem& wi, int par, int cap, int l
             double tot[NR];
             if constexpr (NARROW) {
                 // chunk by chunk within the velocities of one of k_sweep1d's wavefronts, then these in order
-                const int gch = sweep_item_vw(nv, sweep_cap_nw(sizeof(T) == 8, NF, nv, cap)) / CH, nch = (nv + CH - 1) / CH;
+                const int gch = wi.gch, nch = (nv + CH - 1) / CH;
                 double a[NR];
 #pragma unroll
                 for (int m = 0; m < NR; m++) tot[m] = a[m] = 0.0;
-                for (int c0 = 0; c0 < nch; c0 += gch) {
-                    const int c1 = min(nch, c0 + gch);
+                // groups of two chunks (FP32 under a cap of 16, FP64 with two distributions): two groups' loads in
+                // flight
+                constexpr bool PAIRS = (NF == 2) == (sizeof(T) == 8);
+                if (PAIRS && gch == 2) {
+                    for (int c0 = 0; c0 < nch; c0 += 4) {
+                        double v[4][NR];
 #pragma unroll
-                    for (int m = 0; m < NR; m++) a[m] = 0.0;
-#pragma unroll 4
-                    for (int c = c0; c < c1; c++) {
+                        for (int k = 0; k < 4; k++)
 #pragma unroll
-                        for (int m = 0; m < NR; m++) a[m] += lds[(c * NR + m) * kSweepLanes + lane];
+                            for (int m = 0; m < NR; m++) v[k][m] = lds[(min(c0 + k, nch - 1) * NR + m) * kSweepLanes + lane];
+#pragma unroll
+                        for (int k = 0; k < 4; k += 2) {
+                            if (c0 + k >= nch) break;
+#pragma unroll
+                            for (int m = 0; m < NR; m++) tot[m] += c0 + k + 1 < nch ? v[k][m] + v[k + 1][m] : v[k][m];
+                        }
                     }
+                } else {
+                    for (int c0 = 0; c0 < nch; c0 += gch) {
+                        const int c1 = min(nch, c0 + gch);
 #pragma unroll
-                    for (int m = 0; m < NR; m++) tot[m] += a[m];
+                        for (int m = 0; m < NR; m++) a[m] = 0.0;
+#pragma unroll 4
+                        for (int c = c0; c < c1; c++) {
+#pragma unroll
+                            for (int m = 0; m < NR; m++) a[m] += lds[(c * NR + m) * kSweepLanes + lane];
+                        }
+#pragma unroll
+                        for (int m = 0; m < NR; m++) tot[m] += a[m];
+                    }
                 }
             } else if (NW > 1) {
 #pragma unroll
@@ -837,15 +856,15 @@ KBG_D void sweep1d(const Solve1D& S, const WorkItem& wi, int par, int cap, int l
 }
 
 template <class T, int NF, int FLUX, int LIMK, int NSTEP, int VW, bool NARROW>
-KBG_D void sweep_coll(const Solve1D& S, const WorkItem& wi, int par, int cap, int lane, int wave, int NW, double* lds, double* rrow) {
-    if (S.coll == SHAKHOV) sweep1d<T, NF, FLUX, LIMK, true, NSTEP, VW, NARROW>(S, wi, par, cap, lane, wave, NW, lds, rrow);
-    else sweep1d<T, NF, FLUX, LIMK, false, NSTEP, VW, NARROW>(S, wi, par, cap, lane, wave, NW, lds, rrow);
+KBG_D void sweep_coll(const Solve1D& S, const WorkItem& wi, int par, int lane, int wave, int NW, double* lds, double* rrow) {
+    if (S.coll == SHAKHOV) sweep1d<T, NF, FLUX, LIMK, true, NSTEP, VW, NARROW>(S, wi, par, lane, wave, NW, lds, rrow);
+    else sweep1d<T, NF, FLUX, LIMK, false, NSTEP, VW, NARROW>(S, wi, par, lane, wave, NW, lds, rrow);
 }
 template <class T, int NF, int FLUX, int NSTEP, int VW, bool NARROW>
-KBG_D void sweep_lim(const Solve1D& S, const WorkItem& wi, int par, int cap, int lane, int wave, int NW, double* lds, double* rrow) {
-    if (!S.interp2) sweep_coll<T, NF, FLUX, LIM_NONE, NSTEP, VW, NARROW>(S, wi, par, cap, lane, wave, NW, lds, rrow);
-    else if (S.limiter == VANLEER) sweep_coll<T, NF, FLUX, LIM_VANLEER, NSTEP, VW, NARROW>(S, wi, par, cap, lane, wave, NW, lds, rrow);
-    else sweep_coll<T, NF, FLUX, LIM_GENERIC, NSTEP, VW, NARROW>(S, wi, par, cap, lane, wave, NW, lds, rrow);
+KBG_D void sweep_lim(const Solve1D& S, const WorkItem& wi, int par, int lane, int wave, int NW, double* lds, double* rrow) {
+    if (!S.interp2) sweep_coll<T, NF, FLUX, LIM_NONE, NSTEP, VW, NARROW>(S, wi, par, lane, wave, NW, lds, rrow);
+    else if (S.limiter == VANLEER) sweep_coll<T, NF, FLUX, LIM_VANLEER, NSTEP, VW, NARROW>(S, wi, par, lane, wave, NW, lds, rrow);
+    else sweep_coll<T, NF, FLUX, LIM_GENERIC, NSTEP, VW, NARROW>(S, wi, par, lane, wave, NW, lds, rrow);
 }
 
 // LDS of one item (doubles): the wavefronts' (rows: chunks') moment sums and wavefront 0's cell coefficients
@@ -893,11 +912,11 @@ __global__ __launch_bounds__(64 * kSweepMaxWaves) __attribute__((amdgpu_waves_pe
     constexpr int VW = SweepCfg<T, NF, FLUX>::VW;
     if constexpr (FLUX == KFVS) {
         if (nstep == 2) {
-            sweep_lim<T, NF, FLUX, 2, VW, false>(S, wi, par, 0, lane, wave, NW, lds, rrow);
+            sweep_lim<T, NF, FLUX, 2, VW, false>(S, wi, par, lane, wave, NW, lds, rrow);
             return;
         }
     }
-    sweep_lim<T, NF, FLUX, 1, VW, false>(S, wi, par, 0, lane, wave, NW, lds, rrow);
+    sweep_lim<T, NF, FLUX, 1, VW, false>(S, wi, par, lane, wave, NW, lds, rrow);
 }
 
 // The KFVS sweep of small launches: a launch with less than a few wavefronts per SIMD takes as long as one
@@ -909,7 +928,7 @@ __global__ __launch_bounds__(64 * kSweepMaxWaves) __attribute__((amdgpu_waves_pe
 template <class T, int NF>
 __global__ __launch_bounds__(64 * kSweepNarrowWaves) void k_sweep1d_narrow(const Solve1D* __restrict__ solves,
                                                                           const WorkItem* __restrict__ items, int nitems, int par,
-                                                                          int cap, double* __restrict__ rpart, int nstep) {
+                                                                          double* __restrict__ rpart, int nstep) {
     extern __shared__ double kbg_sweep_lds[];
     const int it = blockIdx.x;
     if (it >= nitems) return;
@@ -924,9 +943,9 @@ __global__ __launch_bounds__(64 * kSweepNarrowWaves) void k_sweep1d_narrow(const
     const Solve1D& S = solves[wi.solve];
     double* rrow = rpart ? rpart + (size_t)it * 12 : nullptr;
     constexpr int VW = sweep_vw_narrow(NF);
-    if (nstep == 4) sweep_lim<T, NF, KFVS, 4, VW, true>(S, wi, par, cap, lane, wave, wi.nw, kbg_sweep_lds, rrow);
-    else if (nstep == 2) sweep_lim<T, NF, KFVS, 2, VW, true>(S, wi, par, cap, lane, wave, wi.nw, kbg_sweep_lds, rrow);
-    else sweep_lim<T, NF, KFVS, 1, VW, true>(S, wi, par, cap, lane, wave, wi.nw, kbg_sweep_lds, rrow);
+    if (nstep == 4) sweep_lim<T, NF, KFVS, 4, VW, true>(S, wi, par, lane, wave, wi.nw, kbg_sweep_lds, rrow);
+    else if (nstep == 2) sweep_lim<T, NF, KFVS, 2, VW, true>(S, wi, par, lane, wave, wi.nw, kbg_sweep_lds, rrow);
+    else sweep_lim<T, NF, KFVS, 1, VW, true>(S, wi, par, lane, wave, wi.nw, kbg_sweep_lds, rrow);
 }
 
 template <class T, int NF, int FLUX>
@@ -942,10 +961,10 @@ hipError_t launch_sweep_t(int wg_waves, const Solve1D* d_solves, const WorkItem*
 
 // wg_waves: the largest nw of the items; rows: the most velocity chunks of their solves
 template <class T, int NF>
-hipError_t launch_sweep_narrow_t(int wg_waves, int rows, const Solve1D* d_solves, const WorkItem* d_items, int nitems, int par, int cap,
+hipError_t launch_sweep_narrow_t(int wg_waves, int rows, const Solve1D* d_solves, const WorkItem* d_items, int nitems, int par,
                                  double* d_rpart, int nstep, hipStream_t st) {
     const size_t lds = sweep_lds_item<T, NF, KFVS>(wg_waves, rows) * sizeof(double);
-    hipLaunchKernelGGL((k_sweep1d_narrow<T, NF>), dim3(nitems), dim3(64 * wg_waves), lds, st, d_solves, d_items, nitems, par, cap, d_rpart, nstep);
+    hipLaunchKernelGGL((k_sweep1d_narrow<T, NF>), dim3(nitems), dim3(64 * wg_waves), lds, st, d_solves, d_items, nitems, par, d_rpart, nstep);
     return hipGetLastError();
 }
 template <class T, int NF> hipError_t sweep_narrow_attr_t() {

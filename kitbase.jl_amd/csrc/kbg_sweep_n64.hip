@@ -4,9 +4,9 @@
 namespace kbg {
 
 hipError_t launch_sweep1d_narrow64(int nf, int wg_waves, int rows, const Solve1D* d_solves, const WorkItem* d_items, int nitems,
-                                   int par, int cap, double* d_rpart, int nstep, hipStream_t st) {
-    if (nf == 1) return launch_sweep_narrow_t<double, 1>(wg_waves, rows, d_solves, d_items, nitems, par, cap, d_rpart, nstep, st);
-    return launch_sweep_narrow_t<double, 2>(wg_waves, rows, d_solves, d_items, nitems, par, cap, d_rpart, nstep, st);
+                                   int par, double* d_rpart, int nstep, hipStream_t st) {
+    if (nf == 1) return launch_sweep_narrow_t<double, 1>(wg_waves, rows, d_solves, d_items, nitems, par, d_rpart, nstep, st);
+    return launch_sweep_narrow_t<double, 2>(wg_waves, rows, d_solves, d_items, nitems, par, d_rpart, nstep, st);
 }
 
 hipError_t sweep_narrow_attr64() {

@@ -177,7 +177,9 @@ constexpr int step2d_threads(bool fp64, int nv) {
 // One unit of work of the fused 1D sweep: cells [c0, c1] (physical, at most 60) of solve `solve`,
 // updated by nw wavefronts (1, 2, 4 or 8) that split the velocity grid evenly in multiples of 8.
 struct WorkItem {
-    int solve, c0, c1, nw;
+    int solve, c0, c1;
+    short nw;   // wavefronts
+    short gch;  // chunks of 8 velocities per group of the moment sums: those of one of k_sweep1d's wavefronts
 };
 // A workgroup's share of a sweep launch: items item0 .. item0 + count - 1, all with the same nw,
 // packed side by side (count nw <= the launch's wavefronts per workgroup).
@@ -213,14 +215,13 @@ constexpr int sweep_cap_nw(bool fp64, int nf, int nv, int cap) {
     return nw;
 }
 // The narrow KFVS sweep of small launches: nstep 1, 2 or 4, items of nw <= kSweepNarrowWaves wavefronts of at
-// most sweep_vw_narrow velocities, wg_waves the largest nw, rows the most 8-velocity chunks of the solves; the
-// sums run in the order of k_sweep1d's items of sweep_cap_nw(.., cap) wavefronts
+// most sweep_vw_narrow velocities, wg_waves the largest nw, rows the most 8-velocity chunks of the solves
 constexpr int kSweepNarrowWaves = 16;
 constexpr int sweep_vw_narrow(int nf) { return 16 / nf; }
 hipError_t launch_sweep1d_narrow32(int nf, int wg_waves, int rows, const Solve1D* d_solves, const WorkItem* d_items, int nitems,
-                                   int par, int cap, double* d_rpart, int nstep, hipStream_t st);
+                                   int par, double* d_rpart, int nstep, hipStream_t st);
 hipError_t launch_sweep1d_narrow64(int nf, int wg_waves, int rows, const Solve1D* d_solves, const WorkItem* d_items, int nitems,
-                                   int par, int cap, double* d_rpart, int nstep, hipStream_t st);
+                                   int par, double* d_rpart, int nstep, hipStream_t st);
 hipError_t sweep_narrow_attr32();
 hipError_t sweep_narrow_attr64();
 // The FP64 KCU / UGKS step of small launches (kbg_split1d.hip), one step per launch; items of at most kSplitOut

@@ -448,9 +448,9 @@ def test_sweep_velocity_cap(gpu_ctx, vw):
 @pytest.mark.parametrize("precision", ["fp64", "fp32"])
 @pytest.mark.parametrize("vw", [8, 16, 32])
 def test_sweep_velocity_cap_in_a_batch_that_fills_the_chip(gpu_ctx, vw, precision):
-    """Under a velocity cap a solve steps to the same bits alone and beside 40 tubes of 4000 cells, a batch beyond
-    the narrow sweep's rule: one distribution at velocity counts whose capped, uncapped and 8-velocity widths all
-    differ, and two distributions."""
+    """Under a velocity cap a solve steps to the same bits alone, beside 13 tubes of 4000 cells (the narrow sweep in
+    both precisions) and beside 40, a batch beyond the narrow sweep's rule: one distribution at velocity counts whose
+    capped, uncapped and 8-velocity widths all differ, and two distributions."""
     rng = np.random.default_rng(vw)
     cfgs = [kb.configs.sod_1d1f1v(nx=120, nu=nv) for nv in (9, 64, 101, 256)]
     cfgs += [kb.configs.shock_1d2f1v(nx=70, nu=nv, flux="kfvs") for nv in (64, 128)]
@@ -463,19 +463,24 @@ def test_sweep_velocity_cap_in_a_batch_that_fills_the_chip(gpu_ctx, vw, precisio
     try:
         gpu_ctx.set_sweep_vw(vw)
         small, tube = made[:-1], made[-1]
-        batch = [kb.DeviceSolve(ks, ctr, face, precision, gpu_ctx) for ks, ctr, face, dt in small + [tube] * 40]
-        kb.batch_step(batch, [m[3] for m in small + [tube] * 40], 7, ctx=gpu_ctx)
-        for (ks, ctr, face, dt), b in zip(small, batch):
-            alone = kb.DeviceSolve(ks, ctr, face, precision, gpu_ctx)
-            alone.step(dt, 7)
-            ca, cb = copy.deepcopy(ctr), copy.deepcopy(ctr)
-            alone.download(ca)
-            b.download(cb)
-            alone.close()
-            for x, y in ((ca.f, cb.f), (ca.w, cb.w), (ca.prim, cb.prim)):
-                np.testing.assert_array_equal(x, y, err_msg=f"{ks.vs.nv} velocities")
-        for d in batch:
+        alone = []
+        for ks, ctr, face, dt in small:
+            d, c = kb.DeviceSolve(ks, ctr, face, precision, gpu_ctx), copy.deepcopy(ctr)
+            d.step(dt, 7)
+            d.download(c)
             d.close()
+            alone.append(c)
+        for tubes in (13, 40):
+            made = small + [tube] * tubes
+            batch = [kb.DeviceSolve(ks, ctr, face, precision, gpu_ctx) for ks, ctr, face, dt in made]
+            kb.batch_step(batch, [m[3] for m in made], 7, ctx=gpu_ctx)
+            for (ks, ctr, face, dt), ca, b in zip(small, alone, batch):
+                cb = copy.deepcopy(ctr)
+                b.download(cb)
+                for x, y in ((ca.f, cb.f), (ca.w, cb.w), (ca.prim, cb.prim)):
+                    np.testing.assert_array_equal(x, y, err_msg=f"{ks.vs.nv} velocities, {tubes} tubes")
+            for d in batch:
+                d.close()
     finally:
         gpu_ctx.set_sweep_vw(0)
 
