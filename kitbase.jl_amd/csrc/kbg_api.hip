@@ -1880,10 +1880,11 @@ int batch_step_impl(kbg_ctx* ctx, kbg_solve* const* solves, int n, const double*
             Launch2 L{std::get<0>(kv.first) == 1, std::get<1>(kv.first), std::get<2>(kv.first), (int)kv.second.size(), 0, 0, 0,
                       descs2.size(), 0, 0, 0, 0.0, 0, {0, 0, 0, 0}};
             if (std::get<3>(kv.first)) {
-                long one_row = 0;
+                long wgs[kbg::kTile2dRows + 1] = {};
                 for (int i : kv.second)
-                    one_row += long((solves[i]->d.nx + kbg::kTile2dX - 1) / kbg::kTile2dX) * solves[i]->d.ny * ((solves[i]->d.nv + 255) / 256);
-                L.ty = kbg::tile2d_rows(L.fp64, one_row);
+                    for (int k = 1; k <= kbg::kTile2dRows; k++)
+                        wgs[k] += long((solves[i]->d.nx + kbg::kTile2dX - 1) / kbg::kTile2dX) * ((solves[i]->d.ny + k - 1) / k) * ((solves[i]->d.nv + 255) / 256);
+                L.ty = kbg::tile2d_rows(L.fp64, wgs);
                 std::vector<int> p[4] = {{0}, {0}, {0}, {0}};
                 for (int i : kv.second) {
                     kbg_solve* s = solves[i];

@@ -858,16 +858,22 @@ __global__ __launch_bounds__(256, NEXT || KEEP ? 4 : 6) void k_relax2d(const Sol
 
 int pre2d_wgs(int nx, int ny) { return (interior_faces(nx, ny) + 255) / 256 + wall_cells(nx, ny); }
 int relax2d_wgs(int nx, int ny, int nv) { return pre2d_wgs(nx, ny) + (nx * ny - wall_cells(nx, ny)) * ((nv + 1023) / 1024); }
-// Fewer rows repeat the two faces' and slopes' work of the rows around a tile more often, more rows leave too few
-// workgroups to overlap one's waits with another's work; FP32 holds 4 workgroups per CU, and between 3072 and 4096
-// of one row three rows per tile are a few more than the chip holds at once.  us per step at 1 / 2 / 3 / 4 / 6 rows:
-// FP32 UGKS 24 x 24 cells x 16^2 velocities 28 / 30 / 33 / 36 / 41, 45 x 45 x 28^2 53 / 50 / 48 / 51 / 54, 64 x 64 x
-// 24^2 59 / 54 / 58 / 53 / 72, 64 x 64 x 32^2 69 / 61 / 64 / 61 / 74, 100 x 100 x 40^2 247 / 218 / 214 / 218 / 237,
-// 128 x 128 x 48^2 605 / 510 / 496 / 488 / 544; FP64 (2 workgroups per CU) UGKS 64 x 64 x 32^2 121 / 102 / 103 / 95 /
-// 103, 100 x 100 x 40^2 583 / 500 / 464 / 451 / 435.
-int tile2d_rows(bool fp64, long one_row) {
-    if (fp64) return one_row <= 256 ? 1 : one_row <= 1024 ? 2 : one_row <= 3072 ? 3 : one_row <= 12288 ? 4 : 6;
-    return one_row <= 1024 ? 1 : one_row <= 2560 ? 3 : one_row <= 5120 ? 4 : one_row <= 24576 ? 3 : 4;
+// Fewer rows repeat the two faces' and slopes' work of the rows around a tile more often (about 1.6 rows' work per
+// tile), more rows leave too few workgroups to overlap one's waits with another's work.  FP32 holds 4 workgroups per CU
+// (LDS, up to 4 rows): the rows whose rounds of 1024 workgroups times their work come out least.  us per step at 1 / 2 /
+// 3 / 4 rows: UGKS 24 x 24 cells x 16^2 velocities 28 / 30 / 33 / 36, 45 x 45 x 28^2 53 / 50 / 48 / 51, 64 x 64 x 24^2 59 / 54
+// / 58 / 53 (3072 / 1536 / 1056 / 768 workgroups), 64 x 64 x 32^2 69 / 61 / 64 / 61, 100 x 100 x 40^2 247 / 218 / 214 / 218, 128
+// x 128 x 48^2 605 / 510 / 496 / 488.  FP64 (2 workgroups per CU) UGKS at 1 / 2 / 3 / 4 / 6 rows: 64 x 64 x 32^2 121 / 102 /
+// 103 / 95 / 103, 100 x 100 x 40^2 583 / 500 / 464 / 451 / 435.
+int tile2d_rows(bool fp64, const long* wgs) {
+    if (fp64) return wgs[1] <= 256 ? 1 : wgs[1] <= 1024 ? 2 : wgs[1] <= 3072 ? 3 : wgs[1] <= 12288 ? 4 : 6;
+    int best = 1;
+    double least = 0.0;
+    for (int k = 1; k <= 4; k++) {
+        const double cost = double((wgs[k] + 1023) / 1024) * (k + 1.6);
+        if (k == 1 || cost < least) best = k, least = cost;
+    }
+    return best;
 }
 
 // records, 1 / (dx dy) and sums of a tile of ty rows

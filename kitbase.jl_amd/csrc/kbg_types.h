@@ -322,7 +322,7 @@ hipError_t launch_cell2d(bool fp64, int threads, const Solve2D* d_solves, const 
 // face fluxes, moments and coefficients of Mr where the other kernels do
 hipError_t launch_tile2d(bool fp64, int flux, int ty, const Solve2D* d_solves, const int* d_pref, int n, const int* totals, int rows, int first,
                          int last, hipStream_t st);
-int tile2d_rows(bool fp64, long one_row);  // rows per tile for a group of `one_row` workgroups of one row
+int tile2d_rows(bool fp64, const long* wgs);  // rows per tile for a group of wgs[k] workgroups of k rows, k = 1 .. kTile2dRows
 int pre2d_wgs(int nx, int ny);
 int relax2d_wgs(int nx, int ny, int nv);
 hipError_t tile2d_attr();
