@@ -605,12 +605,21 @@ bool split_1d(const kbg_solve* s) {
 // 24^2 velocities (590 k) 26.8 / 29.7, 45 x 28^2 (1.6 M) 42.8 / 42.7, 64 x 24^2 (2.4 M) 53.6 / 50.3; KFVS FP64 64 x 24^2
 // 70.6 / 74.5, 64 x 32^2 (4.2 M) 114 / 77; KCU / UGKS FP32 12 x 16^2 (37 k) 24.4 / 23.7 and 25.3 / 25.9, 24 x 16^2 (147 k)
 // 27.4 / 24.7 and 28.7 / 26.9; FP64 32 x 24^2 40.0 / 42.6 and 44.1 / 48.1, 45 x 28^2 66.7 / 65.0 and 74.9 / 72.8.
+// Within those sizes the tiles lose where their lanes, columns or cells are few: workgroups of 256 velocities with
+// half of them empty (KCU / UGKS FP32 30 x 30 cells x 121 velocities 26.8 / 28.4, 40 x 40 x 64 26.3 / 29.0; KFVS FP64 100 x
+// 100 x 324 96.4 / 107, 90 x 90 x 400 91.8 / 97.9), an overlap of more than half the columns (5 x 400 x 576 FP32 47.5 /
+// 52.4, 5 x 600 x 576 FP64 83 / 94), in FP32 large velocity grids on few cells, whose walls are the step (12 x 12 x 63^2
+// 42.9 / 53.3, 16 x 16 x 48^2 KCU 38.9 / 42.4, 20 x 20 x 63^2 62 / 65, 20 x 20 x 48^2 50.4 / 47.8).
 // The choice is the solve's own: it sums the face moments in another order, and a solve's result must not
 // depend on its batch.
 bool tiled2d(const kbg_desc& d) {
     const bool fp64 = d.precision == KBG_FP64;
     const size_t FX = size_t(d.nx + 1) * d.ny, FY = size_t(d.nx) * (d.ny + 1), work = size_t(d.nx) * d.ny * d.nv;
     if (work < (d.flux == KBG_KFVS ? (fp64 ? 3000000u : 2000000u) : (fp64 ? 1500000u : 100000u))) return false;
+    const size_t full = work / (size_t(d.nv + 255) / 256 * 256) * d.nv;  // weighted by the share of lanes with a velocity
+    if ((fp64 && d.flux == KBG_KFVS && full < 2700000u) || (!fp64 && d.flux != KBG_KFVS && full < 60000u)) return false;
+    if (!fp64 && size_t(d.nx) * d.ny * 6 < size_t(d.nv)) return false;
+    if ((d.nx + kbg::kTile2dX - 1) / kbg::kTile2dX * kbg::kTile2dX * 2 >= d.nx * 3) return false;
     if (kbg::step2d_threads(fp64, d.nv) == 0 || std::max(FX, FY) * 2 * d.nv * (fp64 ? 8 : 4) >= (size_t(1) << 31)) return false;  // thr2 == 0
     if (d.nx < kbg::kTile2dX || d.interp_order != 2 || d.limiter != KBG_VANLEER || d.collision != KBG_BGK) return false;
     for (int b = 0; b < 4; b++)

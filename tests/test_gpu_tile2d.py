@@ -162,3 +162,14 @@ def test_tiled_fp32_moments_are_no_less_accurate_than_the_face_parallel_ones(gpu
         err.append(np.sqrt(np.mean((got.w - ref.w).reshape(-1, 4) ** 2, axis=0)))
     ks.ps.n[0, 0, 1, 0] = n1
     assert np.all(err[0] <= 1.1 * err[1]), (err[0] / err[1])
+
+
+@pytest.mark.parametrize("space,precision,flux,nx,ny,nu,nv", [
+    ("2d2f2v", "fp32", "ugks", 4, 660, 9, 10),  # one tile column, 90 velocities
+    ("2d2f2v", "fp32", "ugks", 61, 64, 8, 8),  # one wavefront, the last column overlapping by three cells
+    ("2d2f2v", "fp32", "kcu", 6, 100, 16, 16),  # two columns, overlapping by two cells
+    ("2d2f2v", "fp64", "kcu", 9, 240, 28, 30),
+])
+def test_tiled_step_on_narrow_meshes_and_few_velocities(gpu_ctx, space, precision, flux, nx, ny, nu, nv):
+    """Sizes next to the edges of the rule that picks the tiles, where their lanes or columns are few."""
+    test_tiled_step_matches_the_oracle_and_the_phases(gpu_ctx, space, precision, flux, nx, ny, nu, nv)
