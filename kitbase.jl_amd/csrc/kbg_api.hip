@@ -587,7 +587,7 @@ long split1d_waves(const Solve1D& S) {
 }
 // most wavefronts of a k_split1d launch: one per SIMD.  Every wavefront of a segment runs its cells' and faces'
 // chains, so the split pays only where the CUs are idle otherwise.  us per step, k_sweep1d / split, 2 distributions:
-// UGKS 30 cells x 16 velocities (2 wavefronts) 22.5 / 14.2, 400 x 101 (91) 35.7 / 19.0, 4000 x 64 (544) 29.5 / 19.0,
+// UGKS 30 cells x 16 velocities (2 wavefronts) 22.5 / 14.2, 400 x 101 (91) 35.7 / 18.5, 4000 x 64 (544) 29.5 / 19.0,
 // 4000 x 101 (884) 38.1 / 22.2; KCU 400 x 101 23.3 / 16.5, 4000 x 64 18.3 / 16.7, 4000 x 101 24.1 / 19.3.
 constexpr long kSplitWaves = 1024;
 
@@ -858,7 +858,6 @@ int kbg_ctx_create(int device, kbg_ctx** out) {
     if (e == hipSuccess) e = hipMalloc((void**)&c->d_res, 4096 * 5 * sizeof(double));
     if (e == hipSuccess) e = kbg::sweep_narrow_attr32();
     if (e == hipSuccess) e = kbg::sweep_narrow_attr64();
-    if (e == hipSuccess) e = kbg::tile2d_attr();
     if (e != hipSuccess) {
         kbg_ctx_destroy(c);
         return fail(KBG_ERR_HIP, std::string("kbg_ctx_create: ") + hipGetErrorString(e));

@@ -14,7 +14,7 @@
 // Every value is formed by k_sweep1d's operations, the sums in its order (chunks of 8 velocities within the
 // velocities of one of its wavefronts, then these), so the results are the same, bit for bit, whichever kernel a
 // batch takes (kbg_api.hip has the rule).  Bound by the latency of the two chains: 400 cells x 101 velocities,
-// h and b, UGKS 35.7 us per step with k_sweep1d, 19.0 here; KCU 23.3 and 16.5.
+// h and b, UGKS + Shakhov 35.7 us per step with k_sweep1d, 18.5 here; KCU 23.3 and 16.5.
 #include "kbg_sweep.h"
 
 namespace kbg {

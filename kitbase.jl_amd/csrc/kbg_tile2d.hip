@@ -24,10 +24,10 @@
 //
 // k_flux2d / k_cell2d (kbg_step2d.hip) keep every face's flux in memory: seven passes over an array of the
 // size of f per step against four here, three loads per face and velocity, and the cell chain between each
-// cell's loads and stores.  us per step there / here, h and b: UGKS 64 x 64 cells x 32^2 velocities FP32 91 / 63,
-// FP64 151 / 99, 128 x 128 x 48^2 FP32 1140 / 486, 100 x 100 x 40^2 FP64 704 / 425; KFVS 96 x 96 x 32^2 FP32 146 /
-// 95.  k_tile2d is bound by the issue of vector instructions (UGKS FP32: 671 slots per row of 4 cells, 307 us of
-// the 486), k_relax2d by memory (4.6 TB/s), k_chain2d by latency; small KFVS meshes, whose walls' latency is
+// cell's loads and stores.  us per step there / here, h and b: UGKS 64 x 64 cells x 32^2 velocities FP32 91 / 61,
+// FP64 151 / 95, 128 x 128 x 48^2 FP32 1140 / 489, 100 x 100 x 40^2 FP64 704 / 426; KFVS 96 x 96 x 32^2 FP32 146 /
+// 95.  k_tile2d is bound by the issue of vector instructions (UGKS FP32: 315 us of the 489), k_relax2d by memory
+// (4.6 TB/s), k_chain2d by latency; small KFVS meshes, whose walls' latency is
 // the step, stay with the other kernels (tiled2d, kbg_api.hip).
 //
 // The mesh is axis-aligned (x-face normals (n, 0), y-face normals (0, n), n > 0), so a velocity's upwind side
@@ -880,6 +880,7 @@ int tile2d_rows(bool fp64, const long* wgs) {
 template <class T> constexpr size_t tile2d_lds(int ty) {
     return (size_t(ty) * (kTX + 3) + size_t(ty + 3) * kTX) * sizeof(FaceRec<T>) + size_t(ty) * kTX * (sizeof(T) + 4 * 64 * sizeof(double));
 }
+static_assert(tile2d_lds<double>(kTile2dRows) <= 65536, "dynamic LDS a kernel may use without asking");
 
 template <class T, int FLUX>
 static hipError_t launch_tile_t(int ty, const Solve2D* d_solves, const int* d_pref, int n, const int* totals, int rows, int first, int last,
@@ -914,17 +915,6 @@ hipError_t launch_tile2d(bool fp64, int flux, int ty, const Solve2D* d_solves, c
     if (flux == KCU) KBG_T(float, KCU);
     KBG_T(float, UGKS);
 #undef KBG_T
-}
-
-// above the 64 KB of dynamic LDS a kernel may use without asking
-hipError_t tile2d_attr() {
-    constexpr size_t lds = tile2d_lds<double>(kTile2dRows);
-    hipError_t e = hipSuccess;
-    for (const void* k : {(const void*)k_tile2d<double, KFVS, false>, (const void*)k_tile2d<double, KFVS, true>,
-                          (const void*)k_tile2d<double, KCU, false>, (const void*)k_tile2d<double, KCU, true>,
-                          (const void*)k_tile2d<double, UGKS, false>, (const void*)k_tile2d<double, UGKS, true>})
-        if (e == hipSuccess) e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
-    return e;
 }
 
 }  // namespace kbg

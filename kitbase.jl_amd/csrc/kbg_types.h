@@ -325,6 +325,5 @@ hipError_t launch_tile2d(bool fp64, int flux, int ty, const Solve2D* d_solves, c
 int tile2d_rows(bool fp64, const long* wgs);  // rows per tile for a group of wgs[k] workgroups of k rows, k = 1 .. kTile2dRows
 int pre2d_wgs(int nx, int ny);
 int relax2d_wgs(int nx, int ny, int nv);
-hipError_t tile2d_attr();
 
 }  // namespace kbg
